@@ -565,7 +565,8 @@ int add_impl(rsh_batch b, rsh_dirset ds, int64_t n_cells, double albedo, int for
         return hip_fail(e, "batch slot initialisation");
     }
     PanelRef pe;
-    int rc = get_panel(ds, 0, ds->m, 1, form, b->stream, &pe, s.res ? &s.splan : nullptr, kGroupedF64MaxRb);
+    int rc = form == RSH_FORM_FP64 ? get_panel_f64(ds, 0, ds->m, 1, b->stream, s.plan, &pe)
+                                   : get_panel_split(ds, 0, ds->m, 1, form, b->stream, &pe, s.res ? &s.splan : nullptr);
     if (rc) {
         free_slot(b, s);
         return rc;

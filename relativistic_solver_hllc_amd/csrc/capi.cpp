@@ -55,63 +55,90 @@ int check_device(int dev) {
     return RSH_OK;
 }
 
-// Build an entry of the panel cache: on stream st, for rows [k0, k1).
-int build_panel(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, const SplitPlan* resident,
-                int f64_max_rb, PanelEntry& pe) {
-    pe.device = ds->device;
-    hipError_t e = hipSuccess;
-    if (form == RSH_FORM_FP64) {
-        pe.plan = plan_f64(ds->m, k1 - k0, f64_max_rb);
-        const int64_t nd = panel_f64_doubles(pe.plan);
-        e = hipMalloc(&pe.d_panel, std::max<int64_t>(nd, 1) * sizeof(double));
-        if (e == hipSuccess)
-            e = launch_panel_f64(ds->d_P, ds->m, k0, k1, 1.0 / faces, pe.plan, static_cast<double*>(pe.d_panel), st);
-    } else {
-        pe.splan = resident ? *resident : plan_split(ds->m, k1 - k0);
-        const int64_t units = split_panel_units(form, pe.splan);
-        e = hipMalloc(&pe.d_panel, std::max<int64_t>(units, 1) * 16);
-        if (e == hipSuccess) e = hipMalloc(&pe.d_row_inv, std::max(pe.splan.rb_total * 16, 1) * sizeof(float));
-        if (e == hipSuccess)
-            e = launch_split_panel(form, ds->d_P, ds->m, k0, k1, 1.0 / faces, pe.splan, pe.d_panel, pe.d_row_inv, st);
+// Panel cache entry of `key`, if there is one; st waits for its build only while
+// that may still be running.
+static int cached_panel(rsh_dirset ds, const std::tuple<int, int, int, int, int>& key, hipStream_t st, PanelRef* out) {
+    out->reset();
+    auto it = ds->panels.find(key);
+    if (it == ds->panels.end()) return RSH_OK;
+    const PanelEntry& pe = *it->second;
+    if (!pe.built.load(std::memory_order_relaxed)) {
+        const hipError_t q = hipEventQuery(pe.ready);
+        if (q == hipErrorNotReady)
+            RSH_HIP_TRY(hipStreamWaitEvent(st, pe.ready, 0));
+        else if (q == hipSuccess)
+            pe.built.store(true, std::memory_order_relaxed);
     }
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&pe.ready, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(pe.ready, st);
-    if (e != hipSuccess) return hip_fail(e, "phase panel build");
+    *out = it->second;
     return RSH_OK;
 }
 
-// Panel for rows [k0,k1), face count and form, built on stream st if absent.
-int get_panel(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
-              const SplitPlan* resident, int f64_max_rb) {
-    std::lock_guard<std::mutex> lock(ds->mu);
-    // layout: FP64 -> pass cap; split -> 0 streaming plan, 100 + row blocks per group for a resident plan
-    auto key = std::make_tuple(k0, k1, faces, form,
-                               form == RSH_FORM_FP64 ? f64_max_rb : (resident ? 100 + resident->rb_per_pass : 0));
-    auto it = ds->panels.find(key);
-    if (it != ds->panels.end()) {
-        // Make st wait for the build only while it may still be running.
-        if (hipEventQuery(it->second->ready) == hipErrorNotReady)
-            RSH_HIP_TRY(hipStreamWaitEvent(st, it->second->ready, 0));
-        *out = it->second;
-        return RSH_OK;
-    }
-    if (ds->panels.size() >= kPanelCacheCap) {
-        // Bounded cache: evict the entries nobody else holds (batch slots and
-        // calls still enqueuing keep theirs); each is freed after the device
-        // is idle, by its destructor.
-        for (auto e = ds->panels.begin(); e != ds->panels.end();) {
-            if (e->second.use_count() == 1)
-                e = ds->panels.erase(e);
-            else
-                ++e;
-        }
-    }
-    auto pe = std::make_shared<PanelEntry>();
-    int rc = build_panel(ds, k0, k1, faces, form, st, resident, f64_max_rb, *pe);
-    if (rc) return rc;
+// Adds a built entry (its kernels are on stream st) to the panel cache.
+static int store_panel(rsh_dirset ds, const std::tuple<int, int, int, int, int>& key, hipStream_t st,
+                       std::shared_ptr<PanelEntry> pe, hipError_t built, PanelRef* out) {
+    hipError_t e = built;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&pe->ready, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(pe->ready, st);
+    if (e != hipSuccess) return hip_fail(e, "phase panel build");
     ds->panels.emplace(key, pe);
     *out = pe;
     return RSH_OK;
+}
+
+// Bounded cache: evict the entries nobody else holds (batch slots and calls
+// still enqueuing keep theirs); each is freed after the device is idle, by its
+// destructor.
+static void bound_panels(rsh_dirset ds) {
+    if (ds->panels.size() < kPanelCacheCap) return;
+    for (auto e = ds->panels.begin(); e != ds->panels.end();) {
+        if (e->second.use_count() == 1)
+            e = ds->panels.erase(e);
+        else
+            ++e;
+    }
+}
+
+int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out) {
+    std::lock_guard<std::mutex> lock(ds->mu);
+    const int layout = plan.rb_per_pass + (plan.paired ? 100 : 0);
+    const auto key = std::make_tuple(k0, k1, faces, (int)RSH_FORM_FP64, layout);
+    if (int rc = cached_panel(ds, key, st, out)) return rc;
+    if (*out) return RSH_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+        auto it = ds->panels.lower_bound(std::make_tuple(k0, k1, faces, (int)RSH_FORM_FP64, 0));
+        if (it != ds->panels.end() && std::get<0>(it->first) == k0 && std::get<1>(it->first) == k1 &&
+            std::get<2>(it->first) == faces && std::get<3>(it->first) == RSH_FORM_FP64)
+            return cached_panel(ds, it->first, st, out);
+    }
+    bound_panels(ds);
+    auto pe = std::make_shared<PanelEntry>();
+    pe->device = ds->device;
+    pe->plan = plan;
+    const int64_t nd = panel_f64_doubles(plan);
+    hipError_t e = hipMalloc(&pe->d_panel, std::max<int64_t>(nd, 1) * sizeof(double));
+    if (e == hipSuccess)
+        e = launch_panel_f64(ds->d_P, ds->m, k0, k1, 1.0 / faces, plan, static_cast<double*>(pe->d_panel), st);
+    return store_panel(ds, key, st, pe, e, out);
+}
+
+int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
+                    const SplitPlan* resident) {
+    std::lock_guard<std::mutex> lock(ds->mu);
+    // layout: 0 streaming plan, 100 + row blocks per group for a resident plan
+    const auto key = std::make_tuple(k0, k1, faces, form, resident ? 100 + resident->rb_per_pass : 0);
+    if (int rc = cached_panel(ds, key, st, out)) return rc;
+    if (*out) return RSH_OK;
+    bound_panels(ds);
+    auto pe = std::make_shared<PanelEntry>();
+    pe->device = ds->device;
+    pe->splan = resident ? *resident : plan_split(ds->m, k1 - k0);
+    const int64_t units = split_panel_units(form, pe->splan);
+    hipError_t e = hipMalloc(&pe->d_panel, std::max<int64_t>(units, 1) * 16);
+    if (e == hipSuccess) e = hipMalloc(&pe->d_row_inv, std::max(pe->splan.rb_total * 16, 1) * sizeof(float));
+    if (e == hipSuccess)
+        e = launch_split_panel(form, ds->d_P, ds->m, k0, k1, 1.0 / faces, pe->splan, pe->d_panel, pe->d_row_inv, st);
+    return store_panel(ds, key, st, pe, e, out);
 }
 
 }  // namespace rsh
@@ -138,11 +165,18 @@ namespace rsh {
 static std::mutex g_tune_mu;
 static std::map<std::pair<int, int>, rsh_tile> g_tune;
 
-rsh_tile f64_tile_for(int device, int rb) {
+bool f64_tile_tuned(int device, int rb, rsh_tile* t) {
     std::lock_guard<std::mutex> lock(g_tune_mu);
     auto it = g_tune.find({device, rb});
-    if (it != g_tune.end()) return it->second;
-    return rsh_tile{8, 2};
+    if (it == g_tune.end()) return false;
+    *t = it->second;
+    return true;
+}
+
+rsh_tile f64_tile_for(int device, int rb) {
+    rsh_tile t{8, 2};
+    (void)f64_tile_tuned(device, rb, &t);
+    return t;
 }
 
 void set_tuned_tile(int device, int rb, rsh_tile t) {
@@ -173,15 +207,33 @@ int scatter_f64(rsh_dirset ds, const double* d_illum, int faces, int64_t n, int6
         return RSH_OK;
     }
     if (kernel != RSH_F64_AUTO && kernel != RSH_F64_MFMA) return fail(RSH_E_ARG, "unknown FP64 kernel id");
-    rsh_tile t = (tile && kernel == RSH_F64_MFMA) ? *tile
-                                                  : f64_tile_for(ds->device, plan_f64(ds->m, k1 - k0).rb_per_pass);
-    if (!mfma_f64_tile_supported(t.waves, t.chunk_steps))
-        return fail(RSH_E_UNSUPPORTED, "unsupported MFMA tile (waves, chunk_steps)");
+    // A given tile runs the LDS-panel kernel with it; otherwise the route for
+    // this size, with the tile that rsh_autotune_f64 recorded for the class.
+    F64Route rt;
+    if (tile && kernel == RSH_F64_MFMA) {
+        rt.plan = plan_f64(ds->m, k1 - k0);
+        rt.waves = tile->waves;
+        rt.chunk_steps = tile->chunk_steps;
+        if (!mfma_f64_tile_supported(rt.waves, rt.chunk_steps))
+            return fail(RSH_E_UNSUPPORTED, "unsupported MFMA tile (waves, chunk_steps)");
+    } else {
+        rt = route_f64(ds->m, k1 - k0, faces, n, device_cus(ds->device));
+    }
     PanelRef pe;  // held until the launch is enqueued
-    int rc = get_panel(ds, k0, k1, faces, RSH_FORM_FP64, st, &pe);
+    int rc = get_panel_f64(ds, k0, k1, faces, st, rt.plan, &pe);
     if (rc) return rc;
-    RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n, ldx, ds->m, static_cast<const double*>(pe->d_panel), pe->plan,
-                                k1 - k0, d_out, ld, t.waves, t.chunk_steps, st));
+    const double* panel = static_cast<const double*>(pe->d_panel);
+    if (pe->plan.paired) {
+        RSH_HIP_TRY(launch_mfma_f64_reg(d_illum, faces, n, ldx, ds->m, panel, pe->plan, k1 - k0, d_out, ld, st));
+        return RSH_OK;
+    }
+    rsh_tile t{rt.waves, rt.chunk_steps};
+    if (!tile || kernel != RSH_F64_MFMA) {
+        if (t.waves == 0) t = rsh_tile{8, 2};  // a captured stream's cached panel in place of the register-fed one
+        (void)f64_tile_tuned(ds->device, pe->plan.rb_per_pass, &t);
+    }
+    RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n, ldx, ds->m, panel, pe->plan, k1 - k0, d_out, ld, t.waves,
+                                t.chunk_steps, st));
     return RSH_OK;
 }
 
@@ -236,13 +288,13 @@ int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_c
         waves = (resident_ok && 4 * sets * rplan.passes >= 3 * per_xcd) ? 1 : split_default_waves();
     PanelRef pe;  // held until the launch is enqueued
     if (waves == 1) {
-        int rc = get_panel(ds, k0, k1, faces, form, st, &pe, &rplan);
+        int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe, &rplan);
         if (rc) return rc;
         RSH_HIP_TRY(launch_split_resident(form, d_state, n, d_cell_inv, pe->d_panel, pe->d_row_inv, pe->splan, sets,
                                           k1 - k0, d_out, ld, out_f32 ? 1 : 0, st));
         return RSH_OK;
     }
-    int rc = get_panel(ds, k0, k1, faces, form, st, &pe);
+    int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe);
     if (rc) return rc;
     RSH_HIP_TRY(launch_split_mfma(form, d_state, faces, n, d_cell_inv, pe->d_panel, pe->d_row_inv, pe->splan,
                                   k1 - k0, d_out, ld, out_f32 ? 1 : 0, waves, waves == 8 ? 2 : 1, st));

@@ -19,6 +19,8 @@
 //     fragment), prefetched from L2 one chunk ahead;
 //   - the epilogue storing each 16x16 tile as four 128-byte row segments of the
 //     direction-major output with non-temporal stores (S is not re-read).
+#include <type_traits>
+
 #include "mfma_f64_core.hpp"
 
 namespace rsh {
@@ -74,16 +76,18 @@ hipError_t launch_build_phase(const double* d_dirs, const double* d_w, int m, do
 // Panel re-layout (see rsh_internal.hpp for the fragment-major layout).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void panel_f64_kernel(const double* __restrict__ P, int m, int k0, int k1,
-                                                        double scale, int rb_per_pass, int steps, int64_t total,
-                                                        double* __restrict__ panel) {
+                                                        double scale, int rb_per_pass, int steps, int paired,
+                                                        int64_t total, double* __restrict__ panel) {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= total) return;
-    const int lane = (int)(idx & 63);
-    int64_t frag = idx >> 6;
+    // paired: 128 doubles per (step pair, row block), the lane's two steps adjacent
+    const int lane = (int)(paired ? (idx >> 1) & 63 : idx & 63);
+    int64_t frag = paired ? idx >> 7 : idx >> 6;
     const int rb_local = (int)(frag % rb_per_pass);
     frag /= rb_per_pass;
-    const int s = (int)(frag % steps);
-    const int pass = (int)(frag / steps);
+    const int ns = paired ? steps / 2 : steps;
+    const int s = paired ? 2 * (int)(frag % ns) + (int)(idx & 1) : (int)(frag % ns);
+    const int pass = (int)(frag / ns);
     const int k = k0 + (pass * rb_per_pass + rb_local) * 16 + (lane & 15);
     const int j = 4 * s + (lane >> 4);
     double v = 0.0;
@@ -91,17 +95,12 @@ __global__ __launch_bounds__(256) void panel_f64_kernel(const double* __restrict
     panel[idx] = v;
 }
 
-static const int kRbSet[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 13, 16, 20, 25};
-
 F64Plan plan_f64(int m, int rows, int max_rb) {
     F64Plan pl{};
     const int nrb = (rows + 15) / 16;
     if (max_rb < 1 || max_rb > kMaxRowBlocksPerPass) max_rb = kMaxRowBlocksPerPass;
     pl.passes = nrb > 0 ? (nrb + max_rb - 1) / max_rb : 0;
-    const int per = pl.passes > 0 ? (nrb + pl.passes - 1) / pl.passes : 0;
-    pl.rb_per_pass = 0;
-    for (int v : kRbSet)
-        if (v >= per) { pl.rb_per_pass = v; break; }
+    pl.rb_per_pass = pl.passes > 0 ? (nrb + pl.passes - 1) / pl.passes : 0;  // an instance for every count
     pl.rb_total = pl.rb_per_pass * pl.passes;
     const int steps = (m + 3) / 4;
     pl.steps = (steps + kPanelStepAlign - 1) / kPanelStepAlign * kPanelStepAlign;
@@ -116,7 +115,7 @@ hipError_t launch_panel_f64(const double* d_P, int m, int k0, int k1, double sca
     if (total == 0) return hipSuccess;
     const int64_t blocks = (total + 255) / 256;
     hipLaunchKernelGGL(panel_f64_kernel, dim3((unsigned)blocks), dim3(256), 0, st, d_P, m, k0, k1, scale,
-                       pl.rb_per_pass, pl.steps, total, d_panel);
+                       pl.rb_per_pass, pl.steps, pl.paired ? 1 : 0, total, d_panel);
     return hipGetLastError();
 }
 
@@ -166,6 +165,14 @@ hipError_t launch_direct_f64(const double* d_illum, int faces, int64_t n, int m,
     return hipGetLastError();
 }
 
+// Waves per SIMD that the register allocation must leave room for. Four-wave
+// workgroups with 2 j-steps per stage run two (three up to 13 row blocks) to a
+// CU, each with its own barriers; without the bound the compiler spends 512
+// registers on one. 24 and 25 row blocks would spill under it, and are slower.
+constexpr int f64_min_waves(int rb, int w, int sc) {
+    return w == 4 && sc == 2 && rb <= kF64FourWaveMaxRb ? (rb <= 13 ? 3 : 2) : w == 8 ? 2 : 1;
+}
+
 // ---------------------------------------------------------------------------
 // FP64 MFMA GEMM.
 //
@@ -180,7 +187,7 @@ hipError_t launch_direct_f64(const double* d_illum, int faces, int64_t n, int m,
 // through registers into one of two LDS buffers while the other is consumed.
 // ---------------------------------------------------------------------------
 template <int RB, int W, int SC, int FACES>
-__global__ __launch_bounds__(64 * W) void mfma_f64_kernel(const double* __restrict__ illum, int64_t n, int64_t ldx,
+__global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_kernel(const double* __restrict__ illum, int64_t n, int64_t ldx,
                                                           int m, const double* __restrict__ panel, int steps,
                                                           double* __restrict__ out, int64_t ld, int rows) {
     __shared__ v2d lds[2][F64TileShape<RB, W, SC>::UNITS];
@@ -193,13 +200,30 @@ __global__ __launch_bounds__(64 * W) void mfma_f64_kernel(const double* __restri
     mfma_f64_accumulate<RB, W, SC, FACES>(illum, n, ldx, m, panel + (int64_t)blockIdx.y * steps * RB * 64, steps,
                                           cell, lds, acc);
     if (cell >= n) return;
+    // Non-temporal stores where every 128-byte segment of a row is whole (16
+    // cells at a 128-byte boundary); a ragged row stride splits each segment over
+    // two lines, which must meet in L2 before they leave it: with non-temporal
+    // stores 413,519 cells x 302 directions took 1644 us, with plain ones 1528
+    // us (413,568 cells: 1499 us either way; 1.57 M x 400 2 % slower plain).
+    auto store = [&](auto nt) {
 #pragma unroll
-    for (int rb = 0; rb < RB; rb++) {
+        for (int rb = 0; rb < RB; rb++) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = (rb0 + rb) * 16 + jr + 4 * r;
-            if (row < rows) __builtin_nontemporal_store(acc[rb][r], out + (int64_t)row * ld + cell);
+            for (int r = 0; r < 4; r++) {
+                const int row = (rb0 + rb) * 16 + jr + 4 * r;
+                if (row < rows) {
+                    if constexpr (decltype(nt)::value) __builtin_nontemporal_store(acc[rb][r], out + (int64_t)row * ld + cell);
+                    else out[(int64_t)row * ld + cell] = acc[rb][r];
+                }
+            }
         }
+    };
+    if ((ld & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0) {
+        store(std::true_type{});
+    } else {
+        asm volatile("" ::: "memory");  // keeps the compiler from merging the two branches' stores into plain ones
+        store(std::false_type{});
+        asm volatile("" ::: "memory");
     }
 }
 
@@ -213,7 +237,9 @@ static hipError_t launch_mfma_rb(int rb, dim3 grid, hipStream_t st, const double
         break;
     switch (rb) {
         RSH_RB_CASE(1) RSH_RB_CASE(2) RSH_RB_CASE(3) RSH_RB_CASE(4) RSH_RB_CASE(5) RSH_RB_CASE(6)
-        RSH_RB_CASE(7) RSH_RB_CASE(8) RSH_RB_CASE(10) RSH_RB_CASE(13) RSH_RB_CASE(16) RSH_RB_CASE(20)
+        RSH_RB_CASE(7) RSH_RB_CASE(8) RSH_RB_CASE(9) RSH_RB_CASE(10) RSH_RB_CASE(11) RSH_RB_CASE(12)
+        RSH_RB_CASE(13) RSH_RB_CASE(14) RSH_RB_CASE(15) RSH_RB_CASE(16) RSH_RB_CASE(17) RSH_RB_CASE(18)
+        RSH_RB_CASE(19) RSH_RB_CASE(20) RSH_RB_CASE(21) RSH_RB_CASE(22) RSH_RB_CASE(23) RSH_RB_CASE(24)
         RSH_RB_CASE(25)
         default:
             return hipErrorInvalidValue;

@@ -128,7 +128,7 @@ hipError_t launch_batch_zero(BatchProblem* d_probs, int nprobs, unsigned* d_coun
     return hipGetLastError();
 }
 
-// Row-block counts of the instances: every kRbSet value up to kGroupedF64MaxRb.
+// Row-block counts of the instances: every count up to kGroupedF64MaxRb.
 static_assert(kGroupedF64MaxRb == 13, "instance list below covers row blocks 1..13");
 
 template <int W, int SC>
@@ -141,7 +141,7 @@ static hipError_t launch_grouped_rb(int rb, int grid, hipStream_t st, const Batc
         break;
     switch (rb) {
         RSH_RB_CASE(1) RSH_RB_CASE(2) RSH_RB_CASE(3) RSH_RB_CASE(4) RSH_RB_CASE(5) RSH_RB_CASE(6)
-        RSH_RB_CASE(7) RSH_RB_CASE(8) RSH_RB_CASE(10) RSH_RB_CASE(13)
+        RSH_RB_CASE(7) RSH_RB_CASE(8) RSH_RB_CASE(9) RSH_RB_CASE(10) RSH_RB_CASE(11) RSH_RB_CASE(12) RSH_RB_CASE(13)
         default:
             return hipErrorInvalidValue;
     }
@@ -170,7 +170,7 @@ int grouped_iter_f64_resident(int rb, int waves, int chunk_steps, int device) {
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grouped_iter_f64_kernel<V, W, SC>, 64 * W, 0);
 #define RSH_OCC_ALL(V) RSH_OCC(V, 8, 2) RSH_OCC(V, 4, 2) RSH_OCC(V, 4, 4)
     RSH_OCC_ALL(1) RSH_OCC_ALL(2) RSH_OCC_ALL(3) RSH_OCC_ALL(4) RSH_OCC_ALL(5) RSH_OCC_ALL(6) RSH_OCC_ALL(7)
-    RSH_OCC_ALL(8) RSH_OCC_ALL(10) RSH_OCC_ALL(13)
+    RSH_OCC_ALL(8) RSH_OCC_ALL(9) RSH_OCC_ALL(10) RSH_OCC_ALL(11) RSH_OCC_ALL(12) RSH_OCC_ALL(13)
 #undef RSH_OCC_ALL
 #undef RSH_OCC
     if (e != hipSuccess || per_cu < 1) per_cu = 1;

@@ -390,12 +390,16 @@ __global__ __launch_bounds__(64 * W) void split_mfma_kernel(const v4u* __restric
 
 // ------------------------------------------------------------------ launchers
 
+static const int kRbSet[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 13, 16, 20, 25};  // instances
+
 SplitPlan plan_split(int m, int rows) {
     SplitPlan pl{};
-    const F64Plan fp = plan_f64(m, rows);  // same row-block / pass selection
-    pl.rb_per_pass = fp.rb_per_pass;
+    const F64Plan fp = plan_f64(m, rows);  // same passes
+    for (int v : kRbSet)
+        if (v >= fp.rb_per_pass) { pl.rb_per_pass = v; break; }
+    if (fp.rb_per_pass == 0) pl.rb_per_pass = 0;
     pl.passes = fp.passes;
-    pl.rb_total = fp.rb_total;
+    pl.rb_total = pl.rb_per_pass * pl.passes;
     pl.steps = (m + 31) / 32;
     return pl;
 }

@@ -66,8 +66,10 @@ int rsh_scatter_f64_dev_noalloc(rsh_dirset ds, const double* d_illum, int32_t fa
     if (n_cells == 0 || k0 == k1) return RSH_OK;
     if (!d_illum || !d_out) return fail(RSH_E_ARG, "null device pointer");
     if (ld_out < n_cells) return fail(RSH_E_ARG, "ld_out smaller than n_cells");
-    const F64Plan pl = plan_f64(ds->m, k1 - k0);
-    const int64_t bytes = panel_f64_doubles(pl) * (int64_t)sizeof(double);
+    // Which ranges fit does not depend on the kernel: those whose panel fits with
+    // its row blocks per pass padded as the split plan pads them.
+    const F64Plan lds_plan = plan_f64(ds->m, k1 - k0);
+    const int64_t bytes = (int64_t)lds_plan.steps * plan_split(ds->m, k1 - k0).rb_total * 64 * (int64_t)sizeof(double);
     if (bytes > (int64_t)kNoAllocScratchBytes)
         return fail(RSH_E_UNSUPPORTED, "phase panel of " + std::to_string(bytes) + " bytes exceeds the " +
                                            std::to_string(kNoAllocScratchBytes) +
@@ -76,9 +78,19 @@ int rsh_scatter_f64_dev_noalloc(rsh_dirset ds, const double* d_illum, int32_t fa
     void* panel = nullptr;
     int rc = scratch_for(ds->device, &panel);
     if (rc) return rc;
-    const rsh_tile t = f64_tile_for(ds->device, pl.rb_per_pass);
+    F64Route rt = route_f64(ds->m, k1 - k0, faces, n_cells, device_cus(ds->device));
+    if (panel_f64_doubles(rt.plan) * (int64_t)sizeof(double) > (int64_t)kNoAllocScratchBytes)
+        rt = F64Route{lds_plan, 8, 2};  // the register-fed kernel's panel may have more padding rows
+    const F64Plan& pl = rt.plan;
     hipStream_t st = (hipStream_t)stream;
     RSH_HIP_TRY(launch_panel_f64(ds->d_P, ds->m, k0, k1, 1.0 / faces, pl, static_cast<double*>(panel), st));
+    if (pl.paired) {
+        RSH_HIP_TRY(launch_mfma_f64_reg(d_illum, faces, n_cells, n_cells, ds->m, static_cast<const double*>(panel), pl,
+                                        k1 - k0, d_out, ld_out, st));
+        return RSH_OK;
+    }
+    rsh_tile t{rt.waves, rt.chunk_steps};
+    (void)f64_tile_tuned(ds->device, pl.rb_per_pass, &t);
     RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n_cells, n_cells, ds->m, static_cast<const double*>(panel), pl,
                                 k1 - k0, d_out, ld_out, t.waves, t.chunk_steps, st));
     return RSH_OK;

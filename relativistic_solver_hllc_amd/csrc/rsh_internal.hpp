@@ -30,6 +30,8 @@ int hip_fail(hipError_t e, const char* what);
 // contiguous bytes, so a wave reads it with one coalesced load / LDS read.
 constexpr int kPanelStepAlign = 4;      // j-steps padded to a multiple of this
 constexpr int kMaxRowBlocksPerPass = 25; // 400 output directions per pass
+// Most row blocks with which two four-wave workgroups of the LDS-panel kernel fit a CU's registers.
+constexpr int kF64FourWaveMaxRb = 23;
 // The grouped iteration kernel's fused epilogue (B and the previous state read
 // per output) is latency-bound at one workgroup per CU; passes of at most 13 row
 // blocks (208 rows, at 4 waves x 2 j-steps per LDS stage) let two workgroups
@@ -44,11 +46,25 @@ struct F64Plan {
     int rb_per_pass;   // row blocks per workgroup pass (template value)
     int passes;        // grid.y
     int rb_total;      // rb_per_pass * passes (panel rows / 16)
-    int steps;         // padded j-steps (multiple of kPanelStepAlign)
+    int steps;         // padded j-steps (multiple of kPanelStepAlign; of 2 when paired)
+    // Register-fed kernel (kernels_f64_reg.hip): the panel keeps two j-steps of
+    // a lane side by side, so that one 16-byte load brings both:
+    //   panel[((pass * steps / 2 + s / 2) * rb_per_pass + rb) * 128 + 2 lane + s % 2]
+    bool paired;
 };
 
 F64Plan plan_f64(int m, int rows, int max_rb = kMaxRowBlocksPerPass);
 int64_t panel_f64_doubles(const F64Plan& pl);
+// Plan of the register-fed kernel with r row blocks per wave (f64_reg_rows_supported).
+F64Plan plan_f64_reg(int m, int rows, int r);
+bool f64_reg_rows_supported(int r);
+// How one FP64 evaluation runs: waves = 0: the register-fed kernel on `plan`,
+// else the LDS-panel kernel with that tile.
+struct F64Route {
+    F64Plan plan;
+    int waves, chunk_steps;
+};
+F64Route route_f64(int m, int rows, int faces, int64_t n, int cus);
 
 // ------------------------------------------------------------------ kernels
 hipError_t launch_build_phase(const double* d_dirs, const double* d_w, int m, double full_area,
@@ -65,6 +81,10 @@ bool mfma_f64_tile_supported(int waves, int chunk_steps);
 hipError_t launch_mfma_f64(const double* d_illum, int faces, int64_t n, int64_t ldx, int m, const double* d_panel,
                            const F64Plan& pl, int rows, double* d_out, int64_t ld, int waves,
                            int chunk_steps, hipStream_t st);
+
+// Register-fed FP64 kernel: paired plan, one wave per (16-cell tile, row group).
+hipError_t launch_mfma_f64_reg(const double* d_illum, int faces, int64_t n, int64_t ldx, int m, const double* d_panel,
+                               const F64Plan& pl, int rows, double* d_out, int64_t ld, hipStream_t st);
 
 // Relative-error reduction of results against an FP64 reference (gx x gy
 // workgroups, 3 doubles of partial result each: max, sum, count above).

@@ -1,6 +1,7 @@
 // Host-side objects behind the C ABI handles (direction sets, problems).
 #pragma once
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -20,6 +21,7 @@ struct PanelEntry {
     rsh::F64Plan plan{};
     rsh::SplitPlan splan{};
     hipEvent_t ready = nullptr;  // recorded after the panel build
+    mutable std::atomic<bool> built{false};  // the build was seen complete: no need to ask the event again
     PanelEntry() = default;
     PanelEntry(const PanelEntry&) = delete;
     PanelEntry& operator=(const PanelEntry&) = delete;
@@ -40,20 +42,23 @@ struct rsh_dirset_s {
     double* d_P = nullptr;  // [m][m] FP64 phase matrix
     double* d_psi = nullptr;  // [m][kMomentFuncs] moment weights (full_area > 0 only)
     std::mutex mu;
-    // key: (k0, k1, faces, form, layout); layout: FP64 pass cap, split 0 = streaming plan,
-    // 100 + row blocks per group = resident-panel plan
+    // key: (k0, k1, faces, form, layout); layout: FP64 row blocks per pass, 100 + row blocks per wave for the
+    // register-fed kernel; split 0 = streaming plan, 100 + row blocks per group = resident-panel plan
     std::map<std::tuple<int, int, int, int, int>, std::shared_ptr<PanelEntry>> panels;
     bool ref_order() const { return phase == RSH_PHASE_THOMSON && !normalize; }
 };
 
 namespace rsh {
-// Phase panel of (k0, k1, faces, form), built on stream st if absent. A split
-// panel with resident != nullptr uses that row-group plan (layout 1); an FP64
-// panel uses passes of at most f64_max_rb row blocks. The caller holds *out for
-// as long as it enqueues work that reads the panel (a batch slot: until the
-// slot is removed); the cache never frees an entry someone else holds.
-int get_panel(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
-              const SplitPlan* resident = nullptr, int f64_max_rb = kMaxRowBlocksPerPass);
+// FP64 phase panel of (k0, k1, faces) in the layout of `plan`, built on stream
+// st if absent. The caller holds *out for as long as it enqueues work that reads
+// the panel (a batch slot: until the slot is removed); the cache never frees an
+// entry someone else holds. While st is being captured nothing can be allocated:
+// then a panel of another layout of the same range, if there is one, is returned
+// instead of failing (*out carries its plan; every layout gives the same bits).
+int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out);
+// Split phase panel; resident != nullptr: in that row-group plan.
+int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
+                    const SplitPlan* resident = nullptr);
 // Cache capacity of a direction set's panel cache (entries not held elsewhere
 // are evicted beyond it).
 constexpr size_t kPanelCacheCap = 64;
@@ -61,6 +66,7 @@ constexpr size_t kPanelCacheCap = 64;
 int device_cus(int device);
 // Tile of the FP64 MFMA kernel chosen for a row-block class (tuned or default).
 rsh_tile f64_tile_for(int device, int rb);
+bool f64_tile_tuned(int device, int rb, rsh_tile* t);
 void set_tuned_tile(int device, int rb, rsh_tile t);
 int check_device(int dev);
 }  // namespace rsh

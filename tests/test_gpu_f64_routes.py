@@ -1,0 +1,49 @@
+"""The FP64 integral over the sizes between which its route changes: the register-fed kernel (few cells) with
+every number of row blocks per wave, and the LDS-panel kernel in more, shorter passes. Every route adds a result's
+products in the same order, so each must equal the LDS-panel kernel with a given tile bit for bit; against the
+oracle the bound is that kernel's own (1e-12 relative)."""
+import numpy as np
+import pytest
+
+from oracle import orc
+from relativistic_solver_hllc_amd import device as D
+from relativistic_solver_hllc_amd import scatter as rs
+
+pytestmark = pytest.mark.gpu
+
+# (cells, directions, faces, k0, k1): edges of the 16-cell tile, the 4- and 8-direction steps and the 16-row block;
+# then sizes that take 1-8 and 10 row blocks per wave, two passes of four waves, and a range of rows
+SIZES = [(1, 1, 4, 0, 1), (15, 3, 4, 0, 3), (16, 4, 1, 0, 4), (17, 8, 4, 0, 8), (63, 9, 1, 0, 9), (65, 16, 4, 0, 16),
+         (66, 17, 4, 0, 17), (381, 327, 4, 0, 327), (381, 327, 1, 5, 22), (1003, 302, 4, 0, 302), (2958, 200, 4, 0, 200),
+         (2959, 302, 4, 0, 302), (2957, 400, 1, 0, 400), (5001, 302, 4, 0, 302), (5000, 400, 4, 0, 400),
+         (9999, 129, 1, 0, 129), (24577, 113, 4, 0, 113), (24577, 302, 1, 7, 301)]
+
+
+def evaluate(ds, d_in, faces, n, k0, k1, **kw):
+    out = D.DeviceArray((k1 - k0, n + 5))
+    out.fill(-1.0)
+    ds.scatter_f64(d_in, faces, n, k0, k1, out, ld=n + 5, **kw)
+    D.synchronize()
+    got = out.to_host()
+    out.free()
+    assert np.all(got[:, n:] == -1.0)  # nothing past the last cell
+    return got[:, :n]
+
+
+@pytest.mark.parametrize("n,m,faces,k0,k1", SIZES)
+def test_route_equals_lds_panel_kernel(gpu, n, m, faces, k0, k1):
+    rng = np.random.default_rng(n + m)
+    illum = rng.lognormal(0.0, 1.5, size=(m, n, faces))
+    illum[m // 2, n // 2, :] = np.inf  # stays in its own cell, also where directions are padded
+    xyz, w, F = rs.fibonacci_directions(m)
+    d_in = D.DeviceArray.from_host(illum if faces == 4 else illum[..., 0])
+    with rs.DirectionSet(xyz, w, F, phase="hg", g=0.6, normalize=True) as ds:
+        got = evaluate(ds, d_in, faces, n, k0, k1)
+        want = evaluate(ds, d_in, faces, n, k0, k1, kernel="mfma", tile=(8, 2))
+    d_in.free()
+    assert np.array_equal(got, want, equal_nan=True)
+    cells = [c for c in {0, n - 1, n // 3, n // 2 + 1} if 0 <= c < n and c != n // 2]
+    if cells:
+        P = orc.phase_matrix(xyz, w, F, 1, 0.6, True)
+        ref = orc.scatter_matrix(np.ascontiguousarray(illum[:, cells]), P)[k0:k1]
+        assert np.max(np.abs(got[:, cells] - ref) / ref) < 1e-12
