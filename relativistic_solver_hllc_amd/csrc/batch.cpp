@@ -10,7 +10,7 @@
 // One batch iteration = a zeroing kernel + one grouped launch per class. Two
 // iterations (parity 0 then 1) are captured once into a hipGraph; changing the
 // active set rewrites the work lists and counts in device memory, which leaves
-// the captured graph valid (only a new class forces a re-capture).
+// the captured graph valid while it launches every class that has work.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,6 +21,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -30,8 +31,10 @@ using namespace rsh;
 
 namespace {
 
-constexpr int kMaxClasses = 16;
-constexpr int kXcdLists = 8;  // per-XCD work lists of the resident-panel split classes
+// FP64 row-block counts, resident split plans (one per K-step count) and
+// streaming row-block counts of three forms: no mix of problems needs more.
+constexpr int kMaxClasses = 192;
+constexpr int kXcdLists = 8;  // XCDs: the sets of a resident-panel class, and counters per class
 
 // Grouped-launch tuning table, filled by rsh_batch_autotune: FP64 classes by
 // (device, form, row blocks per pass) -> MFMA tile; split forms by (device,
@@ -87,9 +90,10 @@ struct ClassState {
     int* d_n_items = nullptr;
     int n_items = 0;
     int counter_index = 0;
-    // resident-panel split classes: K-steps, per-XCD list begins and counts
+    // resident-panel split classes: K-steps and row groups; d_meta = [problems, row groups, sets]
     bool res = false;
     int steps = 0;
+    int groups = 0;
     int* d_meta = nullptr;
 };
 
@@ -109,6 +113,7 @@ struct rsh_batch_s {
     std::map<std::pair<int, int>, ClassState> classes;  // by (form, row-block class)
     bool lists_dirty = true;
     bool graph_valid = false;
+    std::set<std::pair<int, int>> captured;  // classes that the captured graph launches
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipStream_t stream = nullptr;
@@ -187,12 +192,17 @@ void free_slot(rsh_batch b, Slot& s) {
 
 int slot_rb(const Slot& s) { return s.form == RSH_FORM_FP64 ? s.plan.rb_per_pass : s.splan.rb_per_pass; }
 // Class key: (form, row blocks per pass) for the FP64 and streaming split
-// kernels; resident-panel split classes also separate by K-steps (one kernel
-// instance per plan).
+// kernels; resident-panel split classes also separate by K-steps and row groups
+// (one kernel instance and one work split per plan).
 int slot_class(const Slot& s) {
-    return s.res ? 1000 + (s.res_waves == 4 ? 100000 : 0) + 64 * s.splan.rb_per_pass + s.splan.steps : slot_rb(s);
+    return s.res ? 1000 + (s.res_waves == 4 ? 100000 : 0) + 1000 * s.splan.passes + 64 * s.splan.rb_per_pass +
+                       s.splan.steps
+                 : slot_rb(s);
 }
 int slot_passes(const Slot& s) { return s.form == RSH_FORM_FP64 ? s.plan.passes : s.splan.passes; }
+
+// Sets of `groups` workgroups per XCD of a resident-panel class.
+int res_sets(const ClassState& cs) { return cs.grid / kXcdLists / cs.groups; }
 
 void destroy_graph(rsh_batch b) {
     if (b->exec) hipGraphExecDestroy(b->exec);
@@ -200,6 +210,7 @@ void destroy_graph(rsh_batch b) {
     b->exec = nullptr;
     b->graph = nullptr;
     b->graph_valid = false;
+    b->captured.clear();
 }
 
 // Rebuilds the device descriptor table and every class's work list.
@@ -213,8 +224,7 @@ int rebuild(rsh_batch b) {
         if (b->slots[i].active) order.push_back(i);
     std::sort(order.begin(), order.end(), [&](int x, int y) { return b->slots[x].m > b->slots[y].m; });
     bool new_class = false;
-    std::map<std::pair<int, int>, std::vector<std::vector<BatchItem>>> xlists;  // resident classes: per XCD
-    std::map<std::pair<int, int>, int> xnext;                                   // round-robin XCD of the next chunk
+    std::map<std::pair<int, int>, int64_t> dealt;  // resident classes: chunks of the problems listed so far
     for (int i : order) {
         const Slot& s = b->slots[i];
         const int rb = slot_rb(s);
@@ -239,10 +249,11 @@ int rebuild(rsh_batch b) {
                 cs.tile = rsh_tile{s.res_waves, 1};
                 // one workgroup per CU (8 waves), or two (4 waves; they co-reside
                 // where the panel is streamed by K-step and the LDS is small)
-                cs.grid = device_cus(b->device) / kXcdLists * kXcdLists * (s.res_waves == 4 ? 2 : 1);
+                cs.groups = s.splan.passes;
+                cs.grid = iter_split_res_grid(s.res_waves, device_cus(b->device));
                 RSH_HIP_TRY(launch_grouped_iter_split_res(false, cs.form, rb, cs.steps, cs.tile.waves, 0, nullptr,
-                                                          nullptr, nullptr, nullptr, 0, nullptr));
-                RSH_HIP_TRY(hipMalloc(&cs.d_meta, 2 * kXcdLists * sizeof(int)));
+                                                          nullptr, nullptr, 0, nullptr));
+                RSH_HIP_TRY(hipMalloc(&cs.d_meta, 3 * sizeof(int)));
             } else {
                 cs.tile = rsh_tile{grouped_iter_split_waves(), 1};
                 cs.grid = grouped_iter_split_resident(s.form, rb, b->device);
@@ -253,15 +264,11 @@ int rebuild(rsh_batch b) {
             new_class = true;
         }
         if (s.res) {
-            // items (problem, row group, chunk); a chunk's row groups go to one XCD's list
-            auto& X = xlists[key];
-            X.resize(kXcdLists);
-            const int64_t cc = iter_split_res_chunk_cells();
-            const int64_t chunks = (s.n + cc - 1) / cc;
-            for (int64_t c = 0; c < chunks; c++) {
-                auto& L = X[(size_t)(xnext[key]++ % kXcdLists)];
-                for (int rg = 0; rg < s.splan.passes; rg++) L.push_back(BatchItem{i, rg, c});
-            }
+            // one item per problem: its chunks are dealt to the class's sets after those of the problems before
+            const ClassState& cs = b->classes[key];
+            const int64_t cc = iter_split_res_chunk_cells(cs.tile.waves), slots = (int64_t)kXcdLists * res_sets(cs);
+            lists[key].push_back(BatchItem{i, 0, dealt[key] % slots});
+            dealt[key] += (s.n + cc - 1) / cc;
             continue;
         }
         const int tiles_w = 16 * b->classes[key].tile.waves;
@@ -273,16 +280,6 @@ int rebuild(rsh_batch b) {
     for (auto& kv : b->classes) {
         ClassState& cs = kv.second;
         auto& L = lists[kv.first];
-        int meta[2 * kXcdLists] = {};
-        if (cs.res) {
-            auto& X = xlists[kv.first];
-            X.resize(kXcdLists);
-            for (int x = 0; x < kXcdLists; x++) {
-                meta[x] = (int)L.size();
-                meta[kXcdLists + x] = (int)X[(size_t)x].size();
-                L.insert(L.end(), X[(size_t)x].begin(), X[(size_t)x].end());
-            }
-        }
         if ((int64_t)L.size() > cs.capacity) {
             hipFree(cs.d_items);
             cs.d_items = nullptr;
@@ -294,23 +291,37 @@ int rebuild(rsh_batch b) {
             RSH_HIP_TRY(hipMemcpy(cs.d_items, L.data(), L.size() * sizeof(BatchItem), hipMemcpyHostToDevice));
         cs.n_items = (int)L.size();
         RSH_HIP_TRY(hipMemcpy(cs.d_n_items, &cs.n_items, sizeof(int), hipMemcpyHostToDevice));
-        if (cs.res) RSH_HIP_TRY(hipMemcpy(cs.d_meta, meta, sizeof(meta), hipMemcpyHostToDevice));
+        if (cs.res) {
+            const int meta[3] = {cs.n_items, cs.groups, res_sets(cs)};
+            RSH_HIP_TRY(hipMemcpy(cs.d_meta, meta, sizeof(meta), hipMemcpyHostToDevice));
+        }
     }
     RSH_HIP_TRY(hipMemcpy(b->d_probs, b->h_probs.data(), b->capacity * sizeof(BatchProblem), hipMemcpyHostToDevice));
-    if (new_class) destroy_graph(b);
+    // The graph stays valid while it launches every class that has work and at
+    // most two that have none (an empty launch costs ~4 us per iteration, a new
+    // capture about as much as 30 of them).
+    size_t working = 0;
+    bool missing = false;
+    for (auto& kv : b->classes) {
+        if (kv.second.n_items == 0) continue;
+        working++;
+        missing = missing || !b->captured.count(kv.first);
+    }
+    if (new_class || missing || b->captured.size() > working + 2) destroy_graph(b);
     b->lists_dirty = false;
     return RSH_OK;
 }
 
+// One iteration of every class with work, on the batch stream.
 int enqueue_iteration(rsh_batch b, int parity) {
     RSH_HIP_TRY(launch_batch_zero(b->d_probs, b->capacity, b->d_counters, kMaxClasses * kXcdLists, parity,
                                   b->stream));
     for (auto& kv : b->classes) {
         ClassState& cs = kv.second;
+        if (cs.n_items == 0) continue;
         if (cs.res)
             RSH_HIP_TRY(launch_grouped_iter_split_res(true, cs.form, cs.rb, cs.steps, cs.tile.waves, cs.grid,
-                                                      b->d_probs, cs.d_items, cs.d_meta,
-                                                      b->d_counters + cs.counter_index, parity, b->stream));
+                                                      b->d_probs, cs.d_items, cs.d_meta, parity, b->stream));
         else if (cs.form == RSH_FORM_FP64)
             RSH_HIP_TRY(launch_grouped_iter_f64(cs.rb, cs.tile.waves, cs.tile.chunk_steps, cs.grid, b->d_probs,
                                                 cs.d_items, cs.d_n_items, b->d_counters + cs.counter_index, parity,
@@ -337,6 +348,8 @@ int capture(rsh_batch b) {
     b->graph = g;
     RSH_HIP_TRY(hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0));
     b->graph_valid = true;
+    for (auto& kv : b->classes)
+        if (kv.second.n_items > 0) b->captured.insert(kv.first);
     return RSH_OK;
 }
 
@@ -477,7 +490,8 @@ int add_impl(rsh_batch b, rsh_dirset ds, int64_t n_cells, double albedo, int for
         SplitPlan rplan{};
         int sets = 0;
         if (plan_split_resident(form, ds->m, ds->m, device_cus(b->device), &rplan, &sets, true) &&
-            iter_split_res_supported(form, rplan.rb_per_pass, rplan.steps)) {
+            iter_split_res_supported(form, rplan.rb_per_pass, rplan.steps) &&
+            (split_kernel == 0 || iter_split_res_selectable(rplan.steps))) {
             s.splan = rplan;
             s.res = true;
             s.res_waves = split_kernel == 3 ? 4 : 8;
@@ -692,9 +706,10 @@ int rsh_batch_autotune(int32_t device, int32_t form, int32_t m, int64_t n_cells,
         int slot = -1;
         if (form == RSH_FORM_FP64)
             rc = rsh_batch_set_f64_tile(bb, &cands[c]);
-        else
-            rc = rsh_batch_set_split_kernel(bb, cands[c].waves);
+        else  // the eight-wave resident kernel is what the automatic choice takes where it has a plan for M
+            rc = rsh_batch_set_split_kernel(bb, cands[c].waves == 1 ? 0 : cands[c].waves);
         if (!rc) rc = rsh_batch_add_seeded(bb, ds, n_cells, 0x7E57ull, 0.5, form, &slot);
+        if (!rc && form != RSH_FORM_FP64 && cands[c].waves == 1 && !bb->slots[slot].res) rc = RSH_E_UNSUPPORTED;
         if (rc == RSH_E_UNSUPPORTED) {  // candidate does not apply (e.g. no resident plan for this M)
             rsh_batch_destroy(bb);
             rc = RSH_OK;

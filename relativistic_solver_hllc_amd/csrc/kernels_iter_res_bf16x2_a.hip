@@ -1,0 +1,4 @@
+// Grouped split iteration, resident-panel plans of 1 to 14 K-steps (1 to 448 directions), form bf16x2.
+#include "split_iter_res.hpp"
+
+RSH_ITER_RES_RANGE(0, 2, 1, 14)

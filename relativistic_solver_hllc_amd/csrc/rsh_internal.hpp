@@ -212,17 +212,18 @@ hipError_t launch_grouped_iter_split(int form, int rb, int grid, const BatchProb
                                      const BatchItem* d_items, const int* d_n_items, unsigned* d_counter, int parity,
                                      hipStream_t st);
 int grouped_iter_split_resident(int form, int rb, int device);
-// Grouped iteration on split state, resident-panel form (kernels_split_resident.hip):
-// items (problem, row group, chunk of iter_split_res_chunk_cells() cells) in 8
-// per-XCD lists; meta = [8 list begins, 8 list counts]; counters = 8 per class.
-// waves: 8 (two tiles of 16 cells per wave, two waves per SIMD) or 4 (four
-// tiles per wave, one wave per SIMD); same items, panel and results.
+// Grouped iteration on split state, resident-panel form (split_iter_res.hpp):
+// items = the class's problems (tile = chunks of the problems before, modulo 8
+// sets); meta = [problems, row groups, sets] with sets = workgroups per XCD /
+// row groups. waves: 8 (256-cell chunks, one workgroup per CU) or 4 (128-cell
+// chunks, two); same panel and results.
 bool iter_split_res_supported(int form, int rb, int steps);
-size_t iter_split_res_lds(int form, int rb, int steps);
+bool iter_split_res_selectable(int steps);
 hipError_t launch_grouped_iter_split_res(bool launch, int form, int rb, int steps, int waves, int grid,
                                          const BatchProblem* d_probs, const BatchItem* d_items, const int* d_meta,
-                                         unsigned* d_counters, int parity, hipStream_t st);
-int iter_split_res_chunk_cells();
+                                         int parity, hipStream_t st);
+int iter_split_res_chunk_cells(int waves);
+int iter_split_res_grid(int waves, int cus);
 int grouped_iter_split_waves();
 hipError_t launch_unpack_state(int form, const void* d_state, int64_t n, int m, const float* d_cell_inv,
                                double* d_out, hipStream_t st);

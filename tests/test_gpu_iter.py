@@ -317,6 +317,40 @@ def test_split_resident_kernel_equals_streaming(gpu, form):
         p["ds"].close()
 
 
+@pytest.mark.parametrize("form", ["bf16x2", "bf16x3"])
+def test_split_resident_plans_equal_streaming(gpu, form):
+    """Every K-step count's resident plan (odd and even K-steps, held and streamed panels, 1-5 row blocks, ragged
+    directions and cells; two problems of one plan) against the streaming kernel, more classes in one batch than
+    the 16 of before: the same products in the same order, so states and residuals are bit-identical."""
+    ms = [26, 40, 64, 65, 110, 128, 161, 194, 256, 257, 302, 340, 350, 416, 434, 500, 512, 590, 620, 650, 700, 770, 161]
+    probs = [make(m, 600 + 37 * i if m != 302 else 9001, "hg", 0.6, seed=500 + i) for i, m in enumerate(ms)]
+    out = {}
+    for kind in ("streaming", "auto"):
+        with rs.Batch(len(ms)) as b:
+            b.set_split_kernel(kind)
+            slots = [add_form(b, p, form) for p in probs]
+            configs = {b.slot_config(s, form)[1] for s in slots}
+            assert configs == ({"streaming"} if kind == "streaming" else {"resident"})
+            b.run(5)
+            r, _ = b.residuals()
+            out[kind] = ([state(b, s, p) for s, p in zip(slots, probs)], [r[s] for s in slots])
+            if kind == "auto":  # problems leave and others go on: the same as in the whole mix
+                for s in slots[3:]:
+                    b.remove(s)
+                b.run(2)
+                few = [state(b, s, p) for s, p in zip(slots[:3], probs)]
+    for a, c, p in zip(out["streaming"][0], out["auto"][0], probs):
+        assert np.array_equal(a, c), p["m"]
+    assert out["streaming"][1] == out["auto"][1]
+    with rs.Batch(3) as b:
+        slots = [add_form(b, p, form) for p in probs[:3]]
+        b.run(7)
+        for s, p, a in zip(slots, probs, few):
+            assert np.array_equal(state(b, s, p), a)
+    for p in probs:
+        p["ds"].close()
+
+
 def test_fp64_batch_cell_limit(gpu):
     """FP64 batch problems hold fewer than 2^24 cells (the iteration kernel's
     32-bit buffer offsets span one row block of 16 rows); larger ones are refused
