@@ -115,43 +115,36 @@ hipError_t launch_pack_state(int form, const double* d_illum, int faces, int64_t
                              void* d_state, hipStream_t st);
 hipError_t launch_split_panel(int form, const double* d_P, int m, int k0, int k1, double factor,
                               const SplitPlan& pl, void* d_panel, float* d_row_inv, hipStream_t st);
-// Transport sweep (kernels_sweep.hip). Per direction, cells are grouped in
-// levels (a cell reads only from earlier levels) and each level is cut into
-// passes of kSweepBlock cells, one cell per thread of the direction's
-// workgroup. Everything a pass needs that does not depend on earlier results is
-// stored per position in level order, so that it can be fetched a pass ahead.
-constexpr int kSweepBlock = 512;
-constexpr int kSweepRecStride = 10;  // record slots per position (9 used; 80 bytes = five 16-byte loads)
-// The face values of the last kSweepRing passes stay in an LDS ring (one slot
-// of kSweepBlock x 4 doubles per pass); an upstream value written at most
-// kSweepRingDelta passes before the reading pass is read from there, older
-// ones from global memory (complete by then: see kernels_sweep.hip).
-constexpr int kSweepRing = 4;
-constexpr int kSweepRingDelta = 3;
-struct SweepPos {
-    int32_t cell;
-    // bits 0-3: in faces; 4-7: faces out on both sides whose neighbour came
-    // earlier (this cell also writes the neighbour's entry); 8 + 2q: in-face id
-    // of record slot q (q = 3 r + j: node j of the r-th out face)
-    uint32_t meta;
-    int32_t pr[4];  // pairs of the cell
-    // ring code of in face f in bits 16 (f % 2) of ring[f / 2]: 0 = read the
-    // upstream entry from global memory, else (passes back << 9) | index of the
-    // upstream cell in its pass; for an out face f the same 16 bits hold, in
-    // bit j, class 0's source test for node j of that face (|x - (0.5, 0, 0)|
-    // < 0.05, evaluated once when the direction is set)
-    uint32_t ring[2];
+// Transport sweep (kernels_sweep.hip). Per direction, cells are taken in passes
+// whose upstream cells are in earlier passes; a pass has at most sweep_block() out
+// faces, one per thread of the direction's workgroup, and half as many cells. A
+// face value is kept at its position modulo the ring (kSweepRing passes of full
+// size) in LDS; where a value is read from is coded by the host: >= 0: ring slot;
+// kSweepZero, kSweepOne: that boundary value; <= kSweepFar: out of the ring by
+// then, entry kSweepFar - code of the result in global memory.
+constexpr int kSweepRing = 16;
+constexpr int32_t kSweepZero = -1, kSweepOne = -2, kSweepFar = -3;
+constexpr int kSweepCellBits = 29;  // cells < 2^29: entries 4 cell + face fit in int32
+constexpr uint32_t kSweepCellMask = (1u << kSweepCellBits) - 1;
+struct SweepFace {
+    uint32_t cell;  // bit 29 + j: class 0's source test for node j (|x - (0.5, 0, 0)| < 0.05)
+    int32_t up[3];  // codes of the nodes' in-face values
 };
 struct SweepDirDev {
-    const SweepPos* pos;   // [n] by position in level order
-    const double* s9;      // [n][kSweepRecStride] s of record slot q (0 where unused)
-    const int32_t* pass;   // [passes][2]: first position, count | (complete earlier stores first) << 31
+    const SweepFace* faces;  // by position
+    const double* s3;        // s of the three nodes: per pass [3][faces of the pass]
+    const int32_t* pass;     // [passes][4]: first face, faces, first cell, cells
+    const int32_t* codes;    // [cells][4] by pass: codes of the cell's four face values in the step after it
+    const int32_t* cells;    // cell numbers by pass
+    const int32_t* fix;      // [fixes][2] entries: first takes the value of second at the end
     int32_t passes;
     int32_t levels;
+    int32_t fixes;
 };
-hipError_t launch_sweep(int cls, const SweepDirDev* d_dirs, int m, int64_t n,
-                        const double* d_S, int64_t ld, const double* d_old, double* d_new, double* d_norm,
-                        hipStream_t st);
+// Threads per direction for a mean of `faces` out faces per level, m directions.
+int sweep_block(int64_t faces, int m, int cus);
+hipError_t launch_sweep(int cls, int block, const SweepDirDev* d_dirs, int m, int64_t n, const double* d_S, int64_t ld,
+                        const double* d_old, double* d_new, double* d_norm, hipStream_t st);
 // Resident-panel kernel (cell-level state only): plan and launch. Its result
 // stores address 16 output rows through one 32-bit buffer range, so the output
 // leading dimension must stay below kSplitResidentMaxLd cells.

@@ -1,6 +1,6 @@
 // Host side of the transport sweep: validates the reference-format sweep
 // structures of each direction (sorted_id_cell, face states, vec_x0 records),
-// derives the level of every cell, uploads everything once and launches the
+// plans the passes of the direction, uploads everything once and launches the
 // sweep kernel. Replaces ReadIllumGeometry's in-memory result
 // (file_module/reader_bin.cpp:164-203) and the direction loop of
 // MPI_CalculateIllumAsync (solve_module/illum/Illum_async.cpp:725-784).
@@ -10,11 +10,12 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
 
-#include "rsh_internal.hpp"
+#include "rsh_objects.hpp"
 #include "rsh_scatter.h"
 
 using namespace rsh;
@@ -23,17 +24,27 @@ struct rsh_sweep_s {
     int device = 0;
     int64_t n = 0;
     int m = 0;
+    int block = 0;  // threads per direction, out faces per pass at most; from the first direction set
     // class 0's source test per cell, bit 3 f + j for node j of face f (|x -
     // (0.5, 0, 0)| < 0.05, GetCurIllum's expression); empty without nodes
     std::vector<uint16_t> node_in_source;
-    std::vector<int32_t> pairs;  // host copy: validation, levels, per-position copies
+    std::vector<int32_t> pairs;  // host copy: validation, plans
     struct Dir {
         void* block = nullptr;  // one device allocation per direction
         SweepDirDev dev{};
-        int64_t records = 0;
         bool set = false;
     };
     std::vector<Dir> dirs;
+    // Host arrays of one direction's plan, kept for the next one (a call takes a
+    // set of its own: fresh pages would cost more than half of the planning).
+    struct Work {
+        std::vector<int64_t> x0_off;
+        std::vector<int32_t> pos, level, waits, chain, entries, cells, pos_of, pass_of, pass, touched, next, old, open,
+            codes, fix;
+        std::vector<SweepFace> faces;
+        std::vector<double> s3;
+    };
+    std::vector<std::unique_ptr<Work>> spare;
     SweepDirDev* d_table = nullptr;
     bool table_dirty = true;
     std::mutex mu;
@@ -100,13 +111,33 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     if (!s || k < 0 || k >= s->m || !order || !face_state || n_records < 0 || (n_records > 0 && (!x0_s || !x0_face)))
         return fail(RSH_E_ARG, "invalid direction, null pointer or record count");
     const int64_t n = s->n;
-    std::vector<int32_t> pos((size_t)n, -1), level((size_t)n, 0);
+    struct Lease {  // a Work of this call, given back at its end
+        rsh_sweep s;
+        std::unique_ptr<rsh_sweep_s::Work> w;
+        explicit Lease(rsh_sweep sw) : s(sw) {
+            std::lock_guard<std::mutex> lock(s->mu);
+            if (!s->spare.empty()) {
+                w = std::move(s->spare.back());
+                s->spare.pop_back();
+            }
+            if (!w) w = std::make_unique<rsh_sweep_s::Work>();
+        }
+        ~Lease() {
+            std::lock_guard<std::mutex> lock(s->mu);
+            s->spare.push_back(std::move(w));
+        }
+    } lease(s);
+    rsh_sweep_s::Work& w = *lease.w;
+    auto &pos = w.pos, &level = w.level;
+    pos.assign((size_t)n, -1);
+    level.assign((size_t)n, 0);
     for (int64_t h = 0; h < n; h++) {
         const int32_t c = order[h];
         if (c < 0 || c >= n || pos[(size_t)c] >= 0) return fail(RSH_E_ARG, "order is not a permutation of the cells");
         pos[(size_t)c] = (int32_t)h;
     }
-    std::vector<int64_t> x0_off((size_t)n);
+    auto& x0_off = w.x0_off;
+    x0_off.resize((size_t)n);
     int64_t r = 0;
     int32_t levels = 0;
     for (int64_t h = 0; h < n; h++) {
@@ -141,102 +172,174 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
         levels = std::max(levels, lv + 1);
     }
     if (r != n_records) return fail(RSH_E_ARG, "more x0 records than out-face nodes");
-    // Cells by level, ascending cell number inside a level (cells of one level
-    // are independent; neighbouring numbers share cache lines of the per-cell
-    // arrays the pass reads and writes).
-    std::vector<int32_t> level_ptr((size_t)levels + 1, 0), cells((size_t)n);
-    for (int64_t c = 0; c < n; c++) level_ptr[(size_t)level[(size_t)c] + 1]++;
-    for (int32_t l = 0; l < levels; l++) level_ptr[(size_t)l + 1] += level_ptr[(size_t)l];
-    std::vector<int32_t> fill(level_ptr.begin(), level_ptr.end() - 1);
-    for (int64_t c = 0; c < n; c++) cells[(size_t)fill[(size_t)level[(size_t)c]]++] = (int32_t)c;
-    // Per position in the level order: cell, face states, write-back faces (out
-    // on both sides with the neighbour earlier in the given order: the later
-    // writer wins both entries, as in the sequential walk), the in-face ids of
-    // the cell's records, its pairs; and the records' s values.
-    std::vector<SweepPos> posv((size_t)n);
-    std::vector<double> s9((size_t)n * kSweepRecStride, 0.0);
-    for (int64_t i = 0; i < n; i++) {
-        const int32_t c = cells[(size_t)i];
-        const int st = face_state[c];
-        uint32_t meta = (uint32_t)st;
-        SweepPos& P = posv[(size_t)i];
-        P.cell = c;
-        P.ring[0] = P.ring[1] = 0;
-        int q = 0;
-        for (int f = 0; f < 4; f++) {
-            const int32_t p = s->pairs[(size_t)(c * 4 + f)];
-            P.pr[f] = p;
-            if ((st >> f) & 1) continue;
-            if (p >= 0) {
-                const int32_t u = p / 4;
-                if (!((face_state[u] >> (p % 4)) & 1) && pos[(size_t)u] < pos[(size_t)c]) meta |= 1u << (4 + f);
+    // Cells read by a cell, and the longest chain of cells that still waits on it.
+    auto &waits = w.waits, &chain = w.chain;
+    waits.assign((size_t)n, 0);
+    chain.assign((size_t)n, 0);
+    auto reads = [&](int32_t c, int f) { return ((face_state[c] >> f) & 1) && s->pairs[(size_t)(c * 4 + f)] >= 0; };
+    for (int64_t h = n - 1; h >= 0; h--) {
+        const int32_t c = order[h];
+        for (int f = 0; f < 4; f++)
+            if (reads(c, f)) {
+                const int32_t u = s->pairs[(size_t)(c * 4 + f)] / 4;
+                waits[(size_t)c]++;
+                chain[(size_t)u] = std::max(chain[(size_t)u], chain[(size_t)c] + 1);
             }
-            if (!s->node_in_source.empty())
-                P.ring[f / 2] |= (uint32_t)((s->node_in_source[(size_t)c] >> (3 * f)) & 7u) << (16 * (f % 2));
-            for (int j = 0; j < 3; j++, q++) {
-                const int64_t r = x0_off[(size_t)c] + q;  // records of the cell in out-face order
-                s9[(size_t)(i * kSweepRecStride + q)] = x0_s[r];
-                meta |= (uint32_t)x0_face[r] << (8 + 2 * q);
-            }
-        }
-        P.meta = meta;
     }
-    std::vector<int32_t> pass;
-    for (int32_t l = 0; l < levels; l++)
-        for (int32_t b0 = level_ptr[(size_t)l]; b0 < level_ptr[(size_t)l + 1]; b0 += kSweepBlock) {
-            pass.push_back(b0);
-            pass.push_back(std::min(kSweepBlock, level_ptr[(size_t)l + 1] - b0));
-        }
-    const int32_t passes = (int32_t)(pass.size() / 2);
-    // Ring codes: an in face whose upstream cell was swept 1..kSweepRingDelta
-    // passes earlier reads that cell's values from the LDS ring. A pass that
-    // rewrites the entry of a cell swept one pass earlier (a face out on both
-    // sides) is flagged: the stores of the pass before it are completed ahead
-    // of its barrier, so that the later write lands last.
+    int block;
     {
-        std::vector<int32_t> pass_of((size_t)n), where((size_t)n);
-        for (int32_t pi = 0; pi < passes; pi++) {
-            const int32_t b0 = pass[(size_t)(2 * pi)], cnt = pass[(size_t)(2 * pi + 1)];
-            for (int32_t j = 0; j < cnt; j++) pass_of[(size_t)(b0 + j)] = pi;
-        }
-        for (int64_t i = 0; i < n; i++) where[(size_t)cells[(size_t)i]] = (int32_t)i;
-        for (int64_t i = 0; i < n; i++) {
-            SweepPos& P = posv[(size_t)i];
-            for (int f = 0; f < 4; f++) {
-                const int32_t p = P.pr[f];
-                if (p >= 0 && ((P.meta >> (4 + f)) & 1) &&
-                    pass_of[(size_t)i] - pass_of[(size_t)where[(size_t)(p / 4)]] == 1)
-                    pass[(size_t)(2 * pass_of[(size_t)i] + 1)] |= (int32_t)0x80000000u;
-                if (p < 0 || !((P.meta >> f) & 1)) continue;
-                const int32_t up = where[(size_t)(p / 4)];
-                const int32_t delta = pass_of[(size_t)i] - pass_of[(size_t)up];
-                if (delta < 1 || delta > kSweepRingDelta) continue;
-                const uint32_t code = ((uint32_t)delta << 9) | (uint32_t)(up - pass[(size_t)(2 * pass_of[(size_t)up])]);
-                P.ring[f / 2] |= code << (16 * (f % 2));
+        std::lock_guard<std::mutex> lock(s->mu);
+        if (!s->block) s->block = sweep_block(n_records / 3 / levels, s->m, device_cus(s->device));
+        block = s->block;
+    }
+    // Passes of at most block out faces and block / 2 cells whose upstream cells are in
+    // earlier passes. Taken first: cells of a group of kLineCells that an earlier
+    // pass touched, oldest group first (a 128-byte line of S, four of the result,
+    // is finished while it is in L2); then the cell with the longest chain behind
+    // it (fewest passes). Out faces have positions pass by pass, by cell and face.
+    constexpr int32_t kLineCells = 16;
+    auto &entries = w.entries, &cells = w.cells, &pos_of = w.pos_of, &pass_of = w.pass_of, &pass = w.pass;
+    entries.clear();
+    cells.clear();
+    pass.clear();
+    entries.reserve((size_t)n_records / 3);
+    cells.reserve((size_t)n + 1);
+    pos_of.assign((size_t)n * 4, -1);
+    pass_of.resize((size_t)n);
+    auto& cell_at = w.next;  // a cell taken is in no list any more
+    cell_at.resize((size_t)n);
+    auto out_faces = [&](int32_t c) { return 4 - __builtin_popcount((unsigned)face_state[c]); };
+    {
+        // ready cells as lists: by the pass that touched their group, by their chain
+        auto &touched = w.touched, &next = w.next, &old = w.old, &open = w.open;
+        touched.assign((size_t)(n / kLineCells + 1), -1);
+        old.clear();
+        open.assign((size_t)levels, -1);
+        int32_t oldest = 0, longest = -1;
+        auto push = [&](int32_t c) {
+            const int32_t t = touched[(size_t)(c / kLineCells)], l = chain[(size_t)c];
+            int32_t& head = t >= 0 ? old[(size_t)t] : open[(size_t)l];
+            if (t >= 0) oldest = std::min(oldest, t);
+            else longest = std::max(longest, l);
+            next[(size_t)c] = head;
+            head = c;
+        };
+        auto top = [&]() -> int32_t* {
+            while (oldest < (int32_t)old.size() && old[(size_t)oldest] < 0) oldest++;
+            if (oldest < (int32_t)old.size()) return &old[(size_t)oldest];
+            while (longest >= 0 && open[(size_t)longest] < 0) longest--;
+            return longest >= 0 ? &open[(size_t)longest] : nullptr;
+        };
+        for (int32_t c = (int32_t)n - 1; c >= 0; c--)
+            if (!waits[(size_t)c]) push(c);
+        for (int32_t p = 0; top(); p++) {
+            const size_t first = cells.size();
+            const int32_t face0 = (int32_t)entries.size();
+            int32_t cnt = 0;
+            old.push_back(-1);
+            for (int32_t* head; (int32_t)(cells.size() - first) < block / 2 && (head = top());) {
+                const int32_t c = *head;
+                if ((cnt += out_faces(c)) > block) break;
+                *head = next[(size_t)c];
+                int32_t& t = touched[(size_t)(c / kLineCells)];
+                if (t < 0) t = p;
+                cells.push_back(c);
             }
+            std::sort(cells.begin() + (int64_t)first, cells.end());
+            for (size_t i = first; i < cells.size(); i++) {
+                const int32_t c = cells[i];
+                pass_of[(size_t)c] = p;
+                cell_at[(size_t)c] = (int32_t)i;
+                for (int f = 0; f < 4; f++)
+                    if (!((face_state[c] >> f) & 1)) {
+                        const int32_t q = s->pairs[(size_t)(c * 4 + f)];
+                        pos_of[(size_t)(c * 4 + f)] = (int32_t)entries.size();
+                        entries.push_back(c * 4 + f);
+                        if (q >= 0 && reads(q / 4, q % 4) && --waits[(size_t)(q / 4)] == 0) push(q / 4);
+                    }
+            }
+            pass.insert(pass.end(), {face0, (int32_t)entries.size() - face0, (int32_t)first, (int32_t)(cells.size() - first)});
         }
     }
+    // one more, empty: the last pass's cells are stored in the step after it
+    pass.insert(pass.end(), {(int32_t)entries.size(), 0, (int32_t)n, 0});
+    const int32_t passes = (int32_t)(pass.size() / 4);
+    // Code of an entry's value at step `step`: its own position's for an out face,
+    // the neighbour's for an in face.
+    const int64_t ring = (int64_t)block * kSweepRing;
+    auto code_of = [&](int32_t e, int32_t step) -> int32_t {
+        const int32_t up = s->pairs[(size_t)e];
+        int32_t src = e;
+        if ((face_state[e / 4] >> (e % 4)) & 1) {
+            if (up < 0) return up == RSH_BOUND_OUT_SOURCE ? kSweepOne : kSweepZero;
+            src = up;
+        }
+        const int64_t end = (int64_t)pass[(size_t)step * 4] + pass[(size_t)step * 4 + 1];
+        return pos_of[(size_t)src] >= end - ring ? (int32_t)(pos_of[(size_t)src] & (ring - 1)) : kSweepFar - src;
+    };
+    // one record more than used: threads without work load the one after the last
+    auto& faces = w.faces;
+    auto& s3 = w.s3;
+    auto &codes = w.codes, &fix = w.fix;
+    faces.resize(entries.size() + 1);
+    faces.back() = SweepFace{0, {kSweepZero, kSweepZero, kSweepZero}};
+    s3.resize((entries.size() + 1) * 3);
+    for (int j = 1; j <= 3; j++) s3[s3.size() - (size_t)j] = 0.0;
+    codes.resize((size_t)(n + 1) * 4);
+    for (int j = 1; j <= 4; j++) codes[codes.size() - (size_t)j] = kSweepZero;
+    fix.clear();
+    for (int64_t h = 0; h < n; h++) {
+        const int32_t c = order[h], i = cell_at[(size_t)c], p = pass_of[(size_t)c];
+        const int64_t first = pass[(size_t)p * 4], cnt = pass[(size_t)p * 4 + 1];
+        int64_t r = x0_off[(size_t)c];  // records of the cell in out-face order
+        for (int f = 0; f < 4; f++) {
+            const int32_t e = c * 4 + f;
+            codes[(size_t)i * 4 + (size_t)f] = code_of(e, p + 1);
+            const int32_t at = pos_of[(size_t)e];
+            if (at < 0) continue;
+            SweepFace& F = faces[(size_t)at];
+            F.cell = (uint32_t)c;
+            if (!s->node_in_source.empty())
+                F.cell |= (uint32_t)((s->node_in_source[(size_t)c] >> (3 * f)) & 7u) << kSweepCellBits;
+            for (int j = 0; j < 3; j++, r++) {
+                F.up[j] = code_of(c * 4 + x0_face[r], p);
+                s3[(size_t)(first * 3 + j * cnt + at - first)] = x0_s[r];
+            }
+            // a face out on both sides: the later cell in the given order wins
+            const int32_t q = s->pairs[(size_t)e];
+            if (q >= 0 && pos_of[(size_t)q] >= 0 && pos[(size_t)(q / 4)] < pos[(size_t)c]) fix.insert(fix.end(), {q, e});
+        }
+    }
+    cells.push_back(0);
 
-    const size_t b_pos = align256((size_t)n * sizeof(SweepPos)), b_s9 = align256((size_t)n * kSweepRecStride * 8),
-                 b_pass = align256(pass.size() * 4);
+    const size_t b_faces = align256(faces.size() * sizeof(SweepFace)), b_s3 = align256(s3.size() * 8),
+                 b_pass = align256(pass.size() * 4), b_codes = align256(codes.size() * 4),
+                 b_cells = align256(cells.size() * 4), b_fix = align256(fix.size() * 4);
     std::lock_guard<std::mutex> lock(s->mu);
     RSH_HIP_TRY(hipSetDevice(s->device));
     auto& d = s->dirs[(size_t)k];
     if (d.block) RSH_HIP_TRY(hipFree(d.block));
     d.block = nullptr;
     d.set = false;
-    if (hipMalloc(&d.block, b_pos + b_s9 + b_pass) != hipSuccess)
+    if (hipMalloc(&d.block, b_faces + b_s3 + b_pass + b_codes + b_cells + b_fix) != hipSuccess)
         return fail(RSH_E_NOMEM, "sweep: direction allocation failed");
-    char* base = static_cast<char*>(d.block);
-    RSH_HIP_TRY(hipMemcpy(base, posv.data(), (size_t)n * sizeof(SweepPos), hipMemcpyHostToDevice));
-    RSH_HIP_TRY(hipMemcpy(base + b_pos, s9.data(), (size_t)n * kSweepRecStride * 8, hipMemcpyHostToDevice));
-    RSH_HIP_TRY(hipMemcpy(base + b_pos + b_s9, pass.data(), pass.size() * 4, hipMemcpyHostToDevice));
-    d.dev.pos = reinterpret_cast<const SweepPos*>(base);
-    d.dev.s9 = reinterpret_cast<const double*>(base + b_pos);
-    d.dev.pass = reinterpret_cast<const int32_t*>(base + b_pos + b_s9);
+    char* at = static_cast<char*>(d.block);
+    auto put = [&](const void* src, size_t bytes, size_t room) {
+        char* dst = at;
+        at += room;
+        return !bytes || hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess ? dst : nullptr;
+    };
+    d.dev.faces = reinterpret_cast<const SweepFace*>(put(faces.data(), faces.size() * sizeof(SweepFace), b_faces));
+    d.dev.s3 = reinterpret_cast<const double*>(put(s3.data(), s3.size() * 8, b_s3));
+    d.dev.pass = reinterpret_cast<const int32_t*>(put(pass.data(), pass.size() * 4, b_pass));
+    d.dev.codes = reinterpret_cast<const int32_t*>(put(codes.data(), codes.size() * 4, b_codes));
+    d.dev.cells = reinterpret_cast<const int32_t*>(put(cells.data(), cells.size() * 4, b_cells));
+    d.dev.fix = reinterpret_cast<const int32_t*>(put(fix.data(), fix.size() * 4, b_fix));
+    if (!d.dev.faces || !d.dev.s3 || !d.dev.pass || !d.dev.codes || !d.dev.cells || !d.dev.fix)
+        return fail(RSH_E_HIP, "sweep: upload of a direction failed");
     d.dev.passes = passes;
     d.dev.levels = levels;
-    d.records = n_records;
+    d.dev.fixes = (int32_t)(fix.size() / 2);
     d.set = true;
     s->table_dirty = true;
     return RSH_OK;
@@ -270,8 +373,8 @@ int rsh_sweep_run(rsh_sweep s, int32_t cls, const double* d_scattering, int64_t 
         RSH_HIP_TRY(hipMemcpy(s->d_table, table.data(), table.size() * sizeof(SweepDirDev), hipMemcpyHostToDevice));
         s->table_dirty = false;
     }
-    RSH_HIP_TRY(launch_sweep(cls, s->d_table, s->m, s->n, d_scattering, ld, d_illum_old, d_illum_new,
-                             d_norm, st));
+    RSH_HIP_TRY(launch_sweep(cls, s->block, s->d_table, s->m, s->n, d_scattering, ld, d_illum_old,
+                             d_illum_new, d_norm, st));
     return RSH_OK;
 }
 

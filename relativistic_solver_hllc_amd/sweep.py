@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 from concurrent.futures import ThreadPoolExecutor
+from itertools import islice
 from typing import List, Optional, Tuple
 
 import numpy as np
@@ -228,8 +229,14 @@ class Sweep:
                _p(f) if f.size else None, ss.size)
 
     def set_all(self, per_dir) -> None:
-        for k, d in enumerate(per_dir):
+        # Direction 0 alone (the workgroup size follows from it), then eight at a
+        # time: planning a direction is host work outside the library's lock.
+        it = iter(enumerate(per_dir))
+        for k, d in islice(it, 1):
             self.set_direction(k, *d)
+        with ThreadPoolExecutor(max_workers=8) as ex:
+            while some := list(islice(it, 8)):
+                list(ex.map(lambda kd: self.set_direction(kd[0], *kd[1]), some))
 
     def levels(self, k: int) -> int:
         v = C.c_int32()

@@ -70,6 +70,29 @@ def test_sweep_matches_oracle(gpu, ne, m, cls):
     assert norm.max() == pytest.approx(ref_norm, rel=1e-10) if np.isfinite(ref_norm) else np.isinf(norm.max())
 
 
+@pytest.mark.parametrize("ne,first", [(1, 3), (8, 9), (10, 9), (12, 3), (14, 3)])
+def test_sweep_workgroup_sizes_match_oracle(gpu, ne, first):
+    """128 to 1024 threads per direction (taken from the first direction's faces per level: 4, 114, 179, 432 and 588)
+    on a mesh with shuffled cell numbers. With 128 threads on 3072 cells the axis directions reach past the LDS
+    ring; they also hold the faces out on both sides."""
+    v, pairs = sw.mesh_cube_tetra(ne)
+    n = v.shape[0]
+    perm = np.random.default_rng(ne).permutation(n)
+    inv = np.argsort(perm)
+    pairs = np.where(pairs >= 0, inv[np.maximum(pairs, 0) // 4] * 4 + np.maximum(pairs, 0) % 4, pairs)[perm]
+    v, pairs = v[perm], pairs.astype(np.int32)
+    xyz, _, _ = rs.fibonacci_directions(26)
+    dirs = np.vstack([xyz[[first, 0, 20]], six_axis()])
+    per = sw.prepare(v, pairs, dirs)
+    rng = np.random.default_rng(100 + ne)
+    S = rng.lognormal(size=(len(dirs), n))
+    old = rng.lognormal(size=(len(dirs), n, 4))
+    ref, ref_norm = orc.sweep(per, pairs, S, old, cls=1)
+    got, norm, _ = gpu_sweep(v, pairs, per, S, old, 1)
+    check(got, ref)
+    assert norm.max() == pytest.approx(ref_norm, rel=1e-10) if np.isfinite(ref_norm) else np.isinf(norm.max())
+
+
 @pytest.mark.parametrize("cls", [1, 0])
 def test_sweep_on_reference_placement_matches_oracle(gpu, cls):
     """The sweep fed the records of the reference's own MAKE step (its VTK face numbering, node placement and
