@@ -71,24 +71,10 @@ __device__ inline double cell_sum(double x) {
     return x;
 }
 
-template <int FACES, int FPT, int PIPE>
-__global__ __launch_bounds__(kMomentBlock) void moments_f64_kernel(
-    const double* __restrict__ illum, int64_t n, int m, const double* __restrict__ psi,
-    const double* __restrict__ normals, const double* __restrict__ areas, const double* __restrict__ volume,
-    double* __restrict__ energy, double* __restrict__ stream, double* __restrict__ impuls,
-    double* __restrict__ divstream, double* __restrict__ divimpuls) {
-    constexpr int TPC = FACES / FPT;
-    const int64_t gid = (int64_t)blockIdx.x * kMomentBlock + threadIdx.x;
-    const int64_t cell = gid / TPC;
-    const int fg = (int)(gid % TPC);
-    const bool active = cell < n;
-    // Lanes past the last cell read the last cell (in bounds) and write nothing,
-    // so every lane of a cell group takes part in the shuffles.
-    const int64_t c = active ? cell : n - 1;
-    const double* __restrict__ src = illum + c * FACES + fg * FPT;
-    const int64_t stride = n * FACES;
-
-    double acc[FPT][kMomentFuncs];
+// Sums over the direction rows j0 .. j1 - 1 (at least one) of a thread's faces.
+template <int FPT, int PIPE>
+__device__ inline void sum_rows(const double* __restrict__ src, int64_t stride, int j0, int j1,
+                                const double* __restrict__ psi, double (&acc)[FPT][kMomentFuncs]) {
 #pragma unroll
     for (int f = 0; f < FPT; f++)
 #pragma unroll
@@ -98,76 +84,157 @@ __global__ __launch_bounds__(kMomentBlock) void moments_f64_kernel(
     // row j is consumed (indices past the end re-read the last row, in bounds).
     double ring[PIPE][FPT];
 #pragma unroll
-    for (int u = 0; u < PIPE; u++) load_faces<FPT>(src + (int64_t)(u < m ? u : m - 1) * stride, ring[u]);
-    int j = 0;
-    for (; j + PIPE <= m; j += PIPE) {
+    for (int u = 0; u < PIPE; u++) load_faces<FPT>(src + (int64_t)(j0 + u < j1 ? j0 + u : j1 - 1) * stride, ring[u]);
+    int j = j0;
+    for (; j + PIPE <= j1; j += PIPE) {
 #pragma unroll
         for (int u = 0; u < PIPE; u++) {
             double v[FPT];
 #pragma unroll
             for (int f = 0; f < FPT; f++) v[f] = ring[u][f];
             const int jn = j + u + PIPE;
-            load_faces<FPT>(src + (int64_t)(jn < m ? jn : m - 1) * stride, ring[u]);
+            load_faces<FPT>(src + (int64_t)(jn < j1 ? jn : j1 - 1) * stride, ring[u]);
             accumulate<FPT>(psi + (j + u) * kMomentFuncs, v, acc);
         }
     }
 #pragma unroll
     for (int u = 0; u < PIPE; u++)
-        if (j + u < m) accumulate<FPT>(psi + (j + u) * kMomentFuncs, ring[u], acc);
+        if (j + u < j1) accumulate<FPT>(psi + (j + u) * kMomentFuncs, ring[u], acc);
+}
 
-    double e = 0.0, s[3] = {0.0, 0.0, 0.0}, t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double ds = 0.0, di[3] = {0.0, 0.0, 0.0};
-    const bool want_div = divstream != nullptr || divimpuls != nullptr;
+// Sums of one cell: energy, flux, pressure tensor and the two divergences, each
+// before its factor. The thread's FPT faces, then all lanes of the cell.
+constexpr int kCellSums = 14;
+template <int FACES, int FPT>
+__device__ inline void cell_sums(const double (&acc)[FPT][kMomentFuncs], int64_t c, int fg, bool want_div,
+                                 const double* __restrict__ normals, const double* __restrict__ areas,
+                                 double (&x)[kCellSums]) {
+    constexpr int TPC = FACES / FPT;
+#pragma unroll
+    for (int q = 0; q < kCellSums; q++) x[q] = 0.0;
 #pragma unroll
     for (int f = 0; f < FPT; f++) {
         const double* a = acc[f];
-        e += a[0];
-        s[0] += a[1]; s[1] += a[2]; s[2] += a[3];
 #pragma unroll
-        for (int q = 0; q < 6; q++) t[q] += a[4 + q];
+        for (int q = 0; q < kMomentFuncs; q++) x[q] += a[q];
         if (want_div) {
             const int64_t cf = c * FACES + fg * FPT + f;
             const double nx = normals[3 * cf], ny = normals[3 * cf + 1], nz = normals[3 * cf + 2];
             const double ar = areas[cf];
-            ds += (a[1] * nx + a[2] * ny + a[3] * nz) * ar;
-            di[0] += (a[4] * nx + a[5] * ny + a[6] * nz) * ar;
-            di[1] += (a[5] * nx + a[7] * ny + a[8] * nz) * ar;
-            di[2] += (a[6] * nx + a[8] * ny + a[9] * nz) * ar;
+            x[10] += (a[1] * nx + a[2] * ny + a[3] * nz) * ar;
+            x[11] += (a[4] * nx + a[5] * ny + a[6] * nz) * ar;
+            x[12] += (a[5] * nx + a[7] * ny + a[8] * nz) * ar;
+            x[13] += (a[6] * nx + a[8] * ny + a[9] * nz) * ar;
         }
     }
     if constexpr (TPC > 1) {
-        e = cell_sum<TPC>(e);
 #pragma unroll
-        for (int k = 0; k < 3; k++) s[k] = cell_sum<TPC>(s[k]);
-#pragma unroll
-        for (int q = 0; q < 6; q++) t[q] = cell_sum<TPC>(t[q]);
+        for (int q = 0; q < 10; q++) x[q] = cell_sum<TPC>(x[q]);
         if (want_div) {
-            ds = cell_sum<TPC>(ds);
 #pragma unroll
-            for (int k = 0; k < 3; k++) di[k] = cell_sum<TPC>(di[k]);
+            for (int q = 10; q < kCellSums; q++) x[q] = cell_sum<TPC>(x[q]);
         }
     }
-    if (!active || fg != 0) return;
+}
+
+struct MomentOut {
+    double *energy, *stream, *impuls, *divstream, *divimpuls;
+};
+
+// Stores what one cell sum contributes to: q as in cell_sums.
+template <int FACES>
+__device__ inline void store_sum(const MomentOut& o, int64_t cell, int q, double x, double vol) {
     constexpr double inv_faces = 1.0 / FACES;  // FACES is 1 or 4: exact
-    if (energy) energy[cell] = e * inv_faces;
-    if (stream) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) stream[3 * cell + k] = s[k] * inv_faces;
-    }
-    if (impuls) {
+    if (q == 0) {
+        if (o.energy) o.energy[cell] = x * inv_faces;
+    } else if (q < 4) {
+        if (o.stream) o.stream[3 * cell + q - 1] = x * inv_faces;
+    } else if (q < 10) {
+        if (!o.impuls) return;
         // row-major 3x3 of the symmetric tensor (xx xy xz / xy yy yz / xz yz zz)
-        constexpr int map[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
-#pragma unroll
-        for (int q = 0; q < 9; q++) impuls[9 * cell + q] = t[map[q]] * inv_faces;
+        const int r = q < 7 ? 0 : q < 9 ? 1 : 2, k = q < 7 ? q - 4 : q < 9 ? q - 6 : 2;
+        o.impuls[9 * cell + 3 * r + k] = x * inv_faces;
+        if (r != k) o.impuls[9 * cell + 3 * k + r] = x * inv_faces;
+    } else if (q == 10) {
+        if (o.divstream) o.divstream[cell] = x / vol;
+    } else if (o.divimpuls) {
+        o.divimpuls[3 * cell + q - 11] = x / vol;
     }
-    if (want_div) {
-        const double vol = volume[cell];
-        if (divstream) divstream[cell] = ds / vol;
-        if (divimpuls) {
+}
+
+template <int FACES, int FPT, int PIPE>
+__global__ __launch_bounds__(kMomentBlock) void moments_f64_kernel(
+    const double* __restrict__ illum, int64_t n, int m, const double* __restrict__ psi,
+    const double* __restrict__ normals, const double* __restrict__ areas, const double* __restrict__ volume,
+    MomentOut out) {
+    constexpr int TPC = FACES / FPT;
+    const int64_t gid = (int64_t)blockIdx.x * kMomentBlock + threadIdx.x;
+    const int64_t cell = gid / TPC;
+    const int fg = (int)(gid % TPC);
+    const bool active = cell < n;
+    // Lanes past the last cell read the last cell (in bounds) and write nothing,
+    // so every lane of a cell group takes part in the shuffles.
+    const int64_t c = active ? cell : n - 1;
+    double acc[FPT][kMomentFuncs], x[kCellSums];
+    sum_rows<FPT, PIPE>(illum + c * FACES + fg * FPT, n * FACES, 0, m, psi, acc);
+    const bool want_div = out.divstream || out.divimpuls;
+    cell_sums<FACES, FPT>(acc, c, fg, want_div, normals, areas, x);
+    if (!active || fg != 0) return;
+    const double vol = want_div ? volume[cell] : 1.0;
 #pragma unroll
-            for (int k = 0; k < 3; k++) divimpuls[3 * cell + k] = di[k] / vol;
-        }
+    for (int q = 0; q < kCellSums; q++) store_sum<FACES>(out, cell, q, x[q], vol);
+}
+
+// Few cells: the directions are split over the SLICES waves of a workgroup, which
+// all take the same 64 threads' faces; the slices' cell sums are added in order
+// through LDS, one thread per sum. What bounds the plain kernel there is one
+// thread's chain of rows (four in flight, ~0.5 us per round trip). us per call with
+// 1 / 2 / 4 / 8 / 16 slices (cells x directions, two faces per thread):
+//     528 x 294: 36.4 / 18.0 / 10.5 / 8.4 / 8.0    1733 x 265: 46.1 / 20.8 / 12.4 / 8.7 / 9.0
+//    3762 x 73:  14.7 /  8.4 /  6.0 / 5.4 / 6.0    9000 x 400: 69.0 / 37.6 / 23.0 / 25.2 / 27.5
+//   17170 x 294: 55.2 / 32.1 / 31.2 / 33.7 / 37.3  36000 x 200: 43.9 / 38.6 / 40.2 / 42.4 / 51.6
+//   48000 x 200: 49.1 / 50.1 / 52.8 / 53.7 / 65.6  65536 x 200: 65.7 / 76.2 / 80.1 / 84.3 / 93.8
+// Eight rows in flight instead of four: within 10 % either way.
+template <int FACES, int FPT, int PIPE, int SLICES>
+__global__ __launch_bounds__(64 * SLICES) void moments_f64_sliced_kernel(
+    const double* __restrict__ illum, int64_t n, int m, const double* __restrict__ psi,
+    const double* __restrict__ normals, const double* __restrict__ areas, const double* __restrict__ volume,
+    MomentOut out) {
+    constexpr int TPC = FACES / FPT, CELLS = 64 / TPC;
+    __shared__ double part[SLICES][kCellSums][CELLS];
+    const int lane = threadIdx.x & 63, slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t first = (int64_t)blockIdx.x * CELLS;
+    const int fg = lane % TPC, cl = lane / TPC;
+    const int64_t c = first + cl < n ? first + cl : n - 1;
+    const bool want_div = out.divstream || out.divimpuls;
+    // the host gives every slice at least one row: m >= SLICES
+    const int j0 = (int)((int64_t)m * slice / SLICES), j1 = (int)((int64_t)m * (slice + 1) / SLICES);
+    double acc[FPT][kMomentFuncs], x[kCellSums];
+    sum_rows<FPT, PIPE>(illum + c * FACES + fg * FPT, n * FACES, j0, j1, psi, acc);
+    cell_sums<FACES, FPT>(acc, c, fg, want_div, normals, areas, x);
+    if (fg == 0) {
+#pragma unroll
+        for (int q = 0; q < kCellSums; q++) part[slice][q][cl] = x[q];
     }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kCellSums * CELLS; i += 64 * SLICES) {
+        const int q = i / CELLS;
+        const int64_t cell = first + i % CELLS;
+        if (cell >= n || (q >= 10 && !want_div)) continue;
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < SLICES; w++) sum += part[w][q][i % CELLS];
+        store_sum<FACES>(out, cell, q, sum, q >= 10 ? volume[cell] : 1.0);
+    }
+}
+
+// Slices of the directions: doubled while the chip has fewer than five waves per CU
+// (1280) and a slice keeps at least eight rows, by the times above.
+static int moment_slices(int64_t threads, int m) {
+    const int64_t waves = (threads + 63) / 64;
+    int s = 1;
+    while (s < 16 && waves * s < 1280 && m >= 16 * s) s *= 2;
+    return s;
 }
 
 hipError_t launch_moments_f64(const double* d_illum, int faces, int64_t n, int m, const double* d_psi,
@@ -178,16 +245,31 @@ hipError_t launch_moments_f64(const double* d_illum, int faces, int64_t n, int m
     const int fpt = faces == 1 ? 1 : faces_per_thread;
     const int64_t threads = n * (faces / fpt);
     const dim3 grid((unsigned)((threads + kMomentBlock - 1) / kMomentBlock)), block(kMomentBlock);
-#define RSH_MOM(FA, FP)                                                                                        \
-    hipLaunchKernelGGL((moments_f64_kernel<FA, FP, kMomentPipe>), grid, block, 0, st, d_illum, n, m, d_psi,   \
-                       d_normals, d_areas, d_volume, d_energy, d_stream, d_impuls, d_divstream, d_divimpuls)
-    if (faces == 1) RSH_MOM(1, 1);
-    else if (fpt == 4) RSH_MOM(4, 4);
-    else if (fpt == 2) RSH_MOM(4, 2);
-    else if (fpt == 1) RSH_MOM(4, 1);
-    else return hipErrorInvalidValue;
+    const MomentOut out{d_energy, d_stream, d_impuls, d_divstream, d_divimpuls};
+    const int slices = moment_slices(threads, m);
+#define RSH_MOM_SLICED(FA, FP, S)                                                                                  \
+    if (slices == S) {                                                                                             \
+        hipLaunchKernelGGL((moments_f64_sliced_kernel<FA, FP, kMomentPipe, S>), dim3((unsigned)((threads + 63) / 64)), \
+                           dim3(64 * S), 0, st, d_illum, n, m, d_psi, d_normals, d_areas, d_volume, out);          \
+        return hipGetLastError();                                                                                  \
+    }
+#define RSH_MOM(FA, FP)                                                                                           \
+    if (faces == FA && fpt == FP) {                                                                               \
+        RSH_MOM_SLICED(FA, FP, 2)                                                                                 \
+        RSH_MOM_SLICED(FA, FP, 4)                                                                                 \
+        RSH_MOM_SLICED(FA, FP, 8)                                                                                 \
+        RSH_MOM_SLICED(FA, FP, 16)                                                                                \
+        hipLaunchKernelGGL((moments_f64_kernel<FA, FP, kMomentPipe>), grid, block, 0, st, d_illum, n, m, d_psi,  \
+                           d_normals, d_areas, d_volume, out);                                                    \
+        return hipGetLastError();                                                                                 \
+    }
+    RSH_MOM(1, 1)
+    RSH_MOM(4, 4)
+    RSH_MOM(4, 2)
+    RSH_MOM(4, 1)
 #undef RSH_MOM
-    return hipGetLastError();
+#undef RSH_MOM_SLICED
+    return hipErrorInvalidValue;
 }
 
 }  // namespace rsh

@@ -81,6 +81,22 @@ def test_moments_match_oracle_ragged(gpu, n, fpt):
     check(got, ref, illum, w, F, areas, volume)
 
 
+@pytest.mark.parametrize("n,m,faces,fpt", [(1, 15, 4, 2), (1, 16, 4, 2), (31, 32, 4, 2), (33, 67, 4, 1), (17, 128, 4, 4),
+                                           (65, 131, 1, 1), (3000, 259, 4, 2), (40928, 17, 4, 2), (40960, 17, 4, 2)])
+def test_moments_split_directions_match_oracle(gpu, n, m, faces, fpt):
+    """1 to 16 slices of the directions (15 / 16 / 32 / 64 / 128 directions and 1280 waves are the edges), summed in
+    another order than one thread does: m terms, each within 2^-53 of e, stay below the tolerance for m < 1000."""
+    rng = np.random.default_rng(n + m)
+    xyz, w, F = rs.fibonacci_directions(m)
+    normals, areas, volume, _ = random_tetra_cells(n, rng)
+    illum = rng.lognormal(0.0, 1.0, size=(m, n, faces))
+    which = tuple(WIDTH) if faces == 4 else ("energy", "stream", "impuls")
+    ref = orc.moments(illum, xyz, w, F, *((normals, areas, volume) if faces == 4 else ()), which=which, threads=8)
+    with rs.DirectionSet(xyz, w, F) as ds:
+        got = run(ds, illum, *((normals, areas, volume) if faces == 4 else ()), fpt=fpt, which=which)
+    check(got, ref, illum, w, F, areas, volume)
+
+
 def test_moments_24576x200_sizes(gpu):
     """24,576 cells (16^3 x 6), M = 200 Fibonacci directions, log-normal(0, 1) faces."""
     n, m = 6 * 16 ** 3, 200
