@@ -31,15 +31,17 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", f"-I{RE
 
 HIP_SOURCES = ["kernels_f64.hip", "kernels_f64_reg.hip", "kernels_split.hip", "kernels_iter.hip", "kernels_iter_split.hip",
                "kernels_moments.hip", "kernels_split_resident.hip", "kernels_sweep.hip", "kernels_peak.hip", "noalloc.hip"]
-# Grouped split iteration: an unrolled instance per K-step count and form, in six units that compile in parallel.
-ITER_RES_SOURCES = [f"kernels_iter_res_{form}_{part}.hip" for form in ("bf16x2", "fp16x2", "bf16x3") for part in "ab"]
-HIP_SOURCES = ["kernels_split_resident.hip", *ITER_RES_SOURCES,
+# Resident-panel split kernels, grouped iteration and single problem: an unrolled instance per K-step count and form,
+# in twelve units that compile in parallel.
+RES_SOURCES = [f"kernels_{kind}_{form}_{part}.hip" for kind in ("iter_res", "res")
+               for form in ("bf16x2", "fp16x2", "bf16x3") for part in "ab"]
+HIP_SOURCES = ["kernels_split_resident.hip", *RES_SOURCES,
                *(s for s in HIP_SOURCES if s != "kernels_split_resident.hip")]  # longest first
 HOST_SOURCES = ["capi.cpp", "batch.cpp", "server.cpp", "sweep.cpp", "sweep_prep.cpp"]
 # Per-source device flags. The resident-panel split kernels add each K-step's
 # fresh FP32 products to its main sums with VALU adds: with MFMA results in
 # VGPRs (instead of AGPRs read back one register at a time) it ran 3-8 % faster.
-EXTRA_FLAGS = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for s in ["kernels_split_resident.hip", *ITER_RES_SOURCES]}
+EXTRA_FLAGS = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for s in ["kernels_split_resident.hip", *RES_SOURCES]}
 
 # Drop-in shim of the reference's cuda_solve.h names (stand-alone types) and the
 # test driver that replays the reference's call sequence through it.

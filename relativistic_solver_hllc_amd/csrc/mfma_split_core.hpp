@@ -93,23 +93,24 @@ __device__ __forceinline__ double swap_pair_lanes(double v) {
 // Stores two adjacent output cells (first at byte offset voff + soff of the
 // buffer, second after it) with one 16-byte (FP64) or 8-byte (FP32) store when
 // both are inside the output (both), the first alone when only it is (one).
+template <int AUX>
 __device__ __forceinline__ void store_cell_pair(double first, double second, bool both, bool one,
                                                 __amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
     if (both) {
         const v2u a = __builtin_bit_cast(v2u, first), b = __builtin_bit_cast(v2u, second);
-        __builtin_amdgcn_raw_buffer_store_b128(v4u{a[0], a[1], b[0], b[1]}, rsrc, voff, soff, kNontemporal);
+        __builtin_amdgcn_raw_buffer_store_b128(v4u{a[0], a[1], b[0], b[1]}, rsrc, voff, soff, AUX);
     } else if (one) {
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, first), rsrc, voff, soff, kNontemporal);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, first), rsrc, voff, soff, AUX);
     }
 }
+template <int AUX>
 __device__ __forceinline__ void store_cell_pair(float first, float second, bool both, bool one,
                                                 __amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
     if (both)
         __builtin_amdgcn_raw_buffer_store_b64(
-            v2u{__builtin_bit_cast(unsigned, first), __builtin_bit_cast(unsigned, second)}, rsrc, voff, soff,
-            kNontemporal);
+            v2u{__builtin_bit_cast(unsigned, first), __builtin_bit_cast(unsigned, second)}, rsrc, voff, soff, AUX);
     else if (one)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, first), rsrc, voff, soff, kNontemporal);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, first), rsrc, voff, soff, AUX);
 }
 
 template <int FMT>

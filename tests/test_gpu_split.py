@@ -155,6 +155,42 @@ def test_resident_panel_kernel_bit_identical(gpu, form, n, m, k0, k1):
         assert mx <= TOL[form][0] and mean <= TOL[form][1], (mx, mean)
 
 
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("steps", range(1, 26))
+def test_resident_workgroup_forms_bit_identical(gpu, steps, three):
+    """Every K-step count's resident plan, with either count of row blocks, in the workgroup forms: one tile per wave
+    up to 1 (3 for three parts) rounds of 128 cells per set, then 2 or 4 tiles per wave; FP64 rows with and without
+    whole 128-byte lines. The streaming kernel sums the same products in the same order: equal bits."""
+    form = "bf16x3" if three else ("bf16x2", "fp16x2")[steps % 2]
+    m = 32 * steps - (19 if steps % 3 == 0 else 3)
+    need, fit = (m + 15) // 16, min(5, 163840 // (steps * 2048 + 64))
+    groups = -(-need // fit)
+    rbw = -(-need // groups)
+    slots = 8 * (32 // -(-need // rbw))  # sets of the chip's 8 x 32 CUs
+    sizes = [3 * 128 * slots, 3 * 128 * slots + 1] if three else [128 * slots, 1024 * slots + 16]
+    n_max = max(sizes)
+    cell = np.resize(np.random.default_rng(steps).lognormal(0.0, 1.5, size=1_000_003), (m, n_max, 1))
+    xyz, w, F = rs.fibonacci_directions(m)
+    with rs.DirectionSet(xyz, w, F, phase="hg", g=0.8, normalize=True) as ds:
+        for n in sizes:
+            d_cell = D.DeviceArray.from_host(np.ascontiguousarray(cell[:, :n]))
+            sb, cb = rs.split_sizes(form, 1, n, m)
+            state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+            rs.pack_split_dev(form, d_cell, 1, n, m, state, scale)
+            for f32, ld in ((False, n), (True, n + 3)):
+                outs = []
+                for waves in (1, 8):
+                    out = D.DeviceArray.from_host(np.full((m, ld), -1.0, np.float32 if f32 else np.float64))
+                    ds.scatter_split(form, state, scale, 1, n, 0, m, out, ld=ld, out_f32=f32, waves=waves)
+                    D.synchronize()
+                    outs.append(out.to_host())
+                    out.free()
+                assert np.array_equal(outs[0], outs[1]), (n, f32)
+                assert np.all(outs[0][:, n:] == -1.0)
+            for a in (d_cell, state, scale):
+                a.free()
+
+
 @pytest.mark.parametrize("form", ["bf16x2", "fp16x2", "bf16x3"])
 def test_face_averaged_pack_vs_oracle(gpu, form):
     """rsh_pack_split_avg_dev: 4-face input reduced to a cell-level state in the pack;
