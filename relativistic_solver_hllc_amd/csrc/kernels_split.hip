@@ -217,7 +217,8 @@ __global__ __launch_bounds__(256) void pack_fused_kernel(const double* __restric
     }
 }
 
-// Wide form of the fused pack for M <= 32 kPackWideMaxSteps: a workgroup of
+// Wide form of the fused pack for M <= 32 kPackWideMaxSteps (cell-level input, and
+// 4-face input with shared lines): a workgroup of
 // 16 CPB threads packs CPB / 16 tiles (CPB cells) and keeps the face averages
 // in registers instead of LDS. Thread slot u = t + 16 CPB i stands for
 // (K-step s = u / (4 CPB), row group g = (u / CPB) % 4, cell u % CPB), i.e.
@@ -298,6 +299,105 @@ __global__ __launch_bounds__(16 * CPB) void pack_wide_kernel(const double* __res
         }
 #pragma unroll
         for (int q = 0; q < NT; q++) out[(sk * NT + q) * 64 + lane] = __builtin_bit_cast(v4u, buf[q]);
+    }
+}
+
+// Fused pack of 4-face input for M <= 32 kPackPairMaxSteps: a workgroup of 8
+// waves packs two tiles (32 cells), face averages in registers. Wave w's slot i
+// stands for the 16 directions 16 p + e, p = w + 8 i, i.e. two row groups of 8
+// (half a K-step). Lane pair (2c, 2c + 1) reads cell c of a direction row, 16
+// bytes a lane, so that a load instruction is 1 KB in a row and no line is
+// touched twice (it can be loaded past the caches); the pair then swaps halves:
+// the even lane gets the four faces of the first group's row, the odd lane those
+// of the second's, which are the values each one packs. Same arithmetic, same
+// bits as pack_fused_kernel.
+// What bounds it: HBM (32 M bytes read and 2 NT M written per cell). A form with
+// one lane per cell (two 16-byte loads of stride 32, 64 cells a workgroup, one
+// workgroup per CU: pack_wide_kernel) reads through L1 and leaves most CUs idle
+// below 16,384 cells; a form with the averages in LDS (pack_fused_kernel) fits
+// one or two workgroups a CU. us, before -> now: 1243 x 400 19.9 -> 14.9, 5000 x 100
+// 8.9 -> 6.5, 80,000 x 400 253 -> 228, 1,572,864 x 400 4633 -> 4437 (5.1 TB/s),
+// 1,572,864 x 100 1173 -> 1056, 60,000 x 800 530 -> 302, 300,000 x 800 2655 -> 1606.
+// Loads through the caches: 4841 at 1,572,864 x 400.
+constexpr int kPackPairMaxSteps = 28;  // 7 slots of 8 doubles: 112 registers
+constexpr int kPackPairWaves = 8;
+template <int FMT, int NT, int MAXS>
+__global__ __launch_bounds__(64 * kPackPairWaves, MAXS <= 4 ? 4 : 2) void pack_pair_kernel(
+    const double* __restrict__ illum, int64_t n, int m, int steps, float* __restrict__ inv_scale,
+    v4u* __restrict__ state) {
+    typedef typename Fmt<FMT>::T T;
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    constexpr int W = kPackPairWaves;
+    __shared__ double cmax[2 * W][32];
+    const int lane = threadIdx.x & 63, odd = lane & 1, cc = lane >> 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tiles = (n + 15) / 16;
+    // n not a multiple of 4: rows start inside a 128-byte line, which two workgroups
+    // share. Workgroup b runs on XCD b % 8: neighbouring cells on one XCD then, so
+    // that its L2 serves the second (1015 -> 967 us at 413,519 x 302; with whole
+    // lines the plain order is faster, 4437 against 4528 us at 1,572,864 x 400)
+    const int64_t group = (n & 3) ? (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+    const int64_t cell = group * 32 + cc;
+    const bool cvalid = cell < n;
+    const int64_t cell_c = cvalid ? cell : n - 1;  // invalid cells re-read a valid one, results unused
+    const double* __restrict__ base = illum + cell_c * 4 + 2 * odd;
+    double avg[MAXS][8];
+    double mx = 0.0;
+#pragma unroll
+    for (int i = 0; i < MAXS; i++) {
+        const int j0 = 16 * (wave + W * i);  // rows j0 + e and j0 + 8 + e
+        if (j0 >= m) {  // uniform
+#pragma unroll
+            for (int e = 0; e < 8; e++) avg[i][e] = 0.0;
+            continue;
+        }
+        // rows past M read the last row, results unused: no branch between the loads
+        v2d x[8], y[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int jx = j0 + e < m ? j0 + e : m - 1, jy = j0 + 8 + e < m ? j0 + 8 + e : m - 1;
+            x[e] = __builtin_nontemporal_load(reinterpret_cast<const v2d*>(base + jx * (4 * n)));
+            y[e] = __builtin_nontemporal_load(reinterpret_cast<const v2d*>(base + jy * (4 * n)));
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            mx = fmax(mx, fmax(fmax(fabs(x[e].x), fabs(x[e].y)), fmax(fabs(y[e].x), fabs(y[e].y))));
+            const v2d send = odd ? x[e] : y[e];
+            const v2d recv = {swap_pair_lanes(send.x), swap_pair_lanes(send.y)};
+            const v2d lo = odd ? recv : x[e], hi = odd ? y[e] : recv;
+            const double a = (((lo.x + lo.y) + hi.x) + hi.y) * 0.25;
+            avg[i][e] = cvalid && j0 + 8 * odd + e < m ? a : 0.0;
+        }
+    }
+    // the cell's maximum over the 16 threads that read it
+    cmax[2 * wave + odd][cc] = mx;
+    __syncthreads();
+    double cm = 0.0;
+#pragma unroll
+    for (int w = 0; w < 2 * W; w++) cm = fmax(cm, cmax[w][cc]);
+    const int e = cm > 0.0 ? (kTargetExp - 1 - ilogb(cm)) : 0;
+    const float inv = ldexpf(1.0f, -e);
+    if (threadIdx.x < 64 && !odd && cvalid) inv_scale[cell] = inv;
+    const double scale = cvalid ? 1.0 / (double)inv : 0.0;
+    const int64_t tile = group * 2 + cc / 16;
+    if (tile >= tiles) return;  // no barrier below
+    v4u* out = state + tile * steps * NT * 64;
+#pragma unroll
+    for (int i = 0; i < MAXS; i++) {
+        const int p = wave + W * i, sk = p / 2;
+        if (sk >= steps) break;
+        const int slot = ((p & 1) * 2 + odd) * 16 + cc % 16;
+        T buf[NT][8];
+#pragma unroll
+        for (int e8 = 0; e8 < 8; e8++) {
+            const float v = (float)(avg[i][e8] * scale);
+            T parts[NT];
+            split_parts<FMT, NT>(v, parts);
+#pragma unroll
+            for (int q = 0; q < NT; q++) buf[q][e8] = parts[q];
+        }
+#pragma unroll
+        for (int q = 0; q < NT; q++) out[(sk * NT + q) * 64 + slot] = __builtin_bit_cast(v4u, buf[q]);
     }
 }
 
@@ -468,6 +568,24 @@ hipError_t launch_pack_fused(int form, const double* d_illum, const double* d_ex
     const int steps = (m + 31) / 32;
     v4u* out = static_cast<v4u*>(d_state);
     const int fmt = split_fmt(form), nt = split_terms(form);
+    // Rows of many cells that start inside a line (n not a multiple of 4): 64 cells
+    // a workgroup share fewer lines than 32 (us, wide / pair: 413,519 x 302 892 / 964
+    // two parts, 940 / 971 three, 400 directions 1262 / 1285; 79,999 x 100 63 / 56).
+    const bool wide = n % 4 != 0 && n >= 131072 && steps <= kPackWideMaxSteps;
+    if (faces == 4 && !wide && steps <= kPackPairMaxSteps) {
+        const dim3 pgrid((unsigned)((n + 255) / 256 * 8)), pblock(64 * kPackPairWaves);
+#define RSH_PP(FMT, NT, MAXS)                                                                                       \
+    if (steps <= 4 * MAXS) {                                                                                        \
+        hipLaunchKernelGGL((pack_pair_kernel<FMT, NT, MAXS>), pgrid, pblock, 0, st, d_illum, n, m, steps, d_inv, out); \
+        return hipGetLastError();                                                                                   \
+    }
+#define RSH_PP_SLOTS(FMT, NT) { RSH_PP(FMT, NT, 1) RSH_PP(FMT, NT, 2) RSH_PP(FMT, NT, 4) RSH_PP(FMT, NT, 7) }
+        if (fmt == 0 && nt == 2) RSH_PP_SLOTS(0, 2)
+        if (fmt == 1 && nt == 2) RSH_PP_SLOTS(1, 2)
+        if (nt == 3) RSH_PP_SLOTS(0, 3)
+#undef RSH_PP_SLOTS
+#undef RSH_PP
+    }
     if (steps <= kPackWideMaxSteps) {
         const dim3 wgrid((unsigned)((n + kPackCells - 1) / kPackCells)), wblock(16 * kPackCells);
 #define RSH_PW(FMT, NT, F)                                                                                        \

@@ -216,6 +216,36 @@ def test_face_averaged_pack_vs_oracle(gpu, form):
     assert mx <= TOL[form][0] and mean <= TOL[form][1]
 
 
+@pytest.mark.parametrize("n,m", [(1, 16), (17, 17), (32, 128), (33, 129), (257, 257), (4099, 512), (4100, 513),
+                                 (515, 800), (64, 896), (65, 897), (131072, 20), (131073, 20)])
+def test_face_averaged_pack_exact(gpu, n, m):
+    """Every face-averaged pack form (1, 2, 4 and 7 slots of 128 directions, LDS past 896, 64-cell groups for many
+    cells with rows inside a line) against the packing computed here: averages in FP64 in the same order, one power
+    of two per cell, two FP16 parts with round-to-nearest. Equal bits."""
+    rng = np.random.default_rng(n + m)
+    illum = rng.lognormal(0.0, 3.0, size=(m, n, 4)) * rng.choice([-1.0, 1.0], size=(m, n, 4))
+    d_illum = D.DeviceArray.from_host(illum)
+    sb, cb = rs.split_sizes("fp16x2", 1, n, m)
+    state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+    rs.pack_split_avg_dev("fp16x2", d_illum, n, m, state, scale)
+    D.synchronize()
+    got, inv = state.to_host().view(np.float16), scale.to_host()[:n].astype(np.float64)
+    for a in (d_illum, state, scale):
+        a.free()
+    exponent = np.frexp(np.abs(illum).max(axis=(0, 2)))[1]
+    assert np.unique(np.ldexp(inv, -exponent)).size == 1  # the same power of two above every cell's maximum
+    avg = (((illum[..., 0] + illum[..., 1]) + illum[..., 2]) + illum[..., 3]) * 0.25
+    steps, tiles = -(-m // 32), -(-n // 16)
+    x64 = np.zeros((steps * 32, tiles * 16))
+    x64[:m, :n] = avg / inv
+    x = x64.astype(np.float32)
+    hi = x64.astype(np.float16)  # FP64 to FP16 in one rounding
+    lo = (x - hi.astype(np.float32)).astype(np.float16)
+    # [tile][K-step][part][row group of 8][cell of 16][8]
+    want = np.stack([hi, lo]).reshape(2, steps, 4, 8, tiles, 16).transpose(4, 1, 0, 2, 5, 3)
+    assert np.array_equal(got[:want.size].reshape(want.shape).view(np.uint16), want.astype(np.float16).view(np.uint16))
+
+
 def test_resident_kernel_rejects_face_state(gpu):
     xyz, w, F = rs.fibonacci_directions(26)
     with rs.DirectionSet(xyz, w, F) as ds:
