@@ -369,7 +369,7 @@ def sweep_section(D, rs, edge=32, m=400, steps=5, cpu=True):
         + (f"; cpu {cpu_res['seconds']:.2f} s" if cpu_res else ""))
     return {"workload": f"transport sweep: unit cube in {edge}^3 x 6 = {n} tetrahedra, M={m} Fibonacci directions, "
                         "class_vtk 1 (test task), log-normal scattering, ReCalcIllum residual",
-            "kernel": "sweep_kernel<1> (one workgroup per direction, level-parallel)", "ms": t,
+            "kernel": "sweep_kernel<1> (one workgroup per direction, one thread per out face)", "ms": t,
             "cell_directions_per_s": n * m / (t * 1e-3), "levels_min": int(levels.min()),
             "levels_mean": float(levels.mean()), "levels_max": int(levels.max()),
             "prepare_s": prep_s, "upload_s": upload_s, "records": records,

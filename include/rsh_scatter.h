@@ -312,8 +312,7 @@ int rsh_batch_create(int32_t device, int32_t capacity, int32_t use_graph, rsh_ba
 int rsh_batch_destroy(rsh_batch b);
 /* Kernel of the split-form slots added from now on: 0 = auto (the device's
  * tuned choice for the slot's M, else the resident-panel grouped kernel with
- * 8 waves where its plan fits one XCD and is specialised: M = 200, 400, 800
- * with n_cells < 2^24; else the streaming-panel one), 1 = resident panel,
+ * 8 waves where its plan fits one XCD: M <= 800 with n_cells < 2^24; else the streaming-panel one), 1 = resident panel,
  * 8 waves of 2 cell tiles (rsh_batch_add fails where it does not apply),
  * 2 = streaming panel, 3 = resident panel, 4 waves of 2 cell tiles, two
  * workgroups per CU where the LDS allows (fails as 1). All give bit-identical
@@ -624,8 +623,8 @@ int rsh_sweep_destroy(rsh_sweep s);
 /* Direction k's structures in the reference's formats (sorted_id_cell,
  * face_states, vec_x0's s and in_face_id in traversal order), checked (order a
  * permutation that is upwind, every record naming an in face, record count =
- * 3 x out faces) and uploaded; the cell levels for the parallel sweep are
- * derived here. Replaces the per-direction part of ReadIllumGeometry. */
+ * 3 x out faces) and uploaded; the passes of the parallel sweep are planned
+ * here (calls for different directions may run on several threads). Replaces the per-direction part of ReadIllumGeometry. */
 int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const int32_t* face_state,
                             const double* x0_s, const uint8_t* x0_face, int64_t n_records);
 /* Number of dependency levels of direction k (cells of one level run in parallel). */
