@@ -122,11 +122,20 @@ int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, cons
     return store_panel(ds, key, st, pe, e, out);
 }
 
+static int split_layout(const SplitPlan* resident) {
+    return resident ? 100 + resident->rb_per_pass : 0;  // 0: the streaming plan
+}
+
+// Whether the panel of these rows is there in the layout.
+static bool split_panel_cached(rsh_dirset ds, int k0, int k1, int faces, int form, const SplitPlan* resident) {
+    std::lock_guard<std::mutex> lock(ds->mu);
+    return ds->panels.count(std::make_tuple(k0, k1, faces, form, split_layout(resident))) != 0;
+}
+
 int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
                     const SplitPlan* resident) {
     std::lock_guard<std::mutex> lock(ds->mu);
-    // layout: 0 streaming plan, 100 + row blocks per group for a resident plan
-    const auto key = std::make_tuple(k0, k1, faces, form, resident ? 100 + resident->rb_per_pass : 0);
+    const auto key = std::make_tuple(k0, k1, faces, form, split_layout(resident));
     if (int rc = cached_panel(ds, key, st, out)) return rc;
     if (*out) return RSH_OK;
     bound_panels(ds);
@@ -281,11 +290,25 @@ int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_c
         return fail(RSH_E_UNSUPPORTED, "resident-panel kernel needs cell-level state (faces = 1), ld_out below 2^24 "
                                        "and a panel slice that fits LDS with at most one row group per CU of an XCD");
     // Auto: the resident-panel kernel when its row groups keep at least 3/4 of
-    // the CUs busy (M = 800 needs 17 groups of 3 row blocks: 17 of 32 CUs per
-    // XCD), else the streaming kernel with 8 waves.
+    // the CUs busy, else (M = 769 to 800 needs 17 groups of 3 row blocks: 17 of 32
+    // CUs per XCD) the streaming kernel with 8 waves, but the resident one up to
+    // ten 256-cell chunks per set. us, resident / streaming, 800 directions: 3000 cells
+    // two parts 28 / 49, three 44 / 70; 20,000 cells 106 / 142, 197 / 205;
+    // 100,000 cells 629 / 600, 1054 / 910. A capture takes the form whose panel
+    // is there, the streaming one if both are not.
     const int per_xcd = device_cus(ds->device) / 8;
-    if (waves == 0)
-        waves = (resident_ok && 4 * sets * rplan.passes >= 3 * per_xcd) ? 1 : split_default_waves();
+    if (waves == 0) {
+        bool resident = resident_ok && 4 * sets * rplan.passes >= 3 * per_xcd;
+        if (resident_ok && !resident) {
+            resident = n <= (int64_t)10 * 256 * 8 * sets;
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+                const bool have = split_panel_cached(ds, k0, k1, faces, form, &rplan);
+                resident = have && (resident || !split_panel_cached(ds, k0, k1, faces, form, nullptr));
+            }
+        }
+        waves = resident ? 1 : split_default_waves();
+    }
     PanelRef pe;  // held until the launch is enqueued
     if (waves == 1) {
         int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe, &rplan);

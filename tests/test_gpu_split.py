@@ -155,6 +155,30 @@ def test_resident_panel_kernel_bit_identical(gpu, form, n, m, k0, k1):
         assert mx <= TOL[form][0] and mean <= TOL[form][1], (mx, mean)
 
 
+@pytest.mark.parametrize("n", [20480, 20481])
+def test_automatic_choice_at_800_directions(gpu, n):
+    """17 row groups per XCD: the resident kernel up to 10 chunks of 256 cells for each of its 8 sets, the streaming
+    one beyond. Equal bits on both sides of the line."""
+    m = 800
+    cell = np.resize(np.random.default_rng(n).lognormal(0.0, 1.5, size=1_000_003), (m, n, 1))
+    xyz, w, F = rs.fibonacci_directions(m)
+    with rs.DirectionSet(xyz, w, F) as ds:
+        d_cell = D.DeviceArray.from_host(cell)
+        sb, cb = rs.split_sizes("fp16x2", 1, n, m)
+        state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+        rs.pack_split_dev("fp16x2", d_cell, 1, n, m, state, scale)
+        outs = []
+        for waves in (0, 8):
+            out = D.DeviceArray((m, n))
+            ds.scatter_split("fp16x2", state, scale, 1, n, 0, m, out, waves=waves)
+            D.synchronize()
+            outs.append(out.to_host())
+            out.free()
+        for a in (d_cell, state, scale):
+            a.free()
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("three", [False, True])
 @pytest.mark.parametrize("steps", range(1, 26))
 def test_resident_workgroup_forms_bit_identical(gpu, steps, three):
