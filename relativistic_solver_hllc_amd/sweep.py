@@ -211,6 +211,10 @@ def read_direction_files(main_dir: str, k: int):
 
 # ---------------------------------------------------------------- GPU sweep
 
+def _cpus() -> int:
+    return len(os.sched_getaffinity(0))
+
+
 class Sweep:
     """Device sweep structures for all directions (rsh_sweep_*)."""
 
@@ -229,12 +233,15 @@ class Sweep:
                _p(f) if f.size else None, ss.size)
 
     def set_all(self, per_dir) -> None:
-        # Direction 0 alone (the workgroup size follows from it), then eight at a
-        # time: planning a direction is host work outside the library's lock.
+        """Every direction's structures: a list or tuple, or an iterator, whose item has been taken before it is asked
+        for the next one (it may fill the same arrays again)."""
         it = iter(enumerate(per_dir))
-        for k, d in islice(it, 1):
+        # Planning a direction is host work outside the library's lock: with all of them at hand several at a time,
+        # direction 0 alone (the workgroup size follows from it).
+        some = 1 if isinstance(per_dir, (list, tuple)) and _cpus() > 1 else None
+        for k, d in islice(it, some):
             self.set_direction(k, *d)
-        with ThreadPoolExecutor(max_workers=8) as ex:
+        with ThreadPoolExecutor(max_workers=min(8, _cpus())) as ex:
             while some := list(islice(it, 8)):
                 list(ex.map(lambda kd: self.set_direction(kd[0], *kd[1]), some))
 

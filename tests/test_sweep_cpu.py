@@ -222,3 +222,33 @@ def test_direction_files_roundtrip(tmp_path, mesh4):
             assert np.array_equal(a, b)
     raw = np.fromfile(tmp_path / "LocX05.bin", np.uint8)
     assert raw[:4].view(np.int32)[0] == len(per[5][2]) and raw.size == 4 + 48 * len(per[5][2])
+
+
+class Recorder(sw.Sweep):
+    """A Sweep without a device: set_direction notes what it is given."""
+
+    def __init__(self):
+        self.handle, self.seen = None, {}
+
+    def set_direction(self, k, order, face_state, s, in_face):
+        self.seen[k] = [np.array(a) for a in (order, face_state, s, in_face)]
+
+
+def test_set_all_takes_an_iterators_item_before_the_next():
+    """A generator may hand out the same arrays filled anew: each direction gets its own values, as a list's do."""
+    n = 21
+    items = [[np.full(3, 10 * k + q) for q in range(4)] for k in range(n)]
+
+    def reuse():
+        buf = [np.empty(3) for _ in range(4)]
+        for it in items:
+            for b, a in zip(buf, it):
+                b[:] = a
+            yield tuple(buf)
+
+    for given in (reuse(), iter(items), items, tuple(tuple(i) for i in items)):
+        r = Recorder()
+        r.set_all(given)
+        assert sorted(r.seen) == list(range(n))
+        for k in range(n):
+            assert all(np.array_equal(a, b) for a, b in zip(r.seen[k], items[k]))
