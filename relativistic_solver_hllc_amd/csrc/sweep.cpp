@@ -37,12 +37,19 @@ struct rsh_sweep_s {
     std::vector<Dir> dirs;
     // Host arrays of one direction's plan, kept for the next one (a call takes a
     // set of its own: fresh pages would cost more than half of the planning).
+    struct Cell {
+        int32_t link;   // place in the given order; then, ready: the next cell of its list, taken: its first out face's position
+        int32_t chain;  // cells in the longest chain before it; then in the longest one that still waits on it
+        int32_t out0;   // out faces of the cells before it in the given order (three records each)
+        uint8_t waits;  // cells it reads that are not taken yet
+        uint8_t outs;   // bit f: face f is an out face
+    };
     struct Work {
-        std::vector<int64_t> x0_off;
-        std::vector<int32_t> pos, level, waits, chain, entries, cells, pos_of, pass_of, pass, touched, next, old, open,
-            codes, fix;
-        std::vector<SweepFace> faces;
-        std::vector<double> s3;
+        std::vector<Cell> info;
+        std::vector<int32_t> cells, pass, touched, old, open, fix;
+        std::vector<uint64_t> marks, words;
+        std::unique_ptr<char[]> image;  // what is uploaded
+        size_t room = 0;
     };
     std::vector<std::unique_ptr<Work>> spare;
     SweepDirDev* d_table = nullptr;
@@ -111,6 +118,7 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     if (!s || k < 0 || k >= s->m || !order || !face_state || n_records < 0 || (n_records > 0 && (!x0_s || !x0_face)))
         return fail(RSH_E_ARG, "invalid direction, null pointer or record count");
     const int64_t n = s->n;
+    const int32_t* pairs = s->pairs.data();
     struct Lease {  // a Work of this call, given back at its end
         rsh_sweep s;
         std::unique_ptr<rsh_sweep_s::Work> w;
@@ -128,63 +136,83 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
         }
     } lease(s);
     rsh_sweep_s::Work& w = *lease.w;
-    auto &pos = w.pos, &level = w.level;
-    pos.assign((size_t)n, -1);
-    level.assign((size_t)n, 0);
+    // The loops below go through the cells in an order that is random in memory, over
+    // arrays larger than L2: each fetches what the cells kAhead and 2 kAhead steps on
+    // need (a third of the planning's time).
+    constexpr int kAhead = 12;
+    const auto cell_of = [](int32_t e) { return std::max(e, 0) >> 2; };
+    auto& info = w.info;
+    info.resize((size_t)n);
+    int bad = 0;
+    for (int64_t c = 0; c < n; c++) {
+        bad |= face_state[c] & ~15;
+        info[(size_t)c] = {-1, 0, 0, 0, (uint8_t)(~face_state[c] & 15)};
+    }
     for (int64_t h = 0; h < n; h++) {
         const int32_t c = order[h];
-        if (c < 0 || c >= n || pos[(size_t)c] >= 0) return fail(RSH_E_ARG, "order is not a permutation of the cells");
-        pos[(size_t)c] = (int32_t)h;
+        if (c < 0 || c >= n || info[(size_t)c].link >= 0) return fail(RSH_E_ARG, "order is not a permutation of the cells");
+        info[(size_t)c].link = (int32_t)h;
     }
-    auto& x0_off = w.x0_off;
-    x0_off.resize((size_t)n);
+    if (bad) return fail(RSH_E_ARG, "face state outside 0..15");
+    auto& fix = w.fix;
+    fix.clear();
     int64_t r = 0;
     int32_t levels = 0;
     for (int64_t h = 0; h < n; h++) {
         const int32_t c = order[h];
-        const int st = face_state[c];
-        if (st < 0 || st > 15) return fail(RSH_E_ARG, "face state outside 0..15");
-        x0_off[(size_t)c] = r;
-        int32_t lv = 0;
+        if (h + 2 * kAhead < n) {
+            const int32_t a = order[h + 2 * kAhead], b = order[h + kAhead];
+            __builtin_prefetch(pairs + 4 * (int64_t)a);
+            __builtin_prefetch(&info[(size_t)a], 1);
+            for (int f = 0; f < 4; f++) __builtin_prefetch(&info[(size_t)cell_of(pairs[b * 4 + f])]);
+        }
+        auto& I = info[(size_t)c];
+        I.out0 = (int32_t)(r / 3);
         for (int f = 0; f < 4; f++) {
-            const int32_t p = s->pairs[(size_t)(c * 4 + f)];
-            const bool in = (st >> f) & 1;
+            const int32_t p = pairs[c * 4 + f];
+            const bool in = !((I.outs >> f) & 1);
             if (!in) {
                 for (int j = 0; j < 3; j++, r++) {
                     if (r >= n_records) return fail(RSH_E_ARG, "fewer x0 records than out-face nodes");
                     const int g = x0_face[r];
-                    if (g > 3 || !((st >> g) & 1))
+                    if (g > 3 || ((I.outs >> g) & 1))
                         return fail(RSH_E_ARG, "x0 record " + std::to_string(r) + " does not name an in face");
                 }
             }
             if (p < 0) continue;
             const int32_t u = p / 4;
+            const auto& U = info[(size_t)u];
             // Reads across an in face, and a face both cells treat as out
             // (written by both: the later one in the order wins), order u first.
-            const bool dep = in || (!((face_state[u] >> (p % 4)) & 1) && pos[(size_t)u] < h);
-            if (!dep) continue;
-            if (pos[(size_t)u] > h)
+            const bool both_out = !in && ((U.outs >> (p % 4)) & 1) && U.link < h;
+            if (!in && !both_out) continue;
+            if (both_out) fix.insert(fix.end(), {p, c * 4 + f});  // the later cell in the given order wins
+            if (U.link > h)
                 return fail(RSH_E_ARG, "order is not upwind: cell " + std::to_string(c) + " reads cell " +
                                            std::to_string(u) + " that comes later");
-            lv = std::max(lv, level[(size_t)u] + 1);
+            I.chain = std::max(I.chain, U.chain + 1);
         }
-        level[(size_t)c] = lv;
-        levels = std::max(levels, lv + 1);
+        levels = std::max(levels, I.chain + 1);
     }
     if (r != n_records) return fail(RSH_E_ARG, "more x0 records than out-face nodes");
-    // Cells read by a cell, and the longest chain of cells that still waits on it.
-    auto &waits = w.waits, &chain = w.chain;
-    waits.assign((size_t)n, 0);
-    chain.assign((size_t)n, 0);
-    auto reads = [&](int32_t c, int f) { return ((face_state[c] >> f) & 1) && s->pairs[(size_t)(c * 4 + f)] >= 0; };
+    // What a cell waits for, and the longest chain of cells behind it.
+    for (auto& I : info) I.chain = 0;
     for (int64_t h = n - 1; h >= 0; h--) {
         const int32_t c = order[h];
-        for (int f = 0; f < 4; f++)
-            if (reads(c, f)) {
-                const int32_t u = s->pairs[(size_t)(c * 4 + f)] / 4;
-                waits[(size_t)c]++;
-                chain[(size_t)u] = std::max(chain[(size_t)u], chain[(size_t)c] + 1);
-            }
+        if (h >= 2 * kAhead) {
+            const int32_t a = order[h - 2 * kAhead], b = order[h - kAhead];
+            __builtin_prefetch(pairs + 4 * (int64_t)a);
+            __builtin_prefetch(&info[(size_t)a], 1);
+            for (int f = 0; f < 4; f++) __builtin_prefetch(&info[(size_t)cell_of(pairs[b * 4 + f])], 1);
+        }
+        auto& I = info[(size_t)c];
+        for (int f = 0; f < 4; f++) {
+            const int32_t q = pairs[c * 4 + f];
+            if (((I.outs >> f) & 1) || q < 0) continue;
+            I.waits++;
+            int32_t& chain = info[(size_t)(q / 4)].chain;
+            chain = std::max(chain, I.chain + 1);
+        }
     }
     int block;
     {
@@ -198,30 +226,24 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     // is finished while it is in L2); then the cell with the longest chain behind
     // it (fewest passes). Out faces have positions pass by pass, by cell and face.
     constexpr int32_t kLineCells = 16;
-    auto &entries = w.entries, &cells = w.cells, &pos_of = w.pos_of, &pass_of = w.pass_of, &pass = w.pass;
-    entries.clear();
+    const auto bits = [](unsigned x) { return (int32_t)(0x4332322132212110ull >> (4 * x) & 15); };  // of four: one digit each
+    auto &cells = w.cells, &pass = w.pass;
     cells.clear();
-    pass.clear();
-    entries.reserve((size_t)n_records / 3);
     cells.reserve((size_t)n + 1);
-    pos_of.assign((size_t)n * 4, -1);
-    pass_of.resize((size_t)n);
-    auto& cell_at = w.next;  // a cell taken is in no list any more
-    cell_at.resize((size_t)n);
-    auto out_faces = [&](int32_t c) { return 4 - __builtin_popcount((unsigned)face_state[c]); };
+    pass.clear();
     {
         // ready cells as lists: by the pass that touched their group, by their chain
-        auto &touched = w.touched, &next = w.next, &old = w.old, &open = w.open;
+        auto &touched = w.touched, &old = w.old, &open = w.open;
         touched.assign((size_t)(n / kLineCells + 1), -1);
         old.clear();
         open.assign((size_t)levels, -1);
         int32_t oldest = 0, longest = -1;
         auto push = [&](int32_t c) {
-            const int32_t t = touched[(size_t)(c / kLineCells)], l = chain[(size_t)c];
+            const int32_t t = touched[(size_t)(c / kLineCells)], l = info[(size_t)c].chain;
             int32_t& head = t >= 0 ? old[(size_t)t] : open[(size_t)l];
             if (t >= 0) oldest = std::min(oldest, t);
             else longest = std::max(longest, l);
-            next[(size_t)c] = head;
+            info[(size_t)c].link = head;
             head = c;
         };
         auto top = [&]() -> int32_t* {
@@ -230,113 +252,142 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
             while (longest >= 0 && open[(size_t)longest] < 0) longest--;
             return longest >= 0 ? &open[(size_t)longest] : nullptr;
         };
+        // a pass's cells in ascending order: marked in a bit set with a summary bit per
+        // word (sorting them took a third of the planning)
+        auto &marks = w.marks, &words = w.words;
+        marks.assign((size_t)(n / 64 + 1), 0);
+        words.assign((size_t)(n / 4096 + 1), 0);
+        auto in_order = [&](auto&& f) {
+            for (size_t y = 0; y < words.size(); y++)
+                for (; words[y]; words[y] &= words[y] - 1) {
+                    const size_t x = y * 64 + (size_t)__builtin_ctzll(words[y]);
+                    for (; marks[x]; marks[x] &= marks[x] - 1) f((int32_t)(x * 64 + (size_t)__builtin_ctzll(marks[x])));
+                }
+        };
         for (int32_t c = (int32_t)n - 1; c >= 0; c--)
-            if (!waits[(size_t)c]) push(c);
+            if (!info[(size_t)c].waits) push(c);
+        int32_t positions = 0;  // out faces so far
         for (int32_t p = 0; top(); p++) {
-            const size_t first = cells.size();
-            const int32_t face0 = (int32_t)entries.size();
-            int32_t cnt = 0;
+            const int32_t first = (int32_t)cells.size(), face0 = positions;
+            int32_t cnt = 0, taken = 0;
             old.push_back(-1);
-            for (int32_t* head; (int32_t)(cells.size() - first) < block / 2 && (head = top());) {
+            for (int32_t* head; taken < block / 2 && (head = top()); taken++) {
                 const int32_t c = *head;
-                if ((cnt += out_faces(c)) > block) break;
-                *head = next[(size_t)c];
+                const auto& I = info[(size_t)c];
+                if ((cnt += bits(I.outs)) > block) break;
+                *head = I.link;
                 int32_t& t = touched[(size_t)(c / kLineCells)];
                 if (t < 0) t = p;
+                marks[(size_t)c >> 6] |= uint64_t(1) << (c & 63);
+                words[(size_t)c >> 12] |= uint64_t(1) << ((c >> 6) & 63);
+            }
+            in_order([&](int32_t c) {
+                auto& I = info[(size_t)c];
                 cells.push_back(c);
-            }
-            std::sort(cells.begin() + (int64_t)first, cells.end());
-            for (size_t i = first; i < cells.size(); i++) {
-                const int32_t c = cells[i];
-                pass_of[(size_t)c] = p;
-                cell_at[(size_t)c] = (int32_t)i;
-                for (int f = 0; f < 4; f++)
-                    if (!((face_state[c] >> f) & 1)) {
-                        const int32_t q = s->pairs[(size_t)(c * 4 + f)];
-                        pos_of[(size_t)(c * 4 + f)] = (int32_t)entries.size();
-                        entries.push_back(c * 4 + f);
-                        if (q >= 0 && reads(q / 4, q % 4) && --waits[(size_t)(q / 4)] == 0) push(q / 4);
-                    }
-            }
-            pass.insert(pass.end(), {face0, (int32_t)entries.size() - face0, (int32_t)first, (int32_t)(cells.size() - first)});
+                I.link = positions;
+                positions += bits(I.outs);
+                for (unsigned left = I.outs; left; left &= left - 1) {
+                    const int32_t q = pairs[c * 4 + __builtin_ctz(left)];
+                    if (q < 0) continue;
+                    auto& Q = info[(size_t)(q >> 2)];
+                    if (!((Q.outs >> (q & 3)) & 1) && --Q.waits == 0) push(q >> 2);
+                }
+            });
+            pass.insert(pass.end(), {face0, positions - face0, first, taken});
         }
+        // one more, empty: the last pass's cells are stored in the step after it
+        pass.insert(pass.end(), {positions, 0, (int32_t)n, 0});
     }
-    // one more, empty: the last pass's cells are stored in the step after it
-    pass.insert(pass.end(), {(int32_t)entries.size(), 0, (int32_t)n, 0});
     const int32_t passes = (int32_t)(pass.size() / 4);
-    // Code of an entry's value at step `step`: its own position's for an out face,
-    // the neighbour's for an in face.
-    const int64_t ring = (int64_t)block * kSweepRing;
-    auto code_of = [&](int32_t e, int32_t step) -> int32_t {
-        const int32_t up = s->pairs[(size_t)e];
-        int32_t src = e;
-        if ((face_state[e / 4] >> (e % 4)) & 1) {
-            if (up < 0) return up == RSH_BOUND_OUT_SOURCE ? kSweepOne : kSweepZero;
-            src = up;
-        }
-        const int64_t end = (int64_t)pass[(size_t)step * 4] + pass[(size_t)step * 4 + 1];
-        return pos_of[(size_t)src] >= end - ring ? (int32_t)(pos_of[(size_t)src] & (ring - 1)) : kSweepFar - src;
-    };
-    // one record more than used: threads without work load the one after the last
-    auto& faces = w.faces;
-    auto& s3 = w.s3;
-    auto &codes = w.codes, &fix = w.fix;
-    faces.resize(entries.size() + 1);
-    faces.back() = SweepFace{0, {kSweepZero, kSweepZero, kSweepZero}};
-    s3.resize((entries.size() + 1) * 3);
-    for (int j = 1; j <= 3; j++) s3[s3.size() - (size_t)j] = 0.0;
-    codes.resize((size_t)(n + 1) * 4);
-    for (int j = 1; j <= 4; j++) codes[codes.size() - (size_t)j] = kSweepZero;
-    fix.clear();
-    for (int64_t h = 0; h < n; h++) {
-        const int32_t c = order[h], i = cell_at[(size_t)c], p = pass_of[(size_t)c];
-        const int64_t first = pass[(size_t)p * 4], cnt = pass[(size_t)p * 4 + 1];
-        int64_t r = x0_off[(size_t)c];  // records of the cell in out-face order
-        for (int f = 0; f < 4; f++) {
-            const int32_t e = c * 4 + f;
-            codes[(size_t)i * 4 + (size_t)f] = code_of(e, p + 1);
-            const int32_t at = pos_of[(size_t)e];
-            if (at < 0) continue;
-            SweepFace& F = faces[(size_t)at];
-            F.cell = (uint32_t)c;
-            if (!s->node_in_source.empty())
-                F.cell |= (uint32_t)((s->node_in_source[(size_t)c] >> (3 * f)) & 7u) << kSweepCellBits;
-            for (int j = 0; j < 3; j++, r++) {
-                F.up[j] = code_of(c * 4 + x0_face[r], p);
-                s3[(size_t)(first * 3 + j * cnt + at - first)] = x0_s[r];
+    // What the device gets, as one image: faces and codes with one record more than
+    // used (threads without work load the one after the last).
+    const size_t positions = (size_t)n_records / 3;
+    const size_t b_faces = align256((positions + 1) * sizeof(SweepFace)), b_s3 = align256((positions + 1) * 24),
+                 b_codes = align256((size_t)(n + 1) * 16), b_cells = align256((size_t)(n + 1) * 4),
+                 b_pass = align256(pass.size() * 4), b_fix = align256(fix.size() * 4);
+    const size_t bytes = b_faces + b_s3 + b_codes + b_cells + b_pass + b_fix;
+    if (w.room < bytes) {
+        w.image.reset();
+        w.room = 0;
+        w.image.reset(new char[bytes]);
+        w.room = bytes;
+    }
+    SweepFace* const faces = reinterpret_cast<SweepFace*>(w.image.get());
+    double* const s3 = reinterpret_cast<double*>(w.image.get() + b_faces);
+    int32_t* const codes = reinterpret_cast<int32_t*>(w.image.get() + b_faces + b_s3);
+    int32_t* const cells_out = reinterpret_cast<int32_t*>(w.image.get() + b_faces + b_s3 + b_codes);
+    char* const tables = w.image.get() + b_faces + b_s3 + b_codes + b_cells;
+    faces[positions] = SweepFace{0, {kSweepZero, kSweepZero, kSweepZero}};
+    for (size_t j = 0; j < 3; j++) s3[3 * positions + j] = 0.0;
+    for (size_t j = 0; j < 4; j++) codes[4 * (size_t)n + j] = kSweepZero;
+    cells.push_back(0);
+    std::memcpy(cells_out, cells.data(), cells.size() * 4);
+    std::memcpy(tables, pass.data(), pass.size() * 4);
+    if (!fix.empty()) std::memcpy(tables + b_pass, fix.data(), fix.size() * 4);
+    // Code of a face value in a step: the position that it was written to (its own for
+    // an out face, the neighbour's for an in face) while the ring holds it.
+    const int32_t ring = block * kSweepRing;
+    for (int32_t p = 0; p + 1 < passes; p++) {
+        const int32_t* P = &pass[(size_t)p * 4];
+        const int32_t first = P[0], cnt = P[1];
+        // oldest positions in the ring in step p (node values) and in the step after it (cell values)
+        const int32_t node_lo = first + cnt - ring, cell_lo = P[4] + P[5] - ring;
+        double* s3_pass = s3 + 3 * (int64_t)first;
+        for (int32_t i = P[2]; i < P[2] + P[3]; i++) {
+            if (i + 2 * kAhead < n) {
+                const int32_t ca = cells[(size_t)i + 2 * kAhead], cb = cells[(size_t)i + kAhead];
+                const int64_t rb = 3 * (int64_t)info[(size_t)cb].out0;
+                __builtin_prefetch(pairs + 4 * (int64_t)ca);
+                __builtin_prefetch(&info[(size_t)ca]);
+                __builtin_prefetch(x0_s + rb);
+                __builtin_prefetch(x0_s + rb + 8);
+                __builtin_prefetch(x0_face + rb);
+                for (int f = 0; f < 4; f++) __builtin_prefetch(&info[(size_t)cell_of(pairs[cb * 4 + f])]);
             }
-            // a face out on both sides: the later cell in the given order wins
-            const int32_t q = s->pairs[(size_t)e];
-            if (q >= 0 && pos_of[(size_t)q] >= 0 && pos[(size_t)(q / 4)] < pos[(size_t)c]) fix.insert(fix.end(), {q, e});
+            const int32_t c = cells[(size_t)i];
+            const rsh_sweep_s::Cell I = info[(size_t)c];
+            int32_t node_code[4], *cell_code = codes + (int64_t)i * 4;
+            for (int f = 0; f < 4; f++) {
+                const int32_t q = pairs[c * 4 + f];
+                const int32_t src = (I.outs >> f) & 1 ? c * 4 + f : q;  // < 0: a boundary's value
+                const rsh_sweep_s::Cell& S = info[(size_t)cell_of(src)];
+                const int32_t at = S.link + bits(S.outs & ((1u << (src & 3)) - 1u)), slot = at & (ring - 1),
+                              far = kSweepFar - src;
+                cell_code[f] = at >= cell_lo ? slot : far;
+                node_code[f] = at >= node_lo ? slot : far;
+                if (src < 0) cell_code[f] = node_code[f] = q == RSH_BOUND_OUT_SOURCE ? kSweepOne : kSweepZero;
+            }
+            SweepFace* F = faces + I.link;
+            double* to = s3_pass + (I.link - first);
+            const double* xs = x0_s + 3 * (int64_t)I.out0;  // records of the cell in out-face order
+            const uint8_t* xf = x0_face + 3 * (int64_t)I.out0;
+            const uint32_t in_source = s->node_in_source.empty() ? 0u : s->node_in_source[(size_t)c];
+            for (unsigned left = I.outs; left; left &= left - 1, F++, to++) {
+                F->cell = (uint32_t)c | ((in_source >> (3 * __builtin_ctz(left))) & 7u) << kSweepCellBits;
+                for (int j = 0; j < 3; j++) {
+                    F->up[j] = node_code[*xf++];
+                    to[(int64_t)j * cnt] = *xs++;
+                }
+            }
         }
     }
-    cells.push_back(0);
 
-    const size_t b_faces = align256(faces.size() * sizeof(SweepFace)), b_s3 = align256(s3.size() * 8),
-                 b_pass = align256(pass.size() * 4), b_codes = align256(codes.size() * 4),
-                 b_cells = align256(cells.size() * 4), b_fix = align256(fix.size() * 4);
     std::lock_guard<std::mutex> lock(s->mu);
     RSH_HIP_TRY(hipSetDevice(s->device));
     auto& d = s->dirs[(size_t)k];
     if (d.block) RSH_HIP_TRY(hipFree(d.block));
     d.block = nullptr;
     d.set = false;
-    if (hipMalloc(&d.block, b_faces + b_s3 + b_pass + b_codes + b_cells + b_fix) != hipSuccess)
-        return fail(RSH_E_NOMEM, "sweep: direction allocation failed");
-    char* at = static_cast<char*>(d.block);
-    auto put = [&](const void* src, size_t bytes, size_t room) {
-        char* dst = at;
-        at += room;
-        return !bytes || hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess ? dst : nullptr;
-    };
-    d.dev.faces = reinterpret_cast<const SweepFace*>(put(faces.data(), faces.size() * sizeof(SweepFace), b_faces));
-    d.dev.s3 = reinterpret_cast<const double*>(put(s3.data(), s3.size() * 8, b_s3));
-    d.dev.pass = reinterpret_cast<const int32_t*>(put(pass.data(), pass.size() * 4, b_pass));
-    d.dev.codes = reinterpret_cast<const int32_t*>(put(codes.data(), codes.size() * 4, b_codes));
-    d.dev.cells = reinterpret_cast<const int32_t*>(put(cells.data(), cells.size() * 4, b_cells));
-    d.dev.fix = reinterpret_cast<const int32_t*>(put(fix.data(), fix.size() * 4, b_fix));
-    if (!d.dev.faces || !d.dev.s3 || !d.dev.pass || !d.dev.codes || !d.dev.cells || !d.dev.fix)
+    if (hipMalloc(&d.block, bytes) != hipSuccess) return fail(RSH_E_NOMEM, "sweep: direction allocation failed");
+    if (hipMemcpy(d.block, w.image.get(), bytes, hipMemcpyHostToDevice) != hipSuccess)
         return fail(RSH_E_HIP, "sweep: upload of a direction failed");
+    char* const at = static_cast<char*>(d.block);
+    d.dev.faces = reinterpret_cast<const SweepFace*>(at);
+    d.dev.s3 = reinterpret_cast<const double*>(at + b_faces);
+    d.dev.codes = reinterpret_cast<const int32_t*>(at + b_faces + b_s3);
+    d.dev.cells = reinterpret_cast<const int32_t*>(at + b_faces + b_s3 + b_codes);
+    d.dev.pass = reinterpret_cast<const int32_t*>(at + b_faces + b_s3 + b_codes + b_cells);
+    d.dev.fix = reinterpret_cast<const int32_t*>(at + b_faces + b_s3 + b_codes + b_cells + b_pass);
     d.dev.passes = passes;
     d.dev.levels = levels;
     d.dev.fixes = (int32_t)(fix.size() / 2);
