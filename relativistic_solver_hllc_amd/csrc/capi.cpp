@@ -85,11 +85,25 @@ static int store_panel(rsh_dirset ds, const std::tuple<int, int, int, int, int>&
     return RSH_OK;
 }
 
-// Bounded cache: evict the entries nobody else holds (batch slots and calls
-// still enqueuing keep theirs); each is freed after the device is idle, by its
-// destructor.
-static void bound_panels(rsh_dirset ds) {
-    if (ds->panels.size() < kPanelCacheCap) return;
+// Bounded cache, by ranges (k0, k1, faces, form), whatever layouts each is there
+// in: before a range beyond the cap is added, the entries nobody else holds (batch
+// slots and calls still enqueuing keep theirs) are evicted; each is freed after the
+// device is idle, by its destructor. A size of another layout evicts nothing: a
+// captured graph goes on reading the panel that it was captured with.
+static void bound_panels(rsh_dirset ds, const std::tuple<int, int, int, int, int>& key) {
+    typedef std::tuple<int, int, int, int> Range;
+    const auto range_of = [](const std::tuple<int, int, int, int, int>& k) {
+        return Range{std::get<0>(k), std::get<1>(k), std::get<2>(k), std::get<3>(k)};
+    };
+    size_t ranges = 0;
+    Range last{-1, -1, -1, -1};
+    for (const auto& e : ds->panels) {  // ordered by range
+        const Range r = range_of(e.first);
+        if (r == range_of(key)) return;
+        ranges += r != last;
+        last = r;
+    }
+    if (ranges < kPanelCacheCap) return;
     for (auto e = ds->panels.begin(); e != ds->panels.end();) {
         if (e->second.use_count() == 1)
             e = ds->panels.erase(e);
@@ -111,7 +125,7 @@ int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, cons
             std::get<2>(it->first) == faces && std::get<3>(it->first) == RSH_FORM_FP64)
             return cached_panel(ds, it->first, st, out);
     }
-    bound_panels(ds);
+    bound_panels(ds, key);
     auto pe = std::make_shared<PanelEntry>();
     pe->device = ds->device;
     pe->plan = plan;
@@ -138,7 +152,7 @@ int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStrea
     const auto key = std::make_tuple(k0, k1, faces, form, split_layout(resident));
     if (int rc = cached_panel(ds, key, st, out)) return rc;
     if (*out) return RSH_OK;
-    bound_panels(ds);
+    bound_panels(ds, key);
     auto pe = std::make_shared<PanelEntry>();
     pe->device = ds->device;
     pe->splan = resident ? *resident : plan_split(ds->m, k1 - k0);

@@ -59,8 +59,8 @@ int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, cons
 // Split phase panel; resident != nullptr: in that row-group plan.
 int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
                     const SplitPlan* resident = nullptr);
-// Cache capacity of a direction set's panel cache (entries not held elsewhere
-// are evicted beyond it).
+// Ranges (rows, faces, form) that a direction set's panel cache keeps (entries not
+// held elsewhere are evicted beyond it).
 constexpr size_t kPanelCacheCap = 64;
 // Compute units of a device (cached).
 int device_cus(int device);

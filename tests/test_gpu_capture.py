@@ -1,0 +1,74 @@
+"""Evaluations under stream capture. Nothing can be allocated there, so a captured call needs a phase panel that an
+earlier call has built; a graph is replayed several times, with other work between, and each replay checked."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from relativistic_solver_hllc_amd import _native as N
+from relativistic_solver_hllc_amd import device as D
+from relativistic_solver_hllc_amd import scatter as rs
+
+pytestmark = pytest.mark.gpu
+
+
+def hip(name, *args):
+    """A call of the HIP runtime that the library has loaded."""
+    f = getattr(N.lib, name)
+    f.restype = C.c_int
+    rc = f(*args)
+    assert rc == 0, f"{name}: {rc}"
+
+
+class Graph:
+    """What `record` enqueues on a stream, captured and instantiated."""
+
+    def __init__(self, record):
+        self.stream, self.graph, self.exec = D.Stream(), C.c_void_p(), C.c_void_p()
+        st = C.c_void_p(self.stream.cuda_stream)
+        hip("hipStreamBeginCapture", st, C.c_int(1))  # thread-local
+        try:
+            record(self.stream)
+        finally:
+            rc = N.lib.hipStreamEndCapture(st, C.byref(self.graph))
+        assert rc == 0
+        hip("hipGraphInstantiate", C.byref(self.exec), self.graph, None, None, C.c_size_t(0))
+
+    def replay(self):
+        hip("hipGraphLaunch", self.exec, C.c_void_p(self.stream.cuda_stream))
+        D.synchronize()
+
+    def close(self):
+        hip("hipGraphExecDestroy", self.exec)
+        hip("hipGraphDestroy", self.graph)
+
+
+def dirset(m):
+    xyz, w, F = rs.fibonacci_directions(m)
+    return rs.DirectionSet(xyz, w, F, phase="hg", g=0.6, normalize=True)
+
+
+def test_panels_of_40_ranges_in_two_layouts_stay(gpu):
+    """The panel cache holds 64 ranges. Sizes that take another layout of a range's panel do not count as ranges: after
+    40 of them in two layouts each, the first one is still there for a capture, and the graph's results are those of
+    an eager call after further calls."""
+    m, few, many = 64, 17, 300000
+    with dirset(m) as ds:
+        d_in, out, ref = (D.DeviceArray((m, many)), D.DeviceArray((m, many)), D.DeviceArray((m, many)))
+        N.call("rsh_fill_lognormal_dev", d_in.ptr, m * many, 0.0, 1.0, 7, None)
+        ds.scatter_f64(d_in, 1, few, 0, m, ref)
+        for k in range(40):
+            for n in (few, many):
+                ds.scatter_f64(d_in, 1, n, k, k + 1, out)
+        D.synchronize()
+        g = Graph(lambda st: ds.scatter_f64(d_in, 1, few, 0, m, out, stream=st))
+        want = ref.to_host().reshape(-1)[:m * few]
+        for _ in range(3):
+            out.fill(-1.0)
+            ds.scatter_f64(d_in, 1, many, 3, 4, ref)
+            D.synchronize()
+            g.replay()
+            assert np.array_equal(out.to_host().reshape(-1)[:m * few], want)
+        g.close()
+        for a in (d_in, out, ref):
+            a.free()
