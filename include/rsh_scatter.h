@@ -144,6 +144,23 @@ int rsh_scatter_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
                         int32_t k0, int32_t k1, double* d_out, int64_t ld_out, void* stream,
                         int32_t kernel, const rsh_tile* tile);
 
+/* The kernel that an automatic call of these sizes on `stream` runs as things are
+ * (the sizes, what rsh_autotune_f64 recorded; for a stream under capture, which
+ * can build no phase panel, also the panels that are there). All kernels give the
+ * same bits. No reference counterpart. */
+typedef enum {
+    RSH_KERNEL_PANEL = 0,    /* FP64: phase panel staged through LDS             */
+    RSH_KERNEL_REGISTER = 1  /* FP64: one wave per 16 cells and row group, no LDS */
+} rsh_route_kernel;
+typedef struct {
+    int32_t kernel;      /* rsh_route_kernel                                     */
+    int32_t row_blocks;  /* 16-row blocks per pass or row group                  */
+    int32_t passes;      /* passes or row groups                                 */
+    int32_t waves;       /* waves per workgroup (0: RSH_KERNEL_REGISTER)         */
+} rsh_route;
+int rsh_scatter_f64_route(rsh_dirset ds, int32_t faces, int64_t n_cells, int32_t k0, int32_t k1, void* stream,
+                          rsh_route* route);
+
 /* Radiation moments over all M directions of ds, per cell, on caller-owned
  * device memory:
  *   energy[c]       = sum_j w_j Ibar_j / F

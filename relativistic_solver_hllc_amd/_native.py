@@ -60,6 +60,10 @@ class RequestDesc(C.Structure):
     ]
 
 
+class Route(C.Structure):
+    _fields_ = [("kernel", i32), ("row_blocks", i32), ("passes", i32), ("waves", i32)]
+
+
 class RequestInfo(C.Structure):
     _fields_ = [
         ("status", i32),
@@ -86,6 +90,7 @@ PROTOTYPES = {
     "rsh_dirset_destroy": (C.c_int, [vp]),
     "rsh_dirset_phase_matrix": (C.c_int, [vp, i32, i32, vp]),
     "rsh_scatter_f64_dev": (C.c_int, [vp, vp, i32, i64, i32, i32, vp, i64, vp, i32, C.POINTER(Tile)]),
+    "rsh_scatter_f64_route": (C.c_int, [vp, i32, i64, i32, i32, vp, C.POINTER(Route)]),
     "rsh_split_sizes": (C.c_int, [i32, i32, i64, i32, C.POINTER(i64), C.POINTER(i64)]),
     "rsh_pack_split_dev": (C.c_int, [i32, vp, i32, i64, i32, vp, vp, vp]),
     "rsh_scatter_split_dev": (C.c_int, [vp, i32, vp, vp, i32, i64, i32, i32, vp, i64, i32, vp, i32]),

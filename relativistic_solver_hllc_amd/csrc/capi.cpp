@@ -112,19 +112,60 @@ static void bound_panels(rsh_dirset ds, const std::tuple<int, int, int, int, int
     }
 }
 
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+}
+
+static std::tuple<int, int, int, int, int> f64_key(int k0, int k1, int faces, const F64Plan& plan) {
+    return {k0, k1, faces, (int)RSH_FORM_FP64, plan.rb_per_pass + (plan.paired ? 100 : 0)};
+}
+
+// The plan to run when `want` is asked for on st, its panel if that is there (found,
+// may be null) and whether the least-pass plan's panel is there. While st is being
+// captured nothing can be allocated, so that a panel which is not there is replaced by
+// the least-pass plan's (there after any automatic call outside a capture), else by
+// any of the range. Every plan gives the same bits.
+static int runnable_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& want,
+                        const F64Plan& least, F64Plan* run, bool* have_least, PanelRef* found) {
+    *run = want;
+    std::unique_lock<std::mutex> lock(ds->mu);
+    const bool is_least = !want.paired && want.passes == least.passes;
+    const auto key = f64_key(k0, k1, faces, want);
+    const bool have = ds->panels.count(key) != 0;
+    *have_least = is_least ? have : ds->panels.count(f64_key(k0, k1, faces, least)) != 0;
+    if (have) return found ? cached_panel(ds, key, st, found) : RSH_OK;
+    lock.unlock();
+    if (!capturing(st)) return RSH_OK;
+    lock.lock();
+    auto it = ds->panels.lower_bound({k0, k1, faces, (int)RSH_FORM_FP64, 0});
+    const auto past = std::make_tuple(k0, k1, faces, (int)RSH_FORM_FP64 + 1, 0);
+    if (*have_least) *run = least;
+    else if (it != ds->panels.end() && it->first < past) *run = it->second->plan;
+    return RSH_OK;
+}
+
+static int choose_f64(rsh_dirset ds, int faces, int64_t n, int k0, int k1, hipStream_t st, F64Route* run,
+                      bool* have_least, PanelRef* found) {
+    const F64Route rt = route_f64(ds->m, k1 - k0, faces, n, device_cus(ds->device));
+    *run = rt;
+    if (int rc = runnable_f64(ds, k0, k1, faces, st, rt.plan, plan_f64(ds->m, k1 - k0), &run->plan, have_least, found))
+        return rc;
+    if (run->plan.paired) {
+        run->waves = run->chunk_steps = 0;
+        return RSH_OK;
+    }
+    rsh_tile t{8, 2};
+    const bool tuned = f64_tile_tuned(ds->device, run->plan.rb_per_pass, &t);
+    if (tuned || rt.plan.paired || run->plan.passes != rt.plan.passes) *run = F64Route{run->plan, t.waves, t.chunk_steps};
+    return RSH_OK;
+}
+
 int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out) {
     std::lock_guard<std::mutex> lock(ds->mu);
-    const int layout = plan.rb_per_pass + (plan.paired ? 100 : 0);
-    const auto key = std::make_tuple(k0, k1, faces, (int)RSH_FORM_FP64, layout);
+    const auto key = f64_key(k0, k1, faces, plan);
     if (int rc = cached_panel(ds, key, st, out)) return rc;
     if (*out) return RSH_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
-        auto it = ds->panels.lower_bound(std::make_tuple(k0, k1, faces, (int)RSH_FORM_FP64, 0));
-        if (it != ds->panels.end() && std::get<0>(it->first) == k0 && std::get<1>(it->first) == k1 &&
-            std::get<2>(it->first) == faces && std::get<3>(it->first) == RSH_FORM_FP64)
-            return cached_panel(ds, it->first, st, out);
-    }
     bound_panels(ds, key);
     auto pe = std::make_shared<PanelEntry>();
     pe->device = ds->device;
@@ -232,31 +273,33 @@ int scatter_f64(rsh_dirset ds, const double* d_illum, int faces, int64_t n, int6
     if (kernel != RSH_F64_AUTO && kernel != RSH_F64_MFMA) return fail(RSH_E_ARG, "unknown FP64 kernel id");
     // A given tile runs the LDS-panel kernel with it; otherwise the route for
     // this size, with the tile that rsh_autotune_f64 recorded for the class.
+    const F64Plan least = plan_f64(ds->m, k1 - k0);
     F64Route rt;
+    PanelRef pe;  // held until the launch is enqueued
+    bool have_least;
+    int rc;
     if (tile && kernel == RSH_F64_MFMA) {
-        rt.plan = plan_f64(ds->m, k1 - k0);
-        rt.waves = tile->waves;
-        rt.chunk_steps = tile->chunk_steps;
+        rt = F64Route{least, tile->waves, tile->chunk_steps};
         if (!mfma_f64_tile_supported(rt.waves, rt.chunk_steps))
             return fail(RSH_E_UNSUPPORTED, "unsupported MFMA tile (waves, chunk_steps)");
+        rc = runnable_f64(ds, k0, k1, faces, st, least, least, &rt.plan, &have_least, &pe);
     } else {
-        rt = route_f64(ds->m, k1 - k0, faces, n, device_cus(ds->device));
+        rc = choose_f64(ds, faces, n, k0, k1, st, &rt, &have_least, &pe);
+        // The least-pass panel beside the route's: with it a call of any size can be captured.
+        if (!rc && !have_least && !capturing(st)) {
+            PanelRef built;
+            rc = get_panel_f64(ds, k0, k1, faces, st, least, &built);
+        }
     }
-    PanelRef pe;  // held until the launch is enqueued
-    int rc = get_panel_f64(ds, k0, k1, faces, st, rt.plan, &pe);
+    if (!rc && !pe) rc = get_panel_f64(ds, k0, k1, faces, st, rt.plan, &pe);
     if (rc) return rc;
     const double* panel = static_cast<const double*>(pe->d_panel);
     if (pe->plan.paired) {
         RSH_HIP_TRY(launch_mfma_f64_reg(d_illum, faces, n, ldx, ds->m, panel, pe->plan, k1 - k0, d_out, ld, st));
         return RSH_OK;
     }
-    rsh_tile t{rt.waves, rt.chunk_steps};
-    if (!tile || kernel != RSH_F64_MFMA) {
-        if (t.waves == 0) t = rsh_tile{8, 2};  // a captured stream's cached panel in place of the register-fed one
-        (void)f64_tile_tuned(ds->device, pe->plan.rb_per_pass, &t);
-    }
-    RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n, ldx, ds->m, panel, pe->plan, k1 - k0, d_out, ld, t.waves,
-                                t.chunk_steps, st));
+    RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n, ldx, ds->m, panel, pe->plan, k1 - k0, d_out, ld, rt.waves,
+                                rt.chunk_steps, st));
     return RSH_OK;
 }
 
@@ -341,6 +384,18 @@ int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_c
 }  // namespace
 
 extern "C" {
+
+int rsh_scatter_f64_route(rsh_dirset ds, int32_t faces, int64_t n_cells, int32_t k0, int32_t k1, void* stream,
+                          rsh_route* route) {
+    if (!ds || !route) return fail(RSH_E_ARG, "null direction set or route");
+    if (faces != 1 && faces != 4) return fail(RSH_E_UNSUPPORTED, "faces must be 1 or 4");
+    if (n_cells <= 0 || k0 < 0 || k1 > ds->m || k0 >= k1) return fail(RSH_E_ARG, "invalid cell count or direction range");
+    F64Route rt;
+    bool have_least;
+    if (int rc = choose_f64(ds, faces, n_cells, k0, k1, (hipStream_t)stream, &rt, &have_least, nullptr)) return rc;
+    *route = rsh_route{rt.plan.paired ? RSH_KERNEL_REGISTER : RSH_KERNEL_PANEL, rt.plan.rb_per_pass, rt.plan.passes, rt.waves};
+    return RSH_OK;
+}
 
 int rsh_abi_version(void) { return RSH_ABI_VERSION; }
 

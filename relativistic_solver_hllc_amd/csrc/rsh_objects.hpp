@@ -52,9 +52,7 @@ namespace rsh {
 // FP64 phase panel of (k0, k1, faces) in the layout of `plan`, built on stream
 // st if absent. The caller holds *out for as long as it enqueues work that reads
 // the panel (a batch slot: until the slot is removed); the cache never frees an
-// entry someone else holds. While st is being captured nothing can be allocated:
-// then a panel of another layout of the same range, if there is one, is returned
-// instead of failing (*out carries its plan; every layout gives the same bits).
+// entry someone else holds.
 int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out);
 // Split phase panel; resident != nullptr: in that row-group plan.
 int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,

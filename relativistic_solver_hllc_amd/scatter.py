@@ -29,6 +29,7 @@ from . import _native as N
 PHASES = {"thomson": 0, "hg": 1}
 FORMS = {"fp64": 0, "bf16x2": 1, "fp16x2": 2, "bf16x3": 3}
 F64_KERNELS = {"auto": 0, "direct": 1, "mfma": 2}
+ROUTE_KERNELS = {0: "panel", 1: "register"}
 STREAM_SCATTERING_1, STREAM_SCATTERING_2, STREAM_PARAMS = 0, 1, 2
 
 
@@ -196,6 +197,12 @@ class DirectionSet:
         t = C.byref(N.Tile(*tile)) if tile is not None else None
         N.call("rsh_scatter_f64_dev", self.handle, _ptr(illum), faces, n_cells, k0, k1, _ptr(out),
                n_cells if ld is None else ld, _stream(stream), F64_KERNELS[kernel], t)
+
+    def scatter_f64_route(self, faces: int, n_cells: int, k0: int, k1: int, stream=None) -> Tuple[str, int, int, int]:
+        """What an automatic scatter_f64 of these sizes runs: (kernel, row blocks, passes, waves)."""
+        r = N.Route()
+        N.call("rsh_scatter_f64_route", self.handle, faces, n_cells, k0, k1, _stream(stream), C.byref(r))
+        return ROUTE_KERNELS[r.kernel], r.row_blocks, r.passes, r.waves
 
     def scatter_f64_noalloc(self, illum, faces: int, n_cells: int, k0: int, k1: int, out,
                             ld: Optional[int] = None, stream=None) -> None:

@@ -72,3 +72,43 @@ def test_panels_of_40_ranges_in_two_layouts_stay(gpu):
         g.close()
         for a in (d_in, out, ref):
             a.free()
+
+
+@pytest.mark.parametrize("faces", [1, 4])
+def test_captured_f64_kernel_does_not_depend_on_the_warm_up_size(gpu, faces):
+    """After a call of any one size, a captured call runs its own route if that panel is there and else the plan of
+    fewest passes with eight waves (what every size ran before the routes by size); never another size's plan. The
+    graph's results are the eager call's."""
+    m, sizes = 400, (381, 2957, 24577, 200000)
+    d_in, out, ref = (D.DeviceArray((m, sizes[-1], faces)), D.DeviceArray((m, sizes[-1])), D.DeviceArray((m, sizes[-1])))
+    N.call("rsh_fill_lognormal_dev", d_in.ptr, d_in.size, 0.0, 1.0, 7, None)
+    with dirset(m) as ds:
+        eager = {n: ds.scatter_f64_route(faces, n, 0, m) for n in sizes}
+    assert eager[381][0] == "register" and eager[200000][:3] == ("panel", 25, 1)
+    assert len({r[:3] for r in eager.values()}) >= 3
+    fewest = ("panel", 25, 1, rs.tuned_tile_f64(m)[0])  # eight waves unless another test has tuned the class
+    for warm in sizes:
+        for n in sizes:
+            with dirset(m) as ds:
+                ds.scatter_f64(d_in, faces, warm, 0, m, out)
+                D.synchronize()
+                seen = []
+
+                def record(st):
+                    seen.append(ds.scatter_f64_route(faces, n, 0, m, stream=st))
+                    ds.scatter_f64(d_in, faces, n, 0, m, out, stream=st)
+
+                g = Graph(record)
+                there = eager[n][:3] in (eager[warm][:3], fewest[:3])
+                assert seen == [eager[n] if there else fewest], (warm, n)
+                ds.scatter_f64(d_in, faces, n, 0, m, ref)
+                D.synchronize()
+                want = ref.to_host().reshape(-1)[:m * n]
+                for _ in range(2):
+                    out.fill(-1.0)
+                    D.synchronize()
+                    g.replay()
+                    assert np.array_equal(out.to_host().reshape(-1)[:m * n], want), (warm, n)
+                g.close()
+    for a in (d_in, out, ref):
+        a.free()
