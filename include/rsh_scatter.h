@@ -59,7 +59,7 @@ typedef enum {
 
 /* FP64 kernel family. */
 typedef enum {
-    RSH_F64_AUTO = 0,      /* MFMA GEMM with the tuned tile                      */
+    RSH_F64_AUTO = 0,      /* by size: rsh_scatter_f64_route                     */
     RSH_F64_DIRECT = 1,    /* one thread per (cell, direction), reference order  */
     RSH_F64_MFMA = 2       /* MFMA GEMM, tile given by rsh_tile                  */
 } rsh_f64_kernel;
@@ -138,7 +138,10 @@ int rsh_dirset_phase_matrix(rsh_dirset ds, int32_t k0, int32_t k1, double* host_
  *   d_illum : [M][n_cells][faces] doubles (faces = 4 as in the reference, or 1
  *             for cell-averaged input)
  *   d_out   : rows k0..k1-1 written to d_out[(k - k0) * ld_out + c]
- * kernel = rsh_f64_kernel; tile may be NULL (tuned / default tile).
+ * kernel = rsh_f64_kernel; tile is for RSH_F64_MFMA (NULL: as RSH_F64_AUTO). The
+ * first call on a range of rows builds its phase panel, in the layout of the route
+ * and in that of fewest passes, which any size can run with: after it, calls of
+ * every size can be captured.
  * Replaces d_GetS / d_GetS_MPI / d_GetS_MPI_Stream (cuda/cuda_kernel.cu:23-111). */
 int rsh_scatter_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int64_t n_cells,
                         int32_t k0, int32_t k1, double* d_out, int64_t ld_out, void* stream,
@@ -290,8 +293,10 @@ int rsh_event_elapsed_ms(void* ev_start, void* ev_stop, float* ms);
 /* ------------------------------------------------ tile autotuner */
 /* Times every supported FP64 MFMA tile on a synthetic problem (n_cells cells,
  * m directions, all m output rows) and records the fastest for the row-block
- * class of m; later single-problem FP64 launches (RSH_F64_AUTO) of that class
- * use it. Batches use the grouped kernel's own tile (4 waves, 2 j-steps per
+ * class of m: the blocks per pass of the plan of fewest passes. Later
+ * single-problem FP64 launches (RSH_F64_AUTO) that run such a plan of that class
+ * use it; sizes that run faster in more passes or with the register-fed kernel
+ * (rsh_scatter_f64_route) do not. Batches use the grouped kernel's own tile (4 waves, 2 j-steps per
  * stage, at most 13 row blocks per pass). No reference counterpart. */
 int rsh_autotune_f64(int32_t device, int32_t m, int32_t faces, int64_t n_cells, rsh_tile* best, float* best_ms);
 int rsh_tuned_tile_f64(int32_t device, int32_t m, rsh_tile* tile);

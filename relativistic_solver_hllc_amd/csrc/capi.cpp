@@ -148,15 +148,17 @@ static int runnable_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st
 static int choose_f64(rsh_dirset ds, int faces, int64_t n, int k0, int k1, hipStream_t st, F64Route* run,
                       bool* have_least, PanelRef* found) {
     const F64Route rt = route_f64(ds->m, k1 - k0, faces, n, device_cus(ds->device));
+    const F64Plan least = plan_f64(ds->m, k1 - k0);
     *run = rt;
-    if (int rc = runnable_f64(ds, k0, k1, faces, st, rt.plan, plan_f64(ds->m, k1 - k0), &run->plan, have_least, found))
-        return rc;
+    if (int rc = runnable_f64(ds, k0, k1, faces, st, rt.plan, least, &run->plan, have_least, found)) return rc;
     if (run->plan.paired) {
         run->waves = run->chunk_steps = 0;
         return RSH_OK;
     }
+    // rsh_autotune_f64 times plans of fewest passes: its tile is for those only. A plan
+    // in place of the route's takes the default tile else, not the route's.
     rsh_tile t{8, 2};
-    const bool tuned = f64_tile_tuned(ds->device, run->plan.rb_per_pass, &t);
+    const bool tuned = run->plan.passes == least.passes && f64_tile_tuned(ds->device, run->plan.rb_per_pass, &t);
     if (tuned || rt.plan.paired || run->plan.passes != rt.plan.passes) *run = F64Route{run->plan, t.waves, t.chunk_steps};
     return RSH_OK;
 }
@@ -272,7 +274,7 @@ int scatter_f64(rsh_dirset ds, const double* d_illum, int faces, int64_t n, int6
     }
     if (kernel != RSH_F64_AUTO && kernel != RSH_F64_MFMA) return fail(RSH_E_ARG, "unknown FP64 kernel id");
     // A given tile runs the LDS-panel kernel with it; otherwise the route for
-    // this size, with the tile that rsh_autotune_f64 recorded for the class.
+    // this size, with the tile that rsh_autotune_f64 recorded for its plan.
     const F64Plan least = plan_f64(ds->m, k1 - k0);
     F64Route rt;
     PanelRef pe;  // held until the launch is enqueued

@@ -90,7 +90,7 @@ int rsh_scatter_f64_dev_noalloc(rsh_dirset ds, const double* d_illum, int32_t fa
         return RSH_OK;
     }
     rsh_tile t{rt.waves, rt.chunk_steps};
-    (void)f64_tile_tuned(ds->device, pl.rb_per_pass, &t);
+    if (pl.passes == lds_plan.passes) (void)f64_tile_tuned(ds->device, pl.rb_per_pass, &t);  // timed on such plans only
     RSH_HIP_TRY(launch_mfma_f64(d_illum, faces, n_cells, n_cells, ds->m, static_cast<const double*>(panel), pl,
                                 k1 - k0, d_out, ld_out, t.waves, t.chunk_steps, st));
     return RSH_OK;

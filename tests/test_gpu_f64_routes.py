@@ -12,7 +12,7 @@ from relativistic_solver_hllc_amd import scatter as rs
 pytestmark = pytest.mark.gpu
 
 # (cells, directions, faces, k0, k1): edges of the 16-cell tile, the 4- and 8-direction steps and the 16-row block;
-# then sizes that take 1-8 and 10 row blocks per wave, two passes of four waves, and a range of rows
+# then larger sizes, and ranges of rows
 SIZES = [(1, 1, 4, 0, 1), (15, 3, 4, 0, 3), (16, 4, 1, 0, 4), (17, 8, 4, 0, 8), (63, 9, 1, 0, 9), (65, 16, 4, 0, 16),
          (66, 17, 4, 0, 17), (381, 327, 4, 0, 327), (381, 327, 1, 5, 22), (1003, 302, 4, 0, 302), (2958, 200, 4, 0, 200),
          (2959, 302, 4, 0, 302), (2957, 400, 1, 0, 400), (5001, 302, 4, 0, 302), (5000, 400, 4, 0, 400),
@@ -47,3 +47,22 @@ def test_route_equals_lds_panel_kernel(gpu, n, m, faces, k0, k1):
         P = orc.phase_matrix(xyz, w, F, 1, 0.6, True)
         ref = orc.scatter_matrix(np.ascontiguousarray(illum[:, cells]), P)[k0:k1]
         assert np.max(np.abs(got[:, cells] - ref) / ref) < 1e-12
+
+
+def test_tuned_tile_is_for_the_plan_that_was_timed(gpu):
+    """rsh_autotune_f64 at 200 directions times thirteen row blocks in one pass. 400 directions of some sizes run as two
+    passes of thirteen, in workgroups of eight waves or of four: their route stays, whatever tile the class has. A size
+    of the class in one pass takes the tile."""
+    def dirset(m):
+        xyz, w, F = rs.fibonacci_directions(m)
+        return rs.DirectionSet(xyz, w, F)
+
+    with dirset(400) as two, dirset(200) as one:
+        def routes():
+            return [two.scatter_f64_route(4, n, 0, 400) for n in (14001, 17001)]
+
+        assert routes() == [("panel", 13, 2, 8), ("panel", 13, 2, 4)]
+        tile, _ = rs.autotune_f64(200, faces=4, n_cells=4096)
+        assert rs.tuned_tile_f64(200) == tile
+        assert routes() == [("panel", 13, 2, 8), ("panel", 13, 2, 4)]
+        assert one.scatter_f64_route(4, 300000, 0, 200) == ("panel", 13, 1, tile[0])
