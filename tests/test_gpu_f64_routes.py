@@ -66,3 +66,35 @@ def test_tuned_tile_is_for_the_plan_that_was_timed(gpu):
         assert rs.tuned_tile_f64(200) == tile
         assert routes() == [("panel", 13, 2, 8), ("panel", 13, 2, 4)]
         assert one.scatter_f64_route(4, 300000, 0, 200) == ("panel", 13, 1, tile[0])
+
+
+# One size per kind of route: (cells, directions, faces): row blocks and groups of the register-fed kernel, or row
+# blocks per pass, passes and waves of the LDS-panel kernel
+ROUTES = {(15, 400, 4): ("register", 1, 25, 0), (13521, 27, 4): ("register", 2, 1, 0),
+          (2958, 200, 4): ("register", 3, 5, 0), (2959, 302, 4): ("register", 4, 5, 0),
+          (2957, 400, 1): ("register", 5, 5, 0), (5001, 257, 4): ("register", 6, 3, 0),
+          (14571, 109, 1): ("register", 7, 1, 0), (5001, 350, 4): ("register", 8, 3, 0),
+          (8097, 281, 4): ("register", 10, 2, 0), (40001, 302, 4): ("panel", 19, 1, 4),
+          (14001, 400, 4): ("panel", 13, 2, 8), (40001, 400, 4): ("panel", 13, 2, 4),
+          (33001, 400, 1): ("panel", 5, 5, 4), (150001, 113, 4): ("panel", 8, 1, 8)}
+
+
+@pytest.mark.parametrize("size", ROUTES)
+def test_every_kind_of_route_equals_the_lds_panel_kernel(gpu, size):
+    """The route is the one meant (on 256 CUs; a class that another test has tuned takes its tile's waves), and its
+    results are the given tile's bit for bit."""
+    n, m, faces = size
+    rng = np.random.default_rng(n + m)
+    illum = rng.lognormal(0.0, 1.5, size=(m, n) if faces == 1 else (m, n, faces))
+    xyz, w, F = rs.fibonacci_directions(m)
+    d_in = D.DeviceArray.from_host(illum)
+    with rs.DirectionSet(xyz, w, F, phase="hg", g=0.6, normalize=True) as ds:
+        route = ds.scatter_f64_route(faces, n, 0, m)
+        kernel, blocks, passes, waves = ROUTES[size]
+        if kernel == "panel" and passes == 1 and rs.tuned_tile_f64(m) != (8, 2):
+            waves = rs.tuned_tile_f64(m)[0]
+        assert route == (kernel, blocks, passes, waves)
+        got = evaluate(ds, d_in, faces, n, 0, m)
+        want = evaluate(ds, d_in, faces, n, 0, m, kernel="mfma", tile=(8, 2))
+    d_in.free()
+    assert np.array_equal(got, want)
