@@ -153,16 +153,20 @@ int rsh_scatter_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  * same bits. No reference counterpart. */
 typedef enum {
     RSH_KERNEL_PANEL = 0,    /* FP64: phase panel staged through LDS             */
-    RSH_KERNEL_REGISTER = 1  /* FP64: one wave per 16 cells and row group, no LDS */
+    RSH_KERNEL_REGISTER = 1, /* FP64: one wave per 16 cells and row group, no LDS */
+    RSH_KERNEL_RESIDENT = 2, /* split: panel slice resident in LDS (waves 0)     */
+    RSH_KERNEL_STREAMING = 3 /* split: panel streamed through LDS                */
 } rsh_route_kernel;
 typedef struct {
     int32_t kernel;      /* rsh_route_kernel                                     */
     int32_t row_blocks;  /* 16-row blocks per pass or row group                  */
     int32_t passes;      /* passes or row groups                                 */
-    int32_t waves;       /* waves per workgroup (0: RSH_KERNEL_REGISTER)         */
+    int32_t waves;       /* waves per workgroup (RSH_KERNEL_PANEL, _STREAMING; else 0) */
 } rsh_route;
 int rsh_scatter_f64_route(rsh_dirset ds, int32_t faces, int64_t n_cells, int32_t k0, int32_t k1, void* stream,
                           rsh_route* route);
+int rsh_scatter_split_route(rsh_dirset ds, int32_t form, int32_t faces, int64_t n_cells, int32_t k0, int32_t k1,
+                            int64_t ld_out, void* stream, rsh_route* route);
 
 /* Radiation moments over all M directions of ds, per cell, on caller-owned
  * device memory:
@@ -205,7 +209,8 @@ int rsh_moments_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  *                          tile, each with half of the rows); 1 = resident-panel
  *                          kernel (faces = 1 only: each persistent workgroup
  *                          keeps its rows' panel for all directions in LDS);
- *                          0 = resident-panel kernel where it applies, else 8.
+ *                          0 = resident-panel kernel where it applies and keeps
+ *                          most CUs busy (rsh_scatter_split_route), else 8.
  *                          All kernels give bit-identical results. */
 int rsh_split_sizes(int32_t form, int32_t faces, int64_t n_cells, int32_t m, int64_t* state_bytes,
                     int64_t* scale_bytes);

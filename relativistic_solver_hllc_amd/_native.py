@@ -91,6 +91,7 @@ PROTOTYPES = {
     "rsh_dirset_phase_matrix": (C.c_int, [vp, i32, i32, vp]),
     "rsh_scatter_f64_dev": (C.c_int, [vp, vp, i32, i64, i32, i32, vp, i64, vp, i32, C.POINTER(Tile)]),
     "rsh_scatter_f64_route": (C.c_int, [vp, i32, i64, i32, i32, vp, C.POINTER(Route)]),
+    "rsh_scatter_split_route": (C.c_int, [vp, i32, i32, i64, i32, i32, i64, vp, C.POINTER(Route)]),
     "rsh_split_sizes": (C.c_int, [i32, i32, i64, i32, C.POINTER(i64), C.POINTER(i64)]),
     "rsh_pack_split_dev": (C.c_int, [i32, vp, i32, i64, i32, vp, vp, vp]),
     "rsh_scatter_split_dev": (C.c_int, [vp, i32, vp, vp, i32, i64, i32, i32, vp, i64, i32, vp, i32]),

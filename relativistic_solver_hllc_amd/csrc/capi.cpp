@@ -329,6 +329,29 @@ bool valid_split_form(int form) {
     return form == RSH_FORM_BF16X2 || form == RSH_FORM_FP16X2 || form == RSH_FORM_BF16X3;
 }
 
+// Automatic choice where the resident-panel kernel has a plan: that kernel when its row
+// groups keep at least 3/4 of the CUs busy, else (11 groups: 22 of 32 CUs of an XCD; 17
+// or 18: M = 769 to 832) up to ten 256-cell chunks per set with an unrolled instance
+// (M <= 800), one without; beyond, the streaming kernel. us, resident / streaming:
+//   800 directions, two parts 3000 cells 28 / 49, 20,000 106 / 142, 100,000 629 / 600;
+//     three parts 44 / 70, 197 / 205, 1054 / 910
+//   820 directions, two parts 500 cells 12 / 37, 3000 38 / 38, 10,000 80 / 74, 40,000 290 / 287;
+//     three parts 19 / 57, 46 / 57, 132 / 113, 496 / 439
+//   500 rows of 700 directions, two parts 3000 cells 15 / 28, 40,000 111 / 134; three 27 / 40, 176 / 196
+// A capture takes the kernel whose panel is there, the streaming one if both are not.
+bool choose_split_resident(rsh_dirset ds, int form, int faces, int64_t n, int k0, int k1, hipStream_t st,
+                           const SplitPlan& rplan, int sets) {
+    constexpr int kUnrolledSteps = 25;
+    if (4 * sets * rplan.passes >= 3 * (device_cus(ds->device) / 8)) return true;
+    const bool resident = n <= (int64_t)(rplan.steps <= kUnrolledSteps ? 10 : 1) * 256 * 8 * sets;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+        const bool have = split_panel_cached(ds, k0, k1, faces, form, &rplan);
+        return have && (resident || !split_panel_cached(ds, k0, k1, faces, form, nullptr));
+    }
+    return resident;
+}
+
 int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_cell_inv, int faces, int64_t n,
                   int k0, int k1, void* d_out, int64_t ld, int out_f32, int waves, hipStream_t st) {
     if (waves != 0 && waves != 1 && waves != 4 && waves != 8)
@@ -348,26 +371,8 @@ int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_c
     if (waves == 1 && !resident_ok)
         return fail(RSH_E_UNSUPPORTED, "resident-panel kernel needs cell-level state (faces = 1), ld_out below 2^24 "
                                        "and a panel slice that fits LDS with at most one row group per CU of an XCD");
-    // Auto: the resident-panel kernel when its row groups keep at least 3/4 of
-    // the CUs busy, else (M = 769 to 800 needs 17 groups of 3 row blocks: 17 of 32
-    // CUs per XCD) the streaming kernel with 8 waves, but the resident one up to
-    // ten 256-cell chunks per set. us, resident / streaming, 800 directions: 3000 cells
-    // two parts 28 / 49, three 44 / 70; 20,000 cells 106 / 142, 197 / 205;
-    // 100,000 cells 629 / 600, 1054 / 910. A capture takes the form whose panel
-    // is there, the streaming one if both are not.
-    const int per_xcd = device_cus(ds->device) / 8;
-    if (waves == 0) {
-        bool resident = resident_ok && 4 * sets * rplan.passes >= 3 * per_xcd;
-        if (resident_ok && !resident) {
-            resident = n <= (int64_t)10 * 256 * 8 * sets;
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
-                const bool have = split_panel_cached(ds, k0, k1, faces, form, &rplan);
-                resident = have && (resident || !split_panel_cached(ds, k0, k1, faces, form, nullptr));
-            }
-        }
-        waves = resident ? 1 : split_default_waves();
-    }
+    if (waves == 0)
+        waves = resident_ok && choose_split_resident(ds, form, faces, n, k0, k1, st, rplan, sets) ? 1 : split_default_waves();
     PanelRef pe;  // held until the launch is enqueued
     if (waves == 1) {
         int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe, &rplan);
@@ -396,6 +401,26 @@ int rsh_scatter_f64_route(rsh_dirset ds, int32_t faces, int64_t n_cells, int32_t
     bool have_least;
     if (int rc = choose_f64(ds, faces, n_cells, k0, k1, (hipStream_t)stream, &rt, &have_least, nullptr)) return rc;
     *route = rsh_route{rt.plan.paired ? RSH_KERNEL_REGISTER : RSH_KERNEL_PANEL, rt.plan.rb_per_pass, rt.plan.passes, rt.waves};
+    return RSH_OK;
+}
+
+int rsh_scatter_split_route(rsh_dirset ds, int32_t form, int32_t faces, int64_t n_cells, int32_t k0, int32_t k1,
+                            int64_t ld_out, void* stream, rsh_route* route) {
+    if (!ds || !route) return fail(RSH_E_ARG, "null direction set or route");
+    if (!valid_split_form(form)) return fail(RSH_E_ARG, "not a split form");
+    if (faces != 1 && faces != 4) return fail(RSH_E_UNSUPPORTED, "faces must be 1 or 4");
+    if (n_cells <= 0 || ld_out < n_cells || k0 < 0 || k1 > ds->m || k0 >= k1)
+        return fail(RSH_E_ARG, "invalid cell count, row stride or direction range");
+    SplitPlan pl{};
+    int sets = 0;
+    if (faces == 1 && ld_out < kSplitResidentMaxLd &&
+        plan_split_resident(form, ds->m, k1 - k0, device_cus(ds->device), &pl, &sets, false) &&
+        choose_split_resident(ds, form, faces, n_cells, k0, k1, (hipStream_t)stream, pl, sets)) {
+        *route = rsh_route{RSH_KERNEL_RESIDENT, pl.rb_per_pass, pl.passes, 0};
+        return RSH_OK;
+    }
+    pl = plan_split(ds->m, k1 - k0);
+    *route = rsh_route{RSH_KERNEL_STREAMING, pl.rb_per_pass, pl.passes, split_default_waves()};
     return RSH_OK;
 }
 

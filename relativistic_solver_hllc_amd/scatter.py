@@ -29,7 +29,7 @@ from . import _native as N
 PHASES = {"thomson": 0, "hg": 1}
 FORMS = {"fp64": 0, "bf16x2": 1, "fp16x2": 2, "bf16x3": 3}
 F64_KERNELS = {"auto": 0, "direct": 1, "mfma": 2}
-ROUTE_KERNELS = {0: "panel", 1: "register"}
+ROUTE_KERNELS = {0: "panel", 1: "register", 2: "resident", 3: "streaming"}
 STREAM_SCATTERING_1, STREAM_SCATTERING_2, STREAM_PARAMS = 0, 1, 2
 
 
@@ -216,6 +216,14 @@ class DirectionSet:
         """Split-precision S rows [k0, k1) from a packed state (see pack_split_dev)."""
         N.call("rsh_scatter_split_dev", self.handle, FORMS[form], _ptr(state), _ptr(cell_scale), faces, n_cells, k0,
                k1, _ptr(out), n_cells if ld is None else ld, int(out_f32), _stream(stream), waves)
+
+    def scatter_split_route(self, form: str, faces: int, n_cells: int, k0: int, k1: int, ld: Optional[int] = None,
+                            stream=None) -> Tuple[str, int, int, int]:
+        """What an automatic scatter_split of these sizes runs: (kernel, row blocks, passes or groups, waves)."""
+        r = N.Route()
+        N.call("rsh_scatter_split_route", self.handle, FORMS[form], faces, n_cells, k0, k1,
+               n_cells if ld is None else ld, _stream(stream), C.byref(r))
+        return ROUTE_KERNELS[r.kernel], r.row_blocks, r.passes, r.waves
 
     def moments(self, illum, faces: int, n_cells: int, energy=None, stream_out=None, impuls=None, divstream=None,
                 divimpuls=None, normals=None, areas=None, volume=None, faces_per_thread: int = 0,

@@ -358,3 +358,46 @@ def test_cell_pack_matches_layout_definition(gpu, form, faces):
         r = (r - p).astype(np.float32)
     assert np.array_equal(vals[:, m:, :], np.zeros_like(vals[:, m:, :]))    # padding directions
     assert np.array_equal(vals[:, :, n:], np.zeros_like(vals[:, :, n:]))    # padding cells
+
+
+@pytest.mark.parametrize("form", ["bf16x2", "bf16x3"])
+def test_automatic_choice_of_plans_that_leave_cus_idle(gpu, form):
+    """Where row groups leave a quarter of an XCD's 32 CUs idle (17 or 18 groups: 769 to 832 directions; 11 groups: some
+    ranges of rows) the resident kernel is chosen up to ten 256-cell chunks per set if its K loop is unrolled (800
+    directions and fewer), up to one else, where it was measured to be the faster one; with full XCDs always."""
+    def kernel(ds, n, k1, faces=1, ld=None):
+        return ds.scatter_split_route(form, faces, n, 0, k1, ld=ld)[0]
+
+    def dirset(m):
+        xyz, w, F = rs.fibonacci_directions(m)
+        return rs.DirectionSet(xyz, w, F)
+
+    for m, k1, line in ((800, 800, 20480), (700, 500, 40960), (820, 820, 2048)):
+        with dirset(m) as ds:
+            assert [kernel(ds, n, k1) for n in (1, line, line + 1, 10 * line)] == ["resident"] * 2 + ["streaming"] * 2
+            assert kernel(ds, 17, k1, faces=4) == "streaming" and kernel(ds, 17, k1, ld=1 << 24) == "streaming"
+    for m in (400, 640, 1000):
+        with dirset(m) as ds:
+            assert [kernel(ds, n, m) for n in (1, 1 << 22)] == ["resident"] * 2
+
+
+@pytest.mark.parametrize("n", [2048, 2049])
+def test_automatic_choice_beyond_800_directions(gpu, n):
+    """Both sides of the line at 820 directions (26 K-steps, rolled K loop): the streaming kernel's bits."""
+    m = 820
+    cell = np.resize(np.random.default_rng(n).lognormal(0.0, 1.5, size=1_000_003), (m, n, 1))
+    xyz, w, F = rs.fibonacci_directions(m)
+    with rs.DirectionSet(xyz, w, F) as ds:
+        d_cell, out = D.DeviceArray.from_host(cell), D.DeviceArray((m, n))
+        sb, cb = rs.split_sizes("bf16x3", 1, n, m)
+        state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+        rs.pack_split_dev("bf16x3", d_cell, 1, n, m, state, scale)
+        outs = []
+        for waves in (0, 1, 8):
+            out.fill(-1.0)
+            ds.scatter_split("bf16x3", state, scale, 1, n, 0, m, out, waves=waves)
+            D.synchronize()
+            outs.append(out.to_host())
+        for a in (d_cell, state, scale, out):
+            a.free()
+    assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])
