@@ -112,7 +112,7 @@ static void bound_panels(rsh_dirset ds, const std::tuple<int, int, int, int, int
     }
 }
 
-static bool capturing(hipStream_t st) {
+bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
 }
@@ -338,17 +338,19 @@ bool valid_split_form(int form) {
 //   820 directions, two parts 500 cells 12 / 37, 3000 38 / 38, 10,000 80 / 74, 40,000 290 / 287;
 //     three parts 19 / 57, 46 / 57, 132 / 113, 496 / 439
 //   500 rows of 700 directions, two parts 3000 cells 15 / 28, 40,000 111 / 134; three 27 / 40, 176 / 196
-// A capture takes the kernel whose panel is there, the streaming one if both are not.
+// A capture, which can build no panel, takes the chosen kernel if its panel is there,
+// else the streaming one; that one's panel is there after any automatic call outside
+// a capture that the size decided (*lacks_streaming: it is not yet).
 bool choose_split_resident(rsh_dirset ds, int form, int faces, int64_t n, int k0, int k1, hipStream_t st,
-                           const SplitPlan& rplan, int sets) {
+                           const SplitPlan& rplan, int sets, bool* lacks_streaming) {
     constexpr int kUnrolledSteps = 25;
+    *lacks_streaming = false;
     if (4 * sets * rplan.passes >= 3 * (device_cus(ds->device) / 8)) return true;
     const bool resident = n <= (int64_t)(rplan.steps <= kUnrolledSteps ? 10 : 1) * 256 * 8 * sets;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
-        const bool have = split_panel_cached(ds, k0, k1, faces, form, &rplan);
-        return have && (resident || !split_panel_cached(ds, k0, k1, faces, form, nullptr));
-    }
+    const bool streaming = split_panel_cached(ds, k0, k1, faces, form, nullptr);
+    if (resident ? streaming && split_panel_cached(ds, k0, k1, faces, form, &rplan) : streaming) return resident;
+    if (capturing(st)) return split_panel_cached(ds, k0, k1, faces, form, &rplan) && (resident || !streaming);
+    *lacks_streaming = !streaming;
     return resident;
 }
 
@@ -371,9 +373,14 @@ int scatter_split(rsh_dirset ds, int form, const void* d_state, const float* d_c
     if (waves == 1 && !resident_ok)
         return fail(RSH_E_UNSUPPORTED, "resident-panel kernel needs cell-level state (faces = 1), ld_out below 2^24 "
                                        "and a panel slice that fits LDS with at most one row group per CU of an XCD");
-    if (waves == 0)
-        waves = resident_ok && choose_split_resident(ds, form, faces, n, k0, k1, st, rplan, sets) ? 1 : split_default_waves();
     PanelRef pe;  // held until the launch is enqueued
+    if (waves == 0) {
+        bool lacks_streaming = false;
+        const bool resident = resident_ok && choose_split_resident(ds, form, faces, n, k0, k1, st, rplan, sets, &lacks_streaming);
+        waves = resident ? 1 : split_default_waves();
+        if (resident && lacks_streaming)
+            if (int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe)) return rc;
+    }
     if (waves == 1) {
         int rc = get_panel_split(ds, k0, k1, faces, form, st, &pe, &rplan);
         if (rc) return rc;
@@ -413,9 +420,10 @@ int rsh_scatter_split_route(rsh_dirset ds, int32_t form, int32_t faces, int64_t 
         return fail(RSH_E_ARG, "invalid cell count, row stride or direction range");
     SplitPlan pl{};
     int sets = 0;
+    bool lacks_streaming;
     if (faces == 1 && ld_out < kSplitResidentMaxLd &&
         plan_split_resident(form, ds->m, k1 - k0, device_cus(ds->device), &pl, &sets, false) &&
-        choose_split_resident(ds, form, faces, n_cells, k0, k1, (hipStream_t)stream, pl, sets)) {
+        choose_split_resident(ds, form, faces, n_cells, k0, k1, (hipStream_t)stream, pl, sets, &lacks_streaming)) {
         *route = rsh_route{RSH_KERNEL_RESIDENT, pl.rb_per_pass, pl.passes, 0};
         return RSH_OK;
     }

@@ -112,3 +112,42 @@ def test_captured_f64_kernel_does_not_depend_on_the_warm_up_size(gpu, faces):
                 g.close()
     for a in (d_in, out, ref):
         a.free()
+
+
+@pytest.mark.parametrize("m,few,many", [(800, 3000, 30000), (820, 1000, 5000)])
+def test_captured_split_kernel_does_not_depend_on_the_warm_up_size(gpu, m, few, many):
+    """Where the size decides between the resident and the streaming kernel: after a call of either size a captured large
+    call runs the streaming kernel, and a captured small one the resident kernel if its panel is there. The graph's
+    results are the eager call's."""
+    form = "bf16x2"
+    d_in, out, ref = (D.DeviceArray((m, many)) for _ in range(3))
+    N.call("rsh_fill_lognormal_dev", d_in.ptr, d_in.size, 0.0, 1.0, 7, None)
+    state, scale = {}, {}
+    for n in (few, many):
+        sb, cb = rs.split_sizes(form, 1, n, m)
+        state[n], scale[n] = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+        rs.pack_split_dev(form, d_in, 1, n, m, state[n], scale[n])
+    for warm in (few, many):
+        for n in (few, many):
+            with dirset(m) as ds:
+                ds.scatter_split(form, state[warm], scale[warm], 1, warm, 0, m, out)
+                D.synchronize()
+                seen = []
+
+                def record(st):
+                    seen.append(ds.scatter_split_route(form, 1, n, 0, m, stream=st)[0])
+                    ds.scatter_split(form, state[n], scale[n], 1, n, 0, m, out, stream=st)
+
+                g = Graph(record)
+                assert seen == ["resident" if n == warm == few else "streaming"], (warm, n)
+                ds.scatter_split(form, state[n], scale[n], 1, n, 0, m, ref)
+                D.synchronize()
+                want = ref.to_host().reshape(-1)[:m * n]
+                for _ in range(2):
+                    out.fill(-1.0)
+                    D.synchronize()
+                    g.replay()
+                    assert np.array_equal(out.to_host().reshape(-1)[:m * n], want), (warm, n)
+                g.close()
+    for a in (d_in, out, ref, *state.values(), *scale.values()):
+        a.free()
