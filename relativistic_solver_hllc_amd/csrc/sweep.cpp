@@ -36,7 +36,9 @@ struct rsh_sweep_s {
     };
     std::vector<Dir> dirs;
     // Host arrays of one direction's plan, kept for the next one (a call takes a
-    // set of its own: fresh pages would cost more than half of the planning).
+    // set of its own: fresh pages would cost more than half of the planning) until
+    // every direction is set; at most kSpare sets of about 125 bytes per cell.
+    static constexpr size_t kSpare = 8;
     struct Cell {
         int32_t link;   // place in the given order; then, ready: the next cell of its list, taken: its first out face's position
         int32_t chain;  // cells in the longest chain before it; then in the longest one that still waits on it
@@ -51,7 +53,8 @@ struct rsh_sweep_s {
         std::unique_ptr<char[]> image;  // what is uploaded
         size_t room = 0;
     };
-    std::vector<std::unique_ptr<Work>> spare;
+    std::vector<std::unique_ptr<Work>> spare;  // capacity kSpare
+    int unset = 0;  // directions not set
     SweepDirDev* d_table = nullptr;
     bool table_dirty = true;
     std::mutex mu;
@@ -83,6 +86,8 @@ int rsh_sweep_create(int32_t device, int64_t n_cells, int32_t n_dirs, const int3
     s->m = n_dirs;
     s->pairs.assign(pairs, pairs + n_cells * 4);
     s->dirs.resize((size_t)n_dirs);
+    s->unset = n_dirs;
+    s->spare.reserve(rsh_sweep_s::kSpare);
     auto cleanup = [&](int rc) {
         rsh_sweep_destroy(s);
         return rc;
@@ -119,7 +124,7 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
         return fail(RSH_E_ARG, "invalid direction, null pointer or record count");
     const int64_t n = s->n;
     const int32_t* pairs = s->pairs.data();
-    struct Lease {  // a Work of this call, given back at its end
+    struct Lease {  // a Work of this call, given back at its end (freed with the others once every direction is set)
         rsh_sweep s;
         std::unique_ptr<rsh_sweep_s::Work> w;
         explicit Lease(rsh_sweep sw) : s(sw) {
@@ -132,7 +137,8 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
         }
         ~Lease() {
             std::lock_guard<std::mutex> lock(s->mu);
-            s->spare.push_back(std::move(w));
+            if (s->unset == 0) s->spare.clear();
+            else if (s->spare.size() < rsh_sweep_s::kSpare) s->spare.push_back(std::move(w));
         }
     } lease(s);
     rsh_sweep_s::Work& w = *lease.w;
@@ -377,6 +383,7 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     auto& d = s->dirs[(size_t)k];
     if (d.block) RSH_HIP_TRY(hipFree(d.block));
     d.block = nullptr;
+    if (d.set) s->unset++;
     d.set = false;
     if (hipMalloc(&d.block, bytes) != hipSuccess) return fail(RSH_E_NOMEM, "sweep: direction allocation failed");
     if (hipMemcpy(d.block, w.image.get(), bytes, hipMemcpyHostToDevice) != hipSuccess)
@@ -392,6 +399,7 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     d.dev.levels = levels;
     d.dev.fixes = (int32_t)(fix.size() / 2);
     d.set = true;
+    s->unset--;
     s->table_dirty = true;
     return RSH_OK;
 }

@@ -262,3 +262,34 @@ def test_sweep_all_directions_at_196608_cells(gpu):
     assert n == 196608 and len(levels) == m and max(levels) > 100
     check(got, ref)
     assert norm.max() == pytest.approx(ref_norm, rel=1e-10)
+
+
+def malloc_in_use():
+    import ctypes
+
+    class Info(ctypes.Structure):
+        _fields_ = [(f, ctypes.c_size_t) for f in ("arena ordblks smblks hblks hblkhd usmblks fsmblks uordblks "
+                                                   "fordblks keepcost").split()]
+
+    libc = ctypes.CDLL(None)
+    libc.mallinfo2.restype = Info
+    i = libc.mallinfo2()
+    return i.uordblks + i.hblkhd
+
+
+def test_planning_memory_is_given_back(gpu):
+    """The host arrays of the planning (about 100 bytes per cell and up) are kept between directions only until all
+    are set: then the sweep holds its copy of the pairs (16 bytes per cell) and no more, also after a direction is
+    set again."""
+    v, pairs = sw.mesh_cube_tetra(24)
+    n = pairs.shape[0]
+    dirs = rs.fibonacci_directions(3)[0]
+    per = sw.prepare(v, pairs, dirs)
+    with sw.Sweep(n, 3, pairs) as first:  # what the runtime allocates once
+        first.set_all(iter(per))
+    before = malloc_in_use()
+    with sw.Sweep(n, 3, pairs) as s:
+        s.set_all(iter(per))
+        assert malloc_in_use() - before < 40 * n
+        s.set_direction(1, *per[1])
+        assert malloc_in_use() - before < 40 * n
