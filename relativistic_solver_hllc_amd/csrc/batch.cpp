@@ -57,6 +57,10 @@ void set_grouped_tuned(int device, int form, int key, rsh_tile t) {
     g_gtune[{device, form, key}] = t;
 }
 
+// Split kernel of the tuner's batches: the resident one, 8 waves, for every M that has a
+// plan (by name, 1, only the M of iter_split_res_selectable), whatever is recorded.
+constexpr int kResidentAnyM = -1;
+
 struct Slot {
     bool active = false;
     rsh_dirset ds = nullptr;
@@ -108,7 +112,7 @@ struct rsh_batch_s {
     BatchProblem* d_probs = nullptr;
     unsigned long long* d_resid = nullptr;  // 2 * capacity
     unsigned* d_counters = nullptr;         // kMaxClasses * kXcdLists
-    int split_kernel = 0;                   // 0 auto, 1 resident panel, 2 streaming panel, 3 resident, 4 waves
+    int split_kernel = 0;                   // 0 auto, 1 resident panel, 2 streaming panel, 3 resident, 4 waves, kResidentAnyM
     rsh_tile f64_tile{0, 0};                // FP64 grouped tile of new classes; {0, 0} = tuned or default
     std::map<std::pair<int, int>, ClassState> classes;  // by (form, row-block class)
     bool lists_dirty = true;
@@ -491,11 +495,11 @@ int add_impl(rsh_batch b, rsh_dirset ds, int64_t n_cells, double albedo, int for
         int sets = 0;
         if (plan_split_resident(form, ds->m, ds->m, device_cus(b->device), &rplan, &sets, true) &&
             iter_split_res_supported(form, rplan.rb_per_pass, rplan.steps) &&
-            (split_kernel == 0 || iter_split_res_selectable(rplan.steps))) {
+            (split_kernel == 0 || split_kernel == kResidentAnyM || iter_split_res_selectable(rplan.steps))) {
             s.splan = rplan;
             s.res = true;
             s.res_waves = split_kernel == 3 ? 4 : 8;
-        } else if (split_kernel == 1 || split_kernel == 3) {
+        } else if (split_kernel != 0) {
             return fail(RSH_E_UNSUPPORTED, "resident-panel iteration kernel: no specialised plan for this M");
         }
     }
@@ -706,10 +710,11 @@ int rsh_batch_autotune(int32_t device, int32_t form, int32_t m, int64_t n_cells,
         int slot = -1;
         if (form == RSH_FORM_FP64)
             rc = rsh_batch_set_f64_tile(bb, &cands[c]);
-        else  // the eight-wave resident kernel is what the automatic choice takes where it has a plan for M
-            rc = rsh_batch_set_split_kernel(bb, cands[c].waves == 1 ? 0 : cands[c].waves);
+        else
+            bb->split_kernel = cands[c].waves == 1 ? kResidentAnyM : cands[c].waves;
         if (!rc) rc = rsh_batch_add_seeded(bb, ds, n_cells, 0x7E57ull, 0.5, form, &slot);
-        if (!rc && form != RSH_FORM_FP64 && cands[c].waves == 1 && !bb->slots[slot].res) rc = RSH_E_UNSUPPORTED;
+        // 2^24 cells and more: a slot of the streaming kernel, whatever was asked for
+        if (!rc && form != RSH_FORM_FP64 && cands[c].waves != 2 && !bb->slots[slot].res) rc = RSH_E_UNSUPPORTED;
         if (rc == RSH_E_UNSUPPORTED) {  // candidate does not apply (e.g. no resident plan for this M)
             rsh_batch_destroy(bb);
             rc = RSH_OK;

@@ -429,3 +429,17 @@ def test_batch_autotune_choice_is_used_and_every_tile_agrees(gpu):
             s = add_form(b, p, form)
             assert b.slot_config(s, form) == kchoice
     p["ds"].close()
+
+
+@pytest.mark.parametrize("form", ["fp16x2", "bf16x3"])
+def test_batch_autotune_does_not_time_its_own_record(gpu, form):
+    """A second tuning of a form and M times the same kernels as the first, whatever that recorded. At 2^24 cells only the
+    streaming kernel applies; 16 directions of 200,000 cells run four times as fast with the resident one, which the
+    next tuning has to find, and new slots of fewer than 2^24 cells take."""
+    assert rs.batch_autotune(form, 16, n_cells=1 << 24, iterations=2)[0] == ("kernel", "streaming")
+    assert rs.batch_tuned(form, 16) == ("kernel", "streaming")
+    choice, ms = rs.batch_autotune(form, 16, n_cells=200000, iterations=20)
+    assert choice == ("kernel", "resident") == rs.batch_tuned(form, 16)
+    xyz, w, F = rs.fibonacci_directions(16)
+    with rs.DirectionSet(xyz, w, F) as ds, rs.Batch(1) as b:
+        assert b.slot_config(b.add_seeded(ds, 1000, 1, 0.5, form), form) == ("kernel", "resident")
