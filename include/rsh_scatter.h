@@ -339,10 +339,11 @@ int rsh_batch_create(int32_t device, int32_t capacity, int32_t use_graph, rsh_ba
 int rsh_batch_destroy(rsh_batch b);
 /* Kernel of the split-form slots added from now on: 0 = auto (the device's
  * tuned choice for the slot's M, else the resident-panel grouped kernel with
- * 8 waves where its plan fits one XCD: M <= 800 with n_cells < 2^24; else the streaming-panel one), 1 = resident panel,
- * 8 waves of 2 cell tiles (rsh_batch_add fails where it does not apply),
- * 2 = streaming panel, 3 = resident panel, 4 waves of 2 cell tiles, two
- * workgroups per CU where the LDS allows (fails as 1). All give bit-identical
+ * 8 waves of 2 cell tiles: M <= 800 with n_cells < 2^24; else the
+ * streaming-panel one), 2 = streaming panel; by name, for M = 193 to 224, 385 to
+ * 416 and 769 to 800 (rsh_batch_add fails for other M; 2^24 cells and more take
+ * the streaming one): 1 = resident panel, 8 waves, 3 = resident panel, 4 waves of
+ * 2 cell tiles, two workgroups per CU where the LDS allows. All give bit-identical
  * states and residuals. No reference counterpart
  * (batching is an extension). */
 int rsh_batch_set_split_kernel(rsh_batch b, int32_t kind);
@@ -357,7 +358,8 @@ int rsh_batch_set_split_kernel(rsh_batch b, int32_t kind);
  *                         (row blocks per pass) choose the MFMA tile (waves,
  *                         j-steps per LDS stage) among (4,2), (4,4), (8,2);
  *                         split forms choose, per M, the resident-panel
- *                         grouped kernel with 8 ({1,0}) or 4 waves ({3,0}) or
+ *                         grouped kernel with 8 waves ({1,0}; M <= 800), with
+ *                         4 ({3,0}; the M of rsh_batch_set_split_kernel) or
  *                         the streaming-panel one ({2,0}).
  *                         Classes (FP64) and slots (split) created afterwards
  *                         in any batch on the device use the choice; every
@@ -654,7 +656,8 @@ int rsh_sweep_destroy(rsh_sweep s);
  * here (calls for different directions may run on several threads). Replaces the per-direction part of ReadIllumGeometry. */
 int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const int32_t* face_state,
                             const double* x0_s, const uint8_t* x0_face, int64_t n_records);
-/* Number of dependency levels of direction k (cells of one level run in parallel). */
+/* Number of dependency levels of direction k: the cells of one read only from
+ * levels before it. (A pass of the parallel sweep takes cells of several.) */
 int rsh_sweep_levels(rsh_sweep s, int32_t k, int32_t* levels);
 
 /* One sweep over all directions on a stream (NULL = null stream), device

@@ -31,8 +31,9 @@ using namespace rsh;
 
 namespace {
 
-// FP64 row-block counts, resident split plans (one per K-step count) and
-// streaming row-block counts of three forms: no mix of problems needs more.
+// No mix of problems has more than 156: 13 FP64 row-block counts, and of each split
+// form 31 resident plans of eight waves, three or four of four waves, 13 streaming
+// row-block counts.
 constexpr int kMaxClasses = 192;
 constexpr int kXcdLists = 8;  // XCDs: the sets of a resident-panel class, and counters per class
 
@@ -500,7 +501,8 @@ int add_impl(rsh_batch b, rsh_dirset ds, int64_t n_cells, double albedo, int for
             s.res = true;
             s.res_waves = split_kernel == 3 ? 4 : 8;
         } else if (split_kernel != 0) {
-            return fail(RSH_E_UNSUPPORTED, "resident-panel iteration kernel: no specialised plan for this M");
+            return fail(RSH_E_UNSUPPORTED, "resident-panel iteration kernel by name: M = 193 to 224, 385 to 416 or 769 to 800 "
+                                           "(the automatic choice takes it for every M up to 800)");
         }
     }
     const size_t fbytes = (size_t)ds->m * n_cells * sizeof(double);

@@ -102,8 +102,9 @@ bool iter_split_res_supported(int form, int rb, int steps) {
 }
 
 // Plans that a caller may ask for by name (rsh_batch_set_split_kernel) and that
-// have a four-wave form: M = 200, 400 and 800 with their neighbours. The others
-// are taken by the automatic choice only.
+// have a four-wave form: M = 193 to 224, 385 to 416, 769 to 800, which were the only
+// ones when the names were given. The others are taken by the automatic choice (and
+// by the tuner's eight-wave candidate) only.
 bool iter_split_res_selectable(int steps) { return steps == 7 || steps == 13 || steps == 25; }
 
 hipError_t launch_grouped_iter_split_res(bool launch, int form, int rb, int steps, int waves, int grid,

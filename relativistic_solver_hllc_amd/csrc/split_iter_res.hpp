@@ -43,7 +43,7 @@ struct IterResArgs {
 };
 
 // Source iteration I <- (1 - a) B + a S(I) on split state for a batch of
-// problems, resident-panel form (the grouped counterpart of the kernel above).
+// problems, resident-panel form (the grouped counterpart of split_single_res.hpp).
 // Work: meta = [problems of the class, row groups G, sets]. Workgroup b runs on
 // XCD b % 8; the G workgroups of a set sit on one XCD and take one row group each
 // of the same chunks at about the same time, so they share its L2 copy of the

@@ -9,7 +9,6 @@ namespace rsh {
 
 constexpr int kResWaves = 8;   // waves per workgroup of the grouped iteration kernel (2 per SIMD)
 constexpr int kResTiles = 2;   // 16-cell tiles per wave of the grouped iteration kernel
-constexpr int kResChunkTiles = kResWaves * kResTiles;  // 256 cells per chunk
 constexpr int kXcds = 8;       // MI355X: 8 XCDs, workgroups dispatched round-robin
 constexpr int kResLdsBytes = 160 * 1024;
 // Buffer descriptor word 3 for raw (untyped) gfx9 buffer access: 32-bit data

@@ -320,9 +320,9 @@ class Batch:
         return slot.value
 
     def set_split_kernel(self, kind: str) -> None:
-        """Kernel for split-form slots added afterwards: "auto", "resident" (resident panel, 8 waves of 2 cell
-        tiles), "resident4" (resident panel, 4 waves of 2 cell tiles, two workgroups per CU where the LDS allows)
-        or "streaming"."""
+        """Kernel for split-form slots added afterwards: "auto", "streaming", or for M = 193 to 224, 385 to 416 and
+        769 to 800 "resident" (resident panel, 8 waves of 2 cell tiles) or "resident4" (4 waves, two workgroups
+        per CU where the LDS allows)."""
         N.call("rsh_batch_set_split_kernel", self.handle,
                {"auto": 0, "resident": 1, "streaming": 2, "resident4": 3}[kind])
 
