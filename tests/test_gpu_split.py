@@ -401,3 +401,45 @@ def test_automatic_choice_beyond_800_directions(gpu, n):
         for a in (d_cell, state, scale, out):
             a.free()
     assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("form", ["bf16x2", "fp16x2", "bf16x3"])
+@pytest.mark.parametrize("n,m", [(33, 100), (70, 250), (36, 512), (65, 513), (64, 896), (131073, 20)])
+def test_face_averaged_pack_instances_agree(gpu, form, n, m):
+    """Each instance of the face-averaged pack (1, 2, 4 and 7 slots of lane pairs, 64-cell groups) against the one through
+    LDS, which takes the same rows followed by zero rows up to 897 directions and more: the same scales and the same
+    bits of the first K-steps, for cells without an intensity and with infinities and NaN too."""
+    rng = np.random.default_rng(n * m)
+    illum = rng.lognormal(0.0, 3.0, size=(m, n, 4)) * rng.choice([-1.0, 1.0], size=(m, n, 4))
+    illum[:, 3] = 0.0
+    illum[m // 2, 5, 1] = np.inf
+    illum[m - 1, 7, 2] = np.nan
+    illum[0, 9, 0], illum[0, 9, 3] = np.inf, -np.inf
+    illum[:, 11] = np.nan
+    illum[9, 32, 0] = -np.inf
+
+    def pack(a):
+        rows, cells = a.shape[:2]
+        d = D.DeviceArray.from_host(np.ascontiguousarray(a))
+        sb, cb = rs.split_sizes(form, 1, cells, rows)
+        state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+        rs.pack_split_avg_dev(form, d, cells, rows, state, scale)
+        D.synchronize()
+        got = state.to_host().view(np.uint16), scale.to_host()[:cells]
+        for x in (d, state, scale):
+            x.free()
+        return got
+
+    parts, steps, rows = (3 if form == "bf16x3" else 2), -(-m // 32), 928
+    cells = min(n, 256)
+    big = np.zeros((rows, cells, 4))
+    big[:m] = illum[:, :cells]
+    (got, scale), (want, want_scale) = pack(illum), pack(big)
+    tile = parts * 64 * 8  # 16-bit values of a tile's K-step
+    got = got.reshape(-1, steps, tile)[:-(-cells // 16)]
+    want = want.reshape(-1, rows // 32, tile)[:, :steps]
+    assert np.array_equal(scale[:cells], want_scale)
+    nan = np.isnan(_part_values(got, form))
+    assert np.array_equal(nan, np.isnan(_part_values(want, form)))
+    assert np.array_equal(got[~nan], want[~nan])
+    assert nan.any() and not nan.reshape(nan.shape[0], -1).all(axis=1).any()
