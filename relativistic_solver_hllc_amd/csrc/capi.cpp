@@ -61,28 +61,24 @@ static int cached_panel(rsh_dirset ds, const std::tuple<int, int, int, int, int>
     out->reset();
     auto it = ds->panels.find(key);
     if (it == ds->panels.end()) return RSH_OK;
-    const PanelEntry& pe = *it->second;
-    if (!pe.built.load(std::memory_order_relaxed)) {
-        const hipError_t q = hipEventQuery(pe.ready);
+    PanelMemory& mem = *it->second->memory;
+    if (!mem.built.load(std::memory_order_relaxed)) {
+        const hipError_t q = hipEventQuery(mem.ready);
         if (q == hipErrorNotReady)
-            RSH_HIP_TRY(hipStreamWaitEvent(st, pe.ready, 0));
+            RSH_HIP_TRY(hipStreamWaitEvent(st, mem.ready, 0));
         else if (q == hipSuccess)
-            pe.built.store(true, std::memory_order_relaxed);
+            mem.built.store(true, std::memory_order_relaxed);
     }
     *out = it->second;
     return RSH_OK;
 }
 
-// Adds a built entry (its kernels are on stream st) to the panel cache.
-static int store_panel(rsh_dirset ds, const std::tuple<int, int, int, int, int>& key, hipStream_t st,
-                       std::shared_ptr<PanelEntry> pe, hipError_t built, PanelRef* out) {
+// Marks the end of a build whose kernels are on stream st.
+static int end_build(PanelMemory& mem, hipStream_t st, hipError_t built) {
     hipError_t e = built;
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&pe->ready, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(pe->ready, st);
-    if (e != hipSuccess) return hip_fail(e, "phase panel build");
-    ds->panels.emplace(key, pe);
-    *out = pe;
-    return RSH_OK;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&mem.ready, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(mem.ready, st);
+    return e == hipSuccess ? RSH_OK : hip_fail(e, "phase panel build");
 }
 
 // Bounded cache, by ranges (k0, k1, faces, form), whatever layouts each is there
@@ -163,20 +159,32 @@ static int choose_f64(rsh_dirset ds, int faces, int64_t n, int k0, int k1, hipSt
     return RSH_OK;
 }
 
-int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out) {
+int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out,
+                  const F64Plan* also) {
     std::lock_guard<std::mutex> lock(ds->mu);
     const auto key = f64_key(k0, k1, faces, plan);
     if (int rc = cached_panel(ds, key, st, out)) return rc;
     if (*out) return RSH_OK;
     bound_panels(ds, key);
-    auto pe = std::make_shared<PanelEntry>();
-    pe->device = ds->device;
-    pe->plan = plan;
-    const int64_t nd = panel_f64_doubles(plan);
-    hipError_t e = hipMalloc(&pe->d_panel, std::max<int64_t>(nd, 1) * sizeof(double));
+    // the same plan, or another thread's call was first
+    if (also && (f64_key(k0, k1, faces, *also) == key || ds->panels.count(f64_key(k0, k1, faces, *also)))) also = nullptr;
+    auto mem = std::make_shared<PanelMemory>();
+    mem->device = ds->device;
+    // panels are whole 512-byte fragments
+    const int64_t nd = panel_f64_doubles(plan), nd2 = also ? panel_f64_doubles(*also) : 0;
+    hipError_t e = hipMalloc(&mem->ptr, std::max<int64_t>(nd + nd2, 1) * sizeof(double));
+    double* const at = static_cast<double*>(mem->ptr);
     if (e == hipSuccess)
-        e = launch_panel_f64(ds->d_P, ds->m, k0, k1, 1.0 / faces, plan, static_cast<double*>(pe->d_panel), st);
-    return store_panel(ds, key, st, pe, e, out);
+        e = launch_panel_f64(ds->d_P, ds->m, k0, k1, 1.0 / faces, plan, at, st, also, also ? at + nd : nullptr);
+    if (int rc = end_build(*mem, st, e)) return rc;
+    const auto entry = [&](const F64Plan& p, double* d) {
+        const auto pe = std::make_shared<PanelEntry>(PanelEntry{mem, d, nullptr, p, SplitPlan{}});
+        ds->panels.emplace(f64_key(k0, k1, faces, p), pe);
+        return pe;
+    };
+    if (also) entry(*also, at + nd);
+    *out = entry(plan, at);
+    return RSH_OK;
 }
 
 static int split_layout(const SplitPlan* resident) {
@@ -197,28 +205,32 @@ int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStrea
     if (*out) return RSH_OK;
     bound_panels(ds, key);
     auto pe = std::make_shared<PanelEntry>();
-    pe->device = ds->device;
     pe->splan = resident ? *resident : plan_split(ds->m, k1 - k0);
-    const int64_t units = split_panel_units(form, pe->splan);
-    hipError_t e = hipMalloc(&pe->d_panel, std::max<int64_t>(units, 1) * 16);
-    if (e == hipSuccess) e = hipMalloc(&pe->d_row_inv, std::max(pe->splan.rb_total * 16, 1) * sizeof(float));
+    pe->memory = std::make_shared<PanelMemory>();
+    pe->memory->device = ds->device;
+    const int64_t units = split_panel_units(form, pe->splan);  // 16 bytes each; the row scales follow
+    hipError_t e = hipMalloc(&pe->memory->ptr, std::max<int64_t>(units * 16 + pe->splan.rb_total * 16 * 4, 1));
+    pe->d_panel = pe->memory->ptr;
+    pe->d_row_inv = reinterpret_cast<float*>(static_cast<char*>(pe->d_panel) + units * 16);
     if (e == hipSuccess)
         e = launch_split_panel(form, ds->d_P, ds->m, k0, k1, 1.0 / faces, pe->splan, pe->d_panel, pe->d_row_inv, st);
-    return store_panel(ds, key, st, pe, e, out);
+    if (int rc = end_build(*pe->memory, st, e)) return rc;
+    ds->panels.emplace(key, pe);
+    *out = pe;
+    return RSH_OK;
 }
 
 }  // namespace rsh
 
-PanelEntry::~PanelEntry() {
-    if (d_panel || d_row_inv) {
+PanelMemory::~PanelMemory() {
+    if (ptr) {
         // Work that read the panel may still be queued on any stream of the
         // device: free only once the device is idle.
         int cur = -1;
         const bool have = hipGetDevice(&cur) == hipSuccess;
         if (hipSetDevice(device) == hipSuccess) {
             hipDeviceSynchronize();
-            hipFree(d_panel);
-            hipFree(d_row_inv);
+            hipFree(ptr);
         }
         if (have && cur != device) hipSetDevice(cur);
     }
@@ -278,7 +290,7 @@ int scatter_f64(rsh_dirset ds, const double* d_illum, int faces, int64_t n, int6
     const F64Plan least = plan_f64(ds->m, k1 - k0);
     F64Route rt;
     PanelRef pe;  // held until the launch is enqueued
-    bool have_least;
+    bool have_least = true, both = false;
     int rc;
     if (tile && kernel == RSH_F64_MFMA) {
         rt = F64Route{least, tile->waves, tile->chunk_steps};
@@ -288,12 +300,13 @@ int scatter_f64(rsh_dirset ds, const double* d_illum, int faces, int64_t n, int6
     } else {
         rc = choose_f64(ds, faces, n, k0, k1, st, &rt, &have_least, &pe);
         // The least-pass panel beside the route's: with it a call of any size can be captured.
-        if (!rc && !have_least && !capturing(st)) {
+        both = !rc && !have_least && !capturing(st);
+        if (both && pe) {
             PanelRef built;
             rc = get_panel_f64(ds, k0, k1, faces, st, least, &built);
         }
     }
-    if (!rc && !pe) rc = get_panel_f64(ds, k0, k1, faces, st, rt.plan, &pe);
+    if (!rc && !pe) rc = get_panel_f64(ds, k0, k1, faces, st, rt.plan, &pe, both ? &least : nullptr);
     if (rc) return rc;
     const double* panel = static_cast<const double*>(pe->d_panel);
     if (pe->plan.paired) {

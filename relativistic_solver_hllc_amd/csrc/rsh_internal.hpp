@@ -70,8 +70,9 @@ F64Route route_f64(int m, int rows, int faces, int64_t n, int cus);
 hipError_t launch_build_phase(const double* d_dirs, const double* d_w, int m, double full_area,
                               int kind, double g, int normalize, double* d_P, hipStream_t st);
 
+// Panel of rows [k0, k1) in the plan's layout; with pl2 a second one of the same rows.
 hipError_t launch_panel_f64(const double* d_P, int m, int k0, int k1, double scale, const F64Plan& pl,
-                            double* d_panel, hipStream_t st);
+                            double* d_panel, hipStream_t st, const F64Plan* pl2 = nullptr, double* d_panel2 = nullptr);
 
 hipError_t launch_direct_f64(const double* d_illum, int faces, int64_t n, int m, const double* d_dirs,
                              const double* d_w, double full_area, const double* d_P, int ref_order,

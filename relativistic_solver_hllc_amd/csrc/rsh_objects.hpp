@@ -10,22 +10,27 @@
 
 #include "rsh_internal.hpp"
 
+// Device memory of the panels of one build; released (after the device is idle)
+// when the last of them is.
+struct PanelMemory {
+    int device = 0;
+    void* ptr = nullptr;
+    hipEvent_t ready = nullptr;  // recorded after the build
+    std::atomic<bool> built{false};  // the build was seen complete: no need to ask the event again
+    PanelMemory() = default;
+    PanelMemory(const PanelMemory&) = delete;
+    PanelMemory& operator=(const PanelMemory&) = delete;
+    ~PanelMemory();
+};
 // A cached phase panel. Shared by the direction set's cache, batch slots that
 // point their device problem table at it, and calls that are enqueuing work on
-// it; the device memory is released (after the device is idle) when the last
-// holder lets go.
+// it.
 struct PanelEntry {
-    int device = 0;
+    std::shared_ptr<PanelMemory> memory;
     void* d_panel = nullptr;
     float* d_row_inv = nullptr;  // split forms: per-row inverse scale
     rsh::F64Plan plan{};
     rsh::SplitPlan splan{};
-    hipEvent_t ready = nullptr;  // recorded after the panel build
-    mutable std::atomic<bool> built{false};  // the build was seen complete: no need to ask the event again
-    PanelEntry() = default;
-    PanelEntry(const PanelEntry&) = delete;
-    PanelEntry& operator=(const PanelEntry&) = delete;
-    ~PanelEntry();
 };
 typedef std::shared_ptr<const PanelEntry> PanelRef;
 
@@ -52,8 +57,10 @@ namespace rsh {
 // FP64 phase panel of (k0, k1, faces) in the layout of `plan`, built on stream
 // st if absent. The caller holds *out for as long as it enqueues work that reads
 // the panel (a batch slot: until the slot is removed); the cache never frees an
-// entry someone else holds.
-int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out);
+// entry someone else holds. also: a plan whose panel of these rows is not there and
+// is built in the same launch if this one's is.
+int get_panel_f64(rsh_dirset ds, int k0, int k1, int faces, hipStream_t st, const F64Plan& plan, PanelRef* out,
+                  const F64Plan* also = nullptr);
 // Split phase panel; resident != nullptr: in that row-group plan.
 int get_panel_split(rsh_dirset ds, int k0, int k1, int faces, int form, hipStream_t st, PanelRef* out,
                     const SplitPlan* resident = nullptr);
