@@ -197,10 +197,10 @@ int rsh_moments_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  * then the contraction reads only that state:
  *   rsh_split_sizes        bytes of the state and of the per-cell scale array
  *   rsh_pack_split_dev     FP64 illum [M][n_cells][faces] -> state + cell scales
- *   rsh_pack_split_avg_dev FP64 illum [M][n_cells][4] -> cell-level state (faces = 1);
+ *   rsh_pack_split_avg_dev FP64 illum [M][n_cells][4] -> cell-level state (faces = 1)
+ *                          of the face average (summed in FP64, times 1/4);
  *                          cell-level packs (this one, and rsh_pack_split_dev with
  *                          faces = 1) read the input once for M <= 1280
- *                          of the face average (summed and halved twice in FP64)
  *   rsh_scatter_split_dev  S rows [k0,k1) from the state, FP32 MFMA accumulation,
  *                          written as FP64 (out_f32 = 0) or FP32 (out_f32 = 1)
  *                          to d_out[(k - k0) * ld_out + c]; waves selects the
@@ -211,7 +211,11 @@ int rsh_moments_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  *                          keeps its rows' panel for all directions in LDS);
  *                          0 = resident-panel kernel where it applies and keeps
  *                          most CUs busy (rsh_scatter_split_route), else 8.
- *                          All kernels give bit-identical results. */
+ *                          All kernels give bit-identical results. The resident
+ *                          kernel's K loop is unrolled for M <= 800 where [k0, k1)
+ *                          needs as many row blocks per workgroup as [0, M) does
+ *                          (80 of 400 rows: five, as 400); other ranges run a loop
+ *                          of six K-steps. */
 int rsh_split_sizes(int32_t form, int32_t faces, int64_t n_cells, int32_t m, int64_t* state_bytes,
                     int64_t* scale_bytes);
 int rsh_pack_split_dev(int32_t form, const double* d_illum, int32_t faces, int64_t n_cells, int32_t m,
@@ -222,8 +226,8 @@ int rsh_scatter_split_dev(rsh_dirset ds, int32_t form, const void* d_state, cons
                           int32_t faces, int64_t n_cells, int32_t k0, int32_t k1, void* d_out, int64_t ld_out,
                           int32_t out_f32, void* stream, int32_t waves);
 
-/* Allocation-free variant of rsh_scatter_f64_dev (MFMA kernel, tuned or
- * default tile). No counterpart in the reference: it is for callers that
+/* Allocation-free variant of rsh_scatter_f64_dev (the kernel that an automatic
+ * call of these sizes runs). No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under stream capture, tight serving
  * loops, harnesses that forbid hipMalloc). Instead of the direction set's
  * panel cache it builds the phase panel of [k0, k1) into a fixed per-device

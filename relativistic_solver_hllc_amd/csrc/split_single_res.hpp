@@ -359,7 +359,8 @@ hipError_t launch_res(const SingleResArgs& a) {
 }
 
 // K-steps LO .. HI of one form; explicitly instantiated by the kernels_res_*.hip
-// files. hipErrorNotFound: no unrolled instance of this plan.
+// files. hipErrorNotFound: no unrolled instance of this plan, for instance that of a
+// range of rows whose row blocks per workgroup are not the whole direction set's.
 template <int FMT, int NT, int LO, int HI>
 hipError_t single_res_range(const SingleResArgs& a);
 
