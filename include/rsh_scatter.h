@@ -214,8 +214,9 @@ int rsh_moments_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  *                          All kernels give bit-identical results. The resident
  *                          kernel's K loop is unrolled for M <= 800 where [k0, k1)
  *                          needs as many row blocks per workgroup as [0, M) does
- *                          (80 of 400 rows: five, as 400); other ranges run a loop
- *                          of six K-steps. */
+ *                          (80 of 400 rows: five, as 400); other ranges, and cells
+ *                          too few for two chunks of 128 per workgroup, run a loop of
+ *                          six K-steps. */
 int rsh_split_sizes(int32_t form, int32_t faces, int64_t n_cells, int32_t m, int64_t* state_bytes,
                     int64_t* scale_bytes);
 int rsh_pack_split_dev(int32_t form, const double* d_illum, int32_t faces, int64_t n_cells, int32_t m,

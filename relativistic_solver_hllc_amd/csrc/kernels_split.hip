@@ -311,7 +311,8 @@ __global__ __launch_bounds__(16 * CPB) void pack_wide_kernel(const double* __res
 // the even lane gets the four faces of the first group's row, the odd lane those
 // of the second's, which are the values each one packs. Same arithmetic, same
 // bits as pack_fused_kernel.
-// What bounds it: HBM (32 M bytes read and 2 NT M written per cell). A form with
+// What bounds it: HBM (32 M bytes read and 2 NT M written per cell; the instances of
+// four slots also move 60 bytes of scratch per thread, a tenth of their bytes). A form with
 // one lane per cell (two 16-byte loads of stride 32, 64 cells a workgroup, one
 // workgroup per CU: pack_wide_kernel) reads through L1 and leaves most CUs idle
 // below 16,384 cells; a form with the averages in LDS (pack_fused_kernel) fits
