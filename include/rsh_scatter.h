@@ -200,7 +200,7 @@ int rsh_moments_f64_dev(rsh_dirset ds, const double* d_illum, int32_t faces, int
  *   rsh_pack_split_avg_dev FP64 illum [M][n_cells][4] -> cell-level state (faces = 1)
  *                          of the face average (summed in FP64, times 1/4);
  *                          cell-level packs (this one, and rsh_pack_split_dev with
- *                          faces = 1) read the input once for M <= 1280
+ *                          faces = 1) read the input once for M <= 1248
  *   rsh_scatter_split_dev  S rows [k0,k1) from the state, FP32 MFMA accumulation,
  *                          written as FP64 (out_f32 = 0) or FP32 (out_f32 = 1)
  *                          to d_out[(k - k0) * ld_out + c]; waves selects the

@@ -140,8 +140,10 @@ __global__ __launch_bounds__(256) void pack_state_avg_kernel(const double* __res
 // for F = 1) goes to LDS, its largest |face| (and |extra| when given, F = 1)
 // into the cell's maximum. Then the cell scale is set exactly as
 // cell_scale_kernel sets it and the tile's state vectors are written from LDS
-// as pack_state_avg_kernel / pack_state_kernel<F = 1> write them: the same bits
-// as those two passes, with the input read once instead of twice.
+// as pack_state_avg_kernel / pack_state_kernel<F = 1> write them, with the input
+// read once instead of twice: the same parts, but that a first part whose FP32 value
+// lies halfway between two of the format may be either (here it is rounded from
+// FP64 at once).
 template <int FMT, int NT, int F>
 __global__ __launch_bounds__(256) void pack_fused_kernel(const double* __restrict__ illum,
                                                          const double* __restrict__ extra, int64_t n, int m,
@@ -559,7 +561,8 @@ hipError_t launch_pack_state_avg(int form, const double* d_illum, int64_t n, int
     return hipGetLastError();
 }
 
-bool pack_fused_supported(int m) { return (size_t)((m + 31) / 32) * 32 * 16 * sizeof(double) <= 160 * 1024; }
+// M <= 1248: the averages of a tile and the threads' maxima (cmax) in a CU's LDS.
+bool pack_fused_supported(int m) { return (size_t)(((m + 31) / 32) * 32 * 16 + 4 * 16) * sizeof(double) <= 160 * 1024; }
 
 hipError_t launch_pack_fused(int form, const double* d_illum, const double* d_extra, int faces, int64_t n, int m,
                              float* d_inv, void* d_state, hipStream_t st) {

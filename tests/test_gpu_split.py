@@ -443,3 +443,37 @@ def test_face_averaged_pack_instances_agree(gpu, form, n, m):
     assert np.array_equal(nan, np.isnan(_part_values(want, form)))
     assert np.array_equal(got[~nan], want[~nan])
     assert nan.any() and not nan.reshape(nan.shape[0], -1).all(axis=1).any()
+
+
+@pytest.mark.parametrize("form", ["fp16x2", "bf16x3"])
+@pytest.mark.parametrize("faces", [4, 1])
+@pytest.mark.parametrize("m", [1248, 1249, 1280, 1281])
+def test_cell_pack_around_the_one_pass_limit(gpu, form, faces, m):
+    """Up to 1248 directions the cell-level packs read the input once, with a tile's averages in LDS; beyond, in two
+    passes. Both against the definition (test_cell_pack_matches_layout_definition): the scales, and each part a value
+    of its format nearest to what the parts before it left, a tie broken either way."""
+    n = 37
+    illum = np.random.default_rng(m).lognormal(0.0, 2.0, size=(m, n, faces))
+    d_illum = D.DeviceArray.from_host(illum)
+    sb, cb = rs.split_sizes(form, 1, n, m)
+    state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+    if faces == 4:
+        rs.pack_split_avg_dev(form, d_illum, n, m, state, scale)
+    else:
+        rs.pack_split_dev(form, d_illum, 1, n, m, state, scale)
+    D.synchronize()
+    got_state, got_scale = state.to_host(), scale.to_host()[:n]
+    for a in (d_illum, state, scale):
+        a.free()
+    e = 11 - (np.frexp(np.max(illum, axis=(0, 2)))[1] - 1)
+    assert np.array_equal(got_scale, np.ldexp(np.float32(1.0), -e).astype(np.float32))
+    v = (((illum[..., 0] + illum[..., 1]) + illum[..., 2]) + illum[..., 3]) * 0.25 if faces == 4 else illum[..., 0]
+    steps, tiles, nt = -(-m // 32), -(-n // 16), 3 if form == "bf16x3" else 2
+    r = np.zeros((steps * 32, tiles * 16), np.float32)
+    r[:m, :n] = v * np.ldexp(1.0, e)
+    vals = got_state.view(np.uint16).reshape(tiles, steps, nt, 4, 16, 8).transpose(2, 1, 3, 5, 0, 4)
+    for part in vals.reshape(nt, steps * 32, tiles * 16):
+        p, q = _part_values(part, form), _nearest(r, form)
+        x = r.astype(np.float64)
+        assert np.all((p == q) | (np.abs(x - p) == np.abs(x - q)))
+        r = (r - p).astype(np.float32)
