@@ -33,6 +33,7 @@ int fail(int status, const std::string& msg) {
 }
 
 int hip_fail(hipError_t e, const char* what) {
+    (void)hipGetLastError();  // reported here: not by the check after the next launch as well
     std::string m = std::string(what) + ": " + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ")";
     set_error(m);
     return (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation) ? RSH_E_NOMEM : RSH_E_HIP;
@@ -1131,8 +1132,8 @@ int rsh_scatter_from_host(rsh_problem p, const double* host_illum, int32_t k0, i
         return status;
     };
     for (auto& e : ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-            return cleanup(fail(RSH_E_HIP, "event creation"));
+        if (hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming); rc != hipSuccess)
+            return cleanup(hip_fail(rc, "event creation"));
     const size_t row = (size_t)n * faces * sizeof(double);      // one direction of the illum
     const size_t srow = (size_t)n * sizeof(double);             // one direction of S
     double* s_base = p->d_S + (int64_t)(k0 - p->k_begin) * n;

@@ -92,9 +92,10 @@ int rsh_sweep_create(int32_t device, int64_t n_cells, int32_t n_dirs, const int3
         rsh_sweep_destroy(s);
         return rc;
     };
-    if (hipSetDevice(device) != hipSuccess) return cleanup(fail(RSH_E_HIP, "hipSetDevice failed"));
-    if (hipMalloc(&s->d_table, (size_t)n_dirs * sizeof(SweepDirDev)) != hipSuccess)
-        return cleanup(fail(RSH_E_NOMEM, "sweep: device allocation failed"));
+    hipError_t e = hipSetDevice(device);
+    if (e != hipSuccess) return cleanup(hip_fail(e, "hipSetDevice"));
+    e = hipMalloc(&s->d_table, (size_t)n_dirs * sizeof(SweepDirDev));
+    if (e != hipSuccess) return cleanup(hip_fail(e, "sweep: device allocation"));
     if (nodes) {
         s->node_in_source.assign((size_t)n_cells, 0);
         for (int64_t c = 0; c < n_cells; c++)
@@ -385,9 +386,10 @@ int rsh_sweep_set_direction(rsh_sweep s, int32_t k, const int32_t* order, const 
     d.block = nullptr;
     if (d.set) s->unset++;
     d.set = false;
-    if (hipMalloc(&d.block, bytes) != hipSuccess) return fail(RSH_E_NOMEM, "sweep: direction allocation failed");
-    if (hipMemcpy(d.block, w.image.get(), bytes, hipMemcpyHostToDevice) != hipSuccess)
-        return fail(RSH_E_HIP, "sweep: upload of a direction failed");
+    hipError_t e = hipMalloc(&d.block, bytes);
+    if (e != hipSuccess) return hip_fail(e, "sweep: direction allocation");
+    e = hipMemcpy(d.block, w.image.get(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_fail(e, "sweep: upload of a direction");
     char* const at = static_cast<char*>(d.block);
     d.dev.faces = reinterpret_cast<const SweepFace*>(at);
     d.dev.s3 = reinterpret_cast<const double*>(at + b_faces);

@@ -309,3 +309,22 @@ def test_scatter_from_host_cell_level_state(gpu):
     P = orc.phase_matrix(xyz, w, F, 1, 0.6, True)
     ref = orc.scatter_matrix(cells[:, :, None], P)
     assert rel(a, ref) < 1e-12
+
+
+def test_a_refused_allocation_does_not_fail_the_next_call(gpu):
+    """A HIP error belongs to the call that returns it: an allocation beyond the address space is RSH_E_NOMEM, and the
+    launches after it are checked for their own errors only."""
+    xyz, w, F = rs.fibonacci_directions(26)
+    with pytest.raises(RuntimeError, match="RSH_E_NOMEM"):
+        D.DeviceArray((1 << 58,))
+    with rs.DirectionSet(xyz, w, F) as ds:
+        d_in, out = D.DeviceArray((26, 100)), D.DeviceArray((26, 100))
+        d_in.fill(2.0)
+        with pytest.raises(RuntimeError, match="RSH_E_NOMEM"):
+            D.DeviceArray((1 << 58,))
+        ds.scatter_f64(d_in, 1, 100, 0, 26, out)
+        D.synchronize()
+        P = ds.phase_matrix(0, 26)
+        assert np.allclose(out.to_host(), 2.0 * P.sum(1, keepdims=True), rtol=1e-13)
+        d_in.free()
+        out.free()
