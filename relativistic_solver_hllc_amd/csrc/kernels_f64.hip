@@ -213,7 +213,13 @@ __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_ker
     v4d acc[RB];
     mfma_f64_accumulate<RB, W, SC, FACES>(illum, n, ldx, m, panel + (int64_t)blockIdx.y * steps * RB * 64, steps,
                                           cell, lds, acc);
+    // Loads still in flight here (the last prefetches) are waited for once: left to the
+    // compiler, the wait is in every row's branch, where it also waits for the row
+    // before to be stored (1,000 cells x 64 directions 10.7 us, 9.4 without).
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     if (cell >= n) return;
+    const int row0 = rb0 * 16 + jr;
+    double* ob = out + (int64_t)row0 * ld + cell;
     // Non-temporal stores where every 128-byte segment of a row is whole (16
     // cells at a 128-byte boundary); a ragged row stride splits each segment over
     // two lines, which must meet in L2 before they leave it: with non-temporal
@@ -224,10 +230,10 @@ __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_ker
         for (int rb = 0; rb < RB; rb++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = (rb0 + rb) * 16 + jr + 4 * r;
-                if (row < rows) {
-                    if constexpr (decltype(nt)::value) __builtin_nontemporal_store(acc[rb][r], out + (int64_t)row * ld + cell);
-                    else out[(int64_t)row * ld + cell] = acc[rb][r];
+                if (row0 + 16 * rb + 4 * r < rows) {
+                    double* o = ob + (int64_t)(16 * rb + 4 * r) * ld;
+                    if constexpr (decltype(nt)::value) __builtin_nontemporal_store(acc[rb][r], o);
+                    else *o = acc[rb][r];
                 }
             }
         }
