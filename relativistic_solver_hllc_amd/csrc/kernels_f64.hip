@@ -203,7 +203,7 @@ constexpr int f64_min_waves(int rb, int w, int sc) {
 template <int RB, int W, int SC, int FACES>
 __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_kernel(const double* __restrict__ illum, int64_t n, int64_t ldx,
                                                           int m, const double* __restrict__ panel, int steps,
-                                                          double* __restrict__ out, int64_t ld, int rows) {
+                                                          double* __restrict__ out, int64_t ld, int rows, int nontemporal) {
     __shared__ v2d lds[2][F64TileShape<RB, W, SC>::UNITS];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -220,11 +220,6 @@ __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_ker
     if (cell >= n) return;
     const int row0 = rb0 * 16 + jr;
     double* ob = out + (int64_t)row0 * ld + cell;
-    // Non-temporal stores where every 128-byte segment of a row is whole (16
-    // cells at a 128-byte boundary); a ragged row stride splits each segment over
-    // two lines, which must meet in L2 before they leave it: with non-temporal
-    // stores 413,519 cells x 302 directions took 1644 us, with plain ones 1528
-    // us (413,568 cells: 1499 us either way; 1.57 M x 400 2 % slower plain).
     auto store = [&](auto nt) {
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) {
@@ -238,7 +233,7 @@ __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_ker
             }
         }
     };
-    if ((ld & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 127) == 0) {
+    if (nontemporal) {  // f64_nontemporal
         store(std::true_type{});
     } else {
         asm volatile("" ::: "memory");  // keeps the compiler from merging the two branches' stores into plain ones
@@ -249,11 +244,11 @@ __global__ __launch_bounds__(64 * W, f64_min_waves(RB, W, SC)) void mfma_f64_ker
 
 template <int W, int SC, int FACES>
 static hipError_t launch_mfma_rb(int rb, dim3 grid, hipStream_t st, const double* illum, int64_t n, int64_t ldx, int m,
-                                 const double* panel, int steps, double* out, int64_t ld, int rows) {
+                                 const double* panel, int steps, double* out, int64_t ld, int rows, int nontemporal) {
 #define RSH_RB_CASE(V)                                                                                           \
     case V:                                                                                                      \
         hipLaunchKernelGGL((mfma_f64_kernel<V, W, SC, FACES>), grid, dim3(64 * W), 0, st, illum, n, ldx, m, panel, \
-                           steps, out, ld, rows);                                                                \
+                           steps, out, ld, rows, nontemporal);                                                                \
         break;
     switch (rb) {
         RSH_RB_CASE(1) RSH_RB_CASE(2) RSH_RB_CASE(3) RSH_RB_CASE(4) RSH_RB_CASE(5) RSH_RB_CASE(6)
@@ -273,6 +268,24 @@ bool mfma_f64_tile_supported(int waves, int chunk_steps) {
     return (waves == 4 && (chunk_steps == 2 || chunk_steps == 4)) || (waves == 8 && chunk_steps == 2);
 }
 
+// Whether results are stored past the caches. Where rows start at 64-byte boundaries
+// every store fills whole halves of lines: yes. A ragged row stride splits each
+// 16-cell segment over two lines, whose pieces must meet in L2 before they leave it:
+// plain stores (413,519 cells x 302 directions 1528 us, non-temporal 1644), unless
+// keeping results out of the caches is worth more because the faces are what they
+// hold, in calls on the same or freshly swept faces: everything fits L2 (faces and
+// results up to 60 MB), the results are at most an eighth of the faces, or faces that
+// fit the 256 MB cache share it with results that make it overflow by less than a
+// quarter. us, plain / non-temporal, four faces: 42,851 x 22 9.5 / 7.5; 319,444 cells,
+// 61 of 180 rows 400 / 376; 407,307 x 19 58.3 / 50.5; one: 254,290 x 9 10.2 / 7.9,
+// 872,758 x 23 81 / 72; against 250,003 x 32 26 / 37, 80,001 x 64 20 / 30.
+static bool f64_nontemporal(int faces, int64_t n, int m, int rows, const double* out, int64_t ld) {
+    if (ld % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 64 == 0) return true;
+    const double in = 8.0 * faces * m * (double)n, res = 8.0 * rows * (double)n, cache = 268e6;
+    return in + res <= 60e6 || 8.0 * res <= in ||
+           (in <= 1.25 * cache && in + res > cache && in + res <= (4.0 * res <= in ? 420e6 : 330e6));
+}
+
 hipError_t launch_mfma_f64(const double* d_illum, int faces, int64_t n, int64_t ldx, int m, const double* d_panel,
                            const F64Plan& pl, int rows, double* d_out, int64_t ld, int waves, int chunk_steps,
                            hipStream_t st) {
@@ -282,12 +295,12 @@ hipError_t launch_mfma_f64(const double* d_illum, int faces, int64_t n, int64_t 
     if (pl.steps % chunk_steps != 0) return hipErrorInvalidValue;
     const int64_t bx = (n + 16 * waves - 1) / (16 * waves);
     const dim3 grid((unsigned)bx, (unsigned)pl.passes);
-    const int rb = pl.rb_per_pass;
+    const int rb = pl.rb_per_pass, nt = f64_nontemporal(faces, n, m, rows, d_out, ld) ? 1 : 0;
 #define RSH_TILE(W, SC)                                                                                \
     if (waves == W && chunk_steps == SC) {                                                             \
         if (faces == 4)                                                                                \
-            return launch_mfma_rb<W, SC, 4>(rb, grid, st, d_illum, n, ldx, m, d_panel, pl.steps, d_out, ld, rows); \
-        return launch_mfma_rb<W, SC, 1>(rb, grid, st, d_illum, n, ldx, m, d_panel, pl.steps, d_out, ld, rows);    \
+            return launch_mfma_rb<W, SC, 4>(rb, grid, st, d_illum, n, ldx, m, d_panel, pl.steps, d_out, ld, rows, nt); \
+        return launch_mfma_rb<W, SC, 1>(rb, grid, st, d_illum, n, ldx, m, d_panel, pl.steps, d_out, ld, rows, nt);    \
     }
     RSH_TILE(8, 2)
     RSH_TILE(4, 2)

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from oracle import orc
+from relativistic_solver_hllc_amd import _native as N
 from relativistic_solver_hllc_amd import device as D
 from relativistic_solver_hllc_amd import scatter as rs
 
@@ -98,3 +99,27 @@ def test_every_kind_of_route_equals_the_lds_panel_kernel(gpu, size):
         want = evaluate(ds, d_in, faces, n, 0, m, kernel="mfma", tile=(8, 2))
     d_in.free()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("faces,m,rows,n", [(4, 22, 22, 42851), (1, 64, 64, 80001), (4, 48, 48, 80001), (4, 302, 61, 40001),
+                                            (4, 100, 100, 80003), (1, 200, 200, 250003)])
+def test_every_kind_of_store_gives_the_same_results(gpu, faces, m, rows, n):
+    """Ragged rows are stored plainly or past the caches by the sizes of faces and results (under 60 MB, between, results
+    under an eighth, around the 256 MB cache, far beyond); rows at 64 and 128 bytes past the caches: the same bits, and
+    nothing past a row's cells."""
+    xyz, w, F = rs.fibonacci_directions(m)
+    strides = (n, (n + 7) // 8 * 8, (n + 15) // 16 * 16 + 16)
+    d_in, out = D.DeviceArray((m, n, faces)), D.DeviceArray((rows, strides[-1]))
+    N.call("rsh_fill_lognormal_dev", d_in.ptr, d_in.size, 0.0, 1.0, 5, None)
+    first = None
+    with rs.DirectionSet(xyz, w, F) as ds:
+        for ld in strides:
+            out.fill(-1.0)
+            ds.scatter_f64(d_in, faces, n, 0, rows, out, ld=ld)
+            D.synchronize()
+            got = out.to_host().reshape(-1)[:rows * ld].reshape(rows, ld)
+            first = got[:, :n].copy() if first is None else first
+            assert np.array_equal(got[:, :n], first)
+            assert np.all(got[:, n:] == -1.0)
+    for a in (d_in, out):
+        a.free()
