@@ -179,11 +179,21 @@ hipError_t launch_mfma_f64_reg(const double* d_illum, int faces, int64_t n, int6
 //     the CU's L1 delivers 4 w waves' faces and panel at 64 B/cycle, three quarters
 //     of it beside the MFMAs' time; the first loads and the ring cost ~130 cycles
 //     per j-step.
+//   The register-fed kernel is never faster than the memory, faces and results at 10
+//     TB/s from the caches (256 MB) or 5.5 from HBM (us: 40,000 cells, 47 of 368 rows
+//     98, LDS panel 89; 40,000 x 32 10.4 / 9.0). With one face and fewer than four row
+//     blocks it is left out beyond 32,768 cells, where its loads of 128 bytes a row fall
+//     behind (52,862 x 25 8.8 / 7.0, 149,946 x 6 6.8 / 6.0). Up to four row blocks of all
+//     directions, four faces, the memory bounds the LDS panel too, and fuller rounds
+//     give nothing: eight waves (235,653 x 32 51, four waves 54; x 40 85 / 89; x 64 137 /
+//     148; but 34,167 cells, 58 of 294 rows 74 / 68, 143,340 x 113 157 / 146).
 F64Route route_f64(int m, int rows, int faces, int64_t n, int cus) {
     F64Route best{plan_f64(m, rows), 8, 2};
     const int nrb = (rows + 15) / 16;
     const double steps = (m + 3) / 4;
-    const double face_bytes = 8.0 * faces * m * (double)n;
+    const double face_bytes = 8.0 * faces * m * (double)n, bytes = face_bytes + 8.0 * rows * (double)n;
+    const double memory = bytes / (bytes < 268e6 ? 10e12 : 5.5e12) * 2.4e9;
+    const bool few_rows = nrb <= 4 && faces == 4 && 2 * rows > m;
     auto rounds = [&](int64_t wgs) { return (double)((wgs + cus - 1) / cus); };
     const int p0 = best.plan.passes;
     double cost = 0.0;
@@ -194,7 +204,7 @@ F64Route route_f64(int m, int rows, int faces, int64_t n, int cus) {
         for (int waves : {8, 4}) {
             if (waves == 4 && pl.rb_per_pass > kF64FourWaveMaxRb) continue;
             const double u = waves / 4 * rounds((n + 16 * waves - 1) / (16 * waves) * p);
-            const double c = steps * (u * pl.rb_per_pass * 64 + 670) + again;
+            const double c = std::max(steps * (u * pl.rb_per_pass * 64 + 670), few_rows ? memory : 0.0) + again;
             // the first candidate unless another is clearly better
             if (cost == 0.0 || c < 0.97 * cost) {
                 cost = c;
@@ -202,16 +212,18 @@ F64Route route_f64(int m, int rows, int faces, int64_t n, int cus) {
             }
         }
     }
-    if (n > (int64_t(1) << 18)) return best;  // never cheaper: every wave re-reads the faces and the panel
+    // never cheaper: every wave re-reads the faces and the panel
+    if (n > (int64_t(1) << (faces == 1 && nrb < 4 ? 15 : 18))) return best;
     // 32-bit counts: at most 2^14 tiles, and nrb row groups
     const unsigned tiles = (unsigned)((n + 15) / 16), rb = (unsigned)nrb;
+    double reg = 0.0;
     for (unsigned r = 1; r <= 10; r++) {
         if (!f64_reg_rows_supported((int)r)) continue;
         const unsigned units = tiles * ((rb + r - 1) / r);
         const double w = (units + kRegWaves * cus - 1) / (kRegWaves * cus);
         const double c = steps * (w * r * 64 + 0.75 * w * kRegWaves * (512.0 * faces + 512.0 * r) / 64 + 130);
-        if (c < cost) {
-            cost = c;
+        if (std::max(c, memory) < cost && (reg == 0.0 || c < reg)) {
+            reg = c;
             best = F64Route{plan_f64_reg(m, rows, (int)r), 0, 0};
         }
         if (r >= rb) break;  // more row blocks per wave than there are
