@@ -575,8 +575,16 @@ hipError_t launch_pack_fused(int form, const double* d_illum, const double* d_ex
     // Rows of many cells that start inside a line (n not a multiple of 4): 64 cells
     // a workgroup share fewer lines than 32 (us, wide / pair: 413,519 x 302 892 / 964
     // two parts, 940 / 971 three, 400 directions 1262 / 1285; 79,999 x 100 63 / 56).
-    const bool wide = n % 4 != 0 && n >= 131072 && steps <= kPackWideMaxSteps;
-    if (faces == 4 && !wide && steps <= kPackPairMaxSteps) {
+    // Few cells of four faces: the LDS form's 16 cells a workgroup reach more CUs than 32
+    // (us, LDS / pair: 30 x 784 13.3 / 17.3, 193 x 730 15 / 23, 1024 x 400 10 / 12, 4096 x 512
+    // 17 / 20; 6000 x 640 42 / 26); at 257 to 416 directions, three or four of whose
+    // workgroups share a CU, up to 24,576 cells (16,490 x 321 41 / 50, 32,000 x 400 97 / 92),
+    // at 417 to 512 up to 8192 (8000 x 500 28 / 31), and up to 16,384 the wide form (11,574 x
+    // 500 39, pair 48), one workgroup a CU.
+    const int64_t lds_cells = steps < 9 || steps > 16 ? 4096 : steps <= 13 ? 24576 : 8192;
+    const bool by_lds = faces == 4 && n <= lds_cells;
+    const bool wide = steps <= kPackWideMaxSteps && ((n % 4 != 0 && n >= 131072) || (steps > 13 && n <= 16384));
+    if (faces == 4 && !by_lds && !wide && steps <= kPackPairMaxSteps) {
         const dim3 pgrid((unsigned)((n + 255) / 256 * 8)), pblock(64 * kPackPairWaves);
 #define RSH_PP(FMT, NT, MAXS)                                                                                       \
     if (steps <= 4 * MAXS) {                                                                                        \
@@ -590,7 +598,7 @@ hipError_t launch_pack_fused(int form, const double* d_illum, const double* d_ex
 #undef RSH_PP_SLOTS
 #undef RSH_PP
     }
-    if (steps <= kPackWideMaxSteps) {
+    if (!by_lds && steps <= kPackWideMaxSteps) {
         const dim3 wgrid((unsigned)((n + kPackCells - 1) / kPackCells)), wblock(16 * kPackCells);
 #define RSH_PW(FMT, NT, F)                                                                                        \
     {                                                                                                             \

@@ -404,11 +404,13 @@ def test_automatic_choice_beyond_800_directions(gpu, n):
 
 
 @pytest.mark.parametrize("form", ["bf16x2", "fp16x2", "bf16x3"])
-@pytest.mark.parametrize("n,m", [(33, 100), (70, 250), (36, 512), (65, 513), (64, 896), (131073, 20)])
+@pytest.mark.parametrize("n,m", [(33, 100), (4097, 100), (4099, 250), (24577, 257), (16385, 417), (16384, 417), (8193, 450),
+                                 (8192, 512), (4097, 513), (4100, 896), (131073, 20)])
 def test_face_averaged_pack_instances_agree(gpu, form, n, m):
-    """Each instance of the face-averaged pack (1, 2, 4 and 7 slots of lane pairs, 64-cell groups) against the one through
-    LDS, which takes the same rows followed by zero rows up to 897 directions and more: the same scales and the same
-    bits of the first K-steps, for cells without an intensity and with infinities and NaN too."""
+    """Each instance of the face-averaged pack (1, 2, 4 and 7 slots of lane pairs, 64-cell groups) and the sizes between
+    which they are chosen against the one through LDS, which takes the same rows followed by zero rows up to 897
+    directions and more: the same scales and the same bits of the first K-steps, for cells without an intensity and
+    with infinities and NaN too."""
     rng = np.random.default_rng(n * m)
     illum = rng.lognormal(0.0, 3.0, size=(m, n, 4)) * rng.choice([-1.0, 1.0], size=(m, n, 4))
     illum[:, 3] = 0.0
