@@ -53,6 +53,20 @@ static void single_res_form(int nt, int64_t n, int sets, int out_f32, int* waves
     *tiles = 4;
 }
 
+// Whether results are stored past the caches: FP64 where every 16 cells of a row fill
+// whole 128-byte lines; a line stored in pieces has to meet in L2 (302 directions, three
+// parts, us non-temporal / plain: 413,519 cells, odd rows, FP32 718 / 560, FP64 868 / 616;
+// 393,216 cells FP32 458 / 422, FP64 490 / 500). And both kinds, pieces or not, where many
+// row groups re-read a state that fits the 256 MB cache and plain results would push it
+// out (long slices, 43,477 cells, us non-temporal / plain: 854 directions two parts 370 /
+// 450, FP32 338 / 409, three parts 502 / 655; 80,001 x 640 two parts 288 / 328; but three
+// parts, whose state does not fit, 501 / 440, and 20,001 x 854, all of which fits, 176 / 140).
+static bool single_res_nontemporal(int nt, int64_t n, int steps, int rows, const void* out, int64_t ld, int out_f32) {
+    if (!out_f32 && ld % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 128 == 0) return true;
+    const double state = 64.0 * nt * steps * (double)n, res = (out_f32 ? 4.0 : 8.0) * rows * (double)n, cache = 268e6;
+    return steps >= kResLongSteps && state <= cache && state + res > cache;
+}
+
 hipError_t launch_split_resident(int form, const void* d_state, int64_t n, const float* d_cell_inv,
                                  const void* d_panel, const float* d_row_inv, const SplitPlan& pl, int sets, int rows,
                                  void* d_out, int64_t ld, int out_f32, hipStream_t st) {
@@ -67,7 +81,8 @@ hipError_t launch_split_resident(int form, const void* d_state, int64_t n, const
     const int64_t chunks = (tiles + waves * per_wave - 1) / (waves * per_wave);
     const SingleResArgs a{pl.rb_per_pass, pl.steps, waves, per_wave, kXcds * sets * pl.passes, lds_bytes, st,
                           static_cast<const v4u*>(d_state), n, d_cell_inv, static_cast<const v4u*>(d_panel), d_row_inv,
-                          d_out, ld, rows, out_f32, pl.passes, sets, chunks};
+                          d_out, ld, rows, out_f32,
+                          single_res_nontemporal(nt, n, pl.steps, rows, d_out, ld, out_f32) ? 1 : 0, pl.passes, sets, chunks};
     if (per_wave > 1 && pl.steps <= kSingleResMaxSteps) {
         hipError_t e = hipErrorNotFound;
         switch (form) {

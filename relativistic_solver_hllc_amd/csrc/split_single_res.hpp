@@ -43,6 +43,7 @@ constexpr int kSingleResMaxSteps = 25;
 // One wave per SIMD, 512 registers: five row blocks.
 constexpr int kRes4MaxRbw = 5;
 constexpr int kRes4LdsParts = 2;  // panel parts resident in LDS
+constexpr int kResLongSteps = 20;  // from these K-steps on a slice holds at most three row blocks
 
 // Row blocks per workgroup for rb_need row blocks: the largest slice that fits
 // LDS (panel fragments + row scales), then balanced; 0: not even one fits.
@@ -67,7 +68,7 @@ struct SingleResArgs {
     const float* row_inv;
     void* out;
     int64_t ld;
-    int rows, out_f32, groups, sets;
+    int rows, out_f32, nontemporal, groups, sets;
     int64_t chunks;
 };
 
@@ -93,7 +94,7 @@ template <int RBW, int FMT, int NT, int STEPS, int W, int TT>
 __global__ __launch_bounds__(64 * W) void split_resident_kernel(
     const v4u* __restrict__ state, int64_t n, int steps_rt, const float* __restrict__ cell_inv,
     const v4u* __restrict__ panel, const float* __restrict__ row_inv, void* __restrict__ out, int64_t ld, int rows,
-    int out_f32, int groups, int sets, int64_t chunks) {
+    int out_f32, int nontemporal, int groups, int sets, int64_t chunks) {
     typedef typename Fmt<FMT>::V V;
     constexpr int CT = W * TT;  // tiles per chunk
     constexpr int NL = 2;
@@ -200,7 +201,6 @@ __global__ __launch_bounds__(64 * W) void split_resident_kernel(
         });
     };
 
-    const bool whole_lines = ld % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 128 == 0;
     int64_t chunk = c_begin + set;
     // hi fragments of the next K-step (res_mfma_step reads them a step ahead)
     V ahi[RBW];
@@ -335,15 +335,21 @@ __global__ __launch_bounds__(64 * W) void split_resident_kernel(
             if (full) store_all(elem_tag, std::true_type{}, aux_tag);
             else store_all(elem_tag, std::false_type{}, aux_tag);
         };
-        // Non-temporal only where every 16 cells of a row fill whole 128-byte
-        // lines; a line stored in pieces has to meet in L2. 302 directions, three
-        // parts, us non-temporal / plain: 413,519 cells (odd rows) FP32 718 / 560,
-        // FP64 868 / 616; 393,216 cells FP32 458 / 422, FP64 490 / 500.
         typedef std::integral_constant<int, 0> Plain;
         typedef std::integral_constant<int, kNontemporal> Nt;
-        if (out_f32) stores(0.0f, Plain{});
-        else if (whole_lines) stores(0.0, Nt{});
-        else stores(0.0, Plain{});
+        if (out_f32) {
+            // single_res_nontemporal is for FP64 results but with long slices
+            if constexpr (STEPS == 0 || STEPS >= kResLongSteps) {
+                if (nontemporal) stores(0.0f, Nt{});
+                else stores(0.0f, Plain{});
+            } else {
+                stores(0.0f, Plain{});
+            }
+        } else if (nontemporal) {
+            stores(0.0, Nt{});
+        } else {
+            stores(0.0, Plain{});
+        }
     }
 }
 
@@ -354,7 +360,7 @@ hipError_t launch_res(const SingleResArgs& a) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)a.lds_bytes);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(a.blocks), dim3(64 * W), a.lds_bytes, a.st, a.state, a.n, a.steps, a.cell_inv,
-                       a.panel, a.row_inv, a.out, a.ld, a.rows, a.out_f32, a.groups, a.sets, a.chunks);
+                       a.panel, a.row_inv, a.out, a.ld, a.rows, a.out_f32, a.nontemporal, a.groups, a.sets, a.chunks);
     return hipGetLastError();
 }
 

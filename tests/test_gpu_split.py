@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 from oracle import orc
+from relativistic_solver_hllc_amd import _native as N
 from relativistic_solver_hllc_amd import device as D
 from relativistic_solver_hllc_amd import scatter as rs
 
@@ -479,3 +480,32 @@ def test_cell_pack_around_the_one_pass_limit(gpu, form, faces, m):
         x = r.astype(np.float64)
         assert np.all((p == q) | (np.abs(x - p) == np.abs(x - q)))
         r = (r - p).astype(np.float32)
+
+
+@pytest.mark.parametrize("form,n,m", [("fp16x2", 43477, 854), ("fp16x2", 20001, 854), ("bf16x3", 80001, 640), ("fp16x2", 80001, 640)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_every_kind_of_store_of_the_resident_kernel(gpu, form, n, m, f32):
+    """Long panel slices (20 K-steps and more): results past the caches where the state fits the 256 MB cache and does
+    not with the results, plain elsewhere, FP64 rows of whole lines past the caches always. The same bits, those of the
+    streaming kernel, and nothing past a row's cells."""
+    xyz, w, F = rs.fibonacci_directions(m)
+    rows, strides = 300, (n, (n + 15) // 16 * 16 + 16)
+    sb, cb = rs.split_sizes(form, 1, n, m)
+    state, scale = D.DeviceArray((sb,), np.uint8), D.DeviceArray((cb // 4,), np.float32)
+    d_in, out = D.DeviceArray((m, n)), D.DeviceArray((m, strides[-1]), np.float32 if f32 else np.float64)
+    N.call("rsh_fill_lognormal_dev", d_in.ptr, d_in.size, 0.0, 1.5, 3, None)
+    rs.pack_split_dev(form, d_in, 1, n, m, state, scale)
+    mark = np.full(out.shape, -1.0, out.dtype)
+    with rs.DirectionSet(xyz, w, F) as ds:
+        for k1 in (m, rows):
+            first = None
+            for waves, ld in ((8, n), (1, n), (1, strides[-1])):
+                out.copy_from(mark)
+                ds.scatter_split(form, state, scale, 1, n, 0, k1, out, ld=ld, out_f32=f32, waves=waves)
+                D.synchronize()
+                got = out.to_host().reshape(-1)[:k1 * ld].reshape(k1, ld)
+                first = got[:, :n].copy() if first is None else first
+                assert np.array_equal(got[:, :n], first)
+                assert np.all(got[:, n:] == -1.0)
+    for a in (state, scale, d_in, out):
+        a.free()
