@@ -237,10 +237,14 @@ class Sweep:
         for the next one (it may fill the same arrays again)."""
         it = iter(enumerate(per_dir))
         # Planning a direction is host work outside the library's lock: with all of them at hand several at a time,
-        # direction 0 alone (the workgroup size follows from it).
-        some = 1 if isinstance(per_dir, (list, tuple)) and _cpus() > 1 else None
-        for k, d in islice(it, some):
+        # direction 0 alone (the workgroup size follows from it), where that is more than the threads cost (us per
+        # direction, one at a time / eight: 384 cells x 24 directions 44 / 75, 1296 74 / 80, 3072 163 / 110, 82,944 x 40
+        # 3821 / 1053; 10,368 x 2 494 / 646).
+        several = isinstance(per_dir, (list, tuple)) and len(per_dir) > 2 and self.n >= 2000 and _cpus() > 1
+        for k, d in islice(it, 1 if several else None):
             self.set_direction(k, *d)
+        if not several:
+            return
         with ThreadPoolExecutor(max_workers=min(8, _cpus())) as ex:
             while some := list(islice(it, 8)):
                 list(ex.map(lambda kd: self.set_direction(kd[0], *kd[1]), some))

@@ -227,8 +227,8 @@ def test_direction_files_roundtrip(tmp_path, mesh4):
 class Recorder(sw.Sweep):
     """A Sweep without a device: set_direction notes what it is given."""
 
-    def __init__(self):
-        self.handle, self.seen = None, {}
+    def __init__(self, n=100000):
+        self.handle, self.seen, self.n = None, {}, n
 
     def set_direction(self, k, order, face_state, s, in_face):
         self.seen[k] = [np.array(a) for a in (order, face_state, s, in_face)]
@@ -246,9 +246,11 @@ def test_set_all_takes_an_iterators_item_before_the_next():
                 b[:] = a
             yield tuple(buf)
 
-    for given in (reuse(), iter(items), items, tuple(tuple(i) for i in items)):
-        r = Recorder()
-        r.set_all(given)
-        assert sorted(r.seen) == list(range(n))
-        for k in range(n):
-            assert all(np.array_equal(a, b) for a, b in zip(r.seen[k], items[k]))
+    for cells in (100000, 100):  # directions on several threads, one at a time
+        for given in (reuse(), iter(items), items, tuple(tuple(i) for i in items), items[:2], items[:1], []):
+            r = Recorder(cells)
+            r.set_all(given)
+            count = len(given) if isinstance(given, list) else n
+            assert sorted(r.seen) == list(range(count))
+            for k in range(count):
+                assert all(np.array_equal(a, b) for a, b in zip(r.seen[k], items[k]))
