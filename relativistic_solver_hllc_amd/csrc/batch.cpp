@@ -95,7 +95,7 @@ struct ClassState {
     int* d_n_items = nullptr;
     int n_items = 0;
     int counter_index = 0;
-    // resident-panel split classes: K-steps and row groups; d_meta = [problems, row groups, sets]
+    // resident-panel split classes: K-steps and row groups; d_meta = [problems, row groups, sets, chunks]
     bool res = false;
     int steps = 0;
     int groups = 0;
@@ -258,7 +258,7 @@ int rebuild(rsh_batch b) {
                 cs.grid = iter_split_res_grid(s.res_waves, device_cus(b->device));
                 RSH_HIP_TRY(launch_grouped_iter_split_res(false, cs.form, rb, cs.steps, cs.tile.waves, 0, nullptr,
                                                           nullptr, nullptr, 0, nullptr));
-                RSH_HIP_TRY(hipMalloc(&cs.d_meta, 3 * sizeof(int)));
+                RSH_HIP_TRY(hipMalloc(&cs.d_meta, 4 * sizeof(int)));
             } else {
                 cs.tile = rsh_tile{grouped_iter_split_waves(), 1};
                 cs.grid = grouped_iter_split_resident(s.form, rb, b->device);
@@ -270,9 +270,8 @@ int rebuild(rsh_batch b) {
         }
         if (s.res) {
             // one item per problem: its chunks are dealt to the class's sets after those of the problems before
-            const ClassState& cs = b->classes[key];
-            const int64_t cc = iter_split_res_chunk_cells(cs.tile.waves), slots = (int64_t)kXcdLists * res_sets(cs);
-            lists[key].push_back(BatchItem{i, 0, dealt[key] % slots});
+            const int64_t cc = iter_split_res_chunk_cells(b->classes[key].tile.waves);
+            lists[key].push_back(BatchItem{i, 0, dealt[key]});
             dealt[key] += (s.n + cc - 1) / cc;
             continue;
         }
@@ -297,7 +296,7 @@ int rebuild(rsh_batch b) {
         cs.n_items = (int)L.size();
         RSH_HIP_TRY(hipMemcpy(cs.d_n_items, &cs.n_items, sizeof(int), hipMemcpyHostToDevice));
         if (cs.res) {
-            const int meta[3] = {cs.n_items, cs.groups, res_sets(cs)};
+            const int meta[4] = {cs.n_items, cs.groups, res_sets(cs), (int)dealt[kv.first]};
             RSH_HIP_TRY(hipMemcpy(cs.d_meta, meta, sizeof(meta), hipMemcpyHostToDevice));
         }
     }

@@ -351,6 +351,38 @@ def test_split_resident_plans_equal_streaming(gpu, form):
         p["ds"].close()
 
 
+@pytest.mark.parametrize("form,m", [("fp16x2", 194), ("bf16x3", 200), ("fp16x2", 790)])
+@pytest.mark.parametrize("kind", ["resident", "resident4"])
+def test_runs_of_chunks_across_problems(gpu, form, m, kind):
+    """A class's chunks (256 cells; 128 with four waves) are dealt in runs of equal length: more sets than chunks (one
+    problem of a cell), a few chunks to each set with problems of a chunk, of one cell more and of many sets between,
+    and again after some of them have left. Bits of the streaming kernel."""
+    probs = [make(m, n, "hg", 0.6, seed=700 + i) for i, n in enumerate([1, 256, 257, 14001, 128, 3000, 30011, 129])]
+    out = {}
+    for k in ("streaming", kind):
+        with rs.Batch(len(probs)) as b:
+            b.set_split_kernel(k)
+            got = []
+            slots = [add_form(b, p, form) for p in probs[:1]]
+            b.run(3)
+            slots += [add_form(b, p, form) for p in probs[1:]]
+            assert {b.slot_config(s, form) for s in slots} == {("kernel", k)}
+            b.run(3)
+            got += [state(b, s, p) for s, p in zip(slots, probs)]
+            for s in slots[2:4] + slots[6:7]:
+                b.remove(s)
+            kept = slots[:2] + slots[4:6] + slots[7:]
+            b.run(2)
+            got += [state(b, s, probs[slots.index(s)]) for s in kept]
+            r, _ = b.residuals()
+            out[k] = (got, [r[s] for s in kept])
+    for x, y in zip(out["streaming"][0], out[kind][0]):
+        assert np.array_equal(x, y)
+    assert out["streaming"][1] == out[kind][1]
+    for p in probs:
+        p["ds"].close()
+
+
 def test_fp64_batch_cell_limit(gpu):
     """FP64 batch problems hold fewer than 2^24 cells (the iteration kernel's
     32-bit buffer offsets span one row block of 16 rows); larger ones are refused
