@@ -318,9 +318,10 @@ __global__ __launch_bounds__(16 * CPB) void pack_wide_kernel(const double* __res
 // one lane per cell (two 16-byte loads of stride 32, 64 cells a workgroup, one
 // workgroup per CU: pack_wide_kernel) reads through L1 and leaves most CUs idle
 // below 16,384 cells; a form with the averages in LDS (pack_fused_kernel) fits
-// one or two workgroups a CU. us, before -> now: 1243 x 400 19.9 -> 14.9, 5000 x 100
-// 8.9 -> 6.5, 80,000 x 400 253 -> 228, 1,572,864 x 400 4633 -> 4437 (5.1 TB/s),
-// 1,572,864 x 100 1173 -> 1056, 60,000 x 800 530 -> 302, 300,000 x 800 2655 -> 1606.
+// one or two workgroups a CU, which pays for few cells only (launch_pack_fused). us,
+// the wide or LDS form -> this one: 5000 x 100 8.9 -> 6.5, 80,000 x 400 253 -> 228,
+// 1,572,864 x 400 4633 -> 4437 (5.1 TB/s), 1,572,864 x 100 1173 -> 1056, 60,000 x 800
+// 530 -> 302, 300,000 x 800 2655 -> 1606.
 // Loads through the caches: 4841 at 1,572,864 x 400.
 constexpr int kPackPairMaxSteps = 28;  // 7 slots of 8 doubles: 112 registers
 constexpr int kPackPairWaves = 8;

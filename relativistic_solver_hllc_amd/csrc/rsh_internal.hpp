@@ -158,9 +158,9 @@ hipError_t launch_split_resident(int form, const void* d_state, int64_t n, const
                                  void* d_out, int64_t ld, int out_f32, hipStream_t st);
 // Cell scale and cell-level state in one pass over the input (faces = 4: the
 // face average; faces = 1: the values, with d_extra joining the scale's
-// maximum); bit-identical to launch_cell_scale followed by
-// launch_pack_state_avg (faces = 4) or launch_pack_state (faces = 1). Needs the
-// tile's averages in LDS: M <= 1280.
+// maximum); as launch_cell_scale followed by launch_pack_state_avg (faces = 4)
+// or launch_pack_state (faces = 1), bit for bit but for the side that fp16x2
+// breaks a tie to. Needs the tile's averages in LDS: M <= 1248.
 bool pack_fused_supported(int m);
 hipError_t launch_pack_fused(int form, const double* d_illum, const double* d_extra, int faces, int64_t n, int m,
                              float* d_inv, void* d_state, hipStream_t st);
